@@ -233,6 +233,7 @@ int launch_step(tlm_ctx *c, int n, const tlm::MonitorArgs &m, int nmon, hipEvent
     a.rho = c->rho;
     a.nmat = c->nmat;
     a.mstrips = tlm::magic_div((unsigned)c->strips);
+    a.mPp = tlm::magic_div((unsigned)c->Pp);
     a.mnx = tlm::magic_div((unsigned)c->nx);
     a.xm = c->xchunk > 0 ? tlm::xcd_chunk_map(c->groups, c->xchunk) : tlm::xcd_map(c->blocks, c->groups);
     a.fold = fold_of(c, n);
@@ -264,6 +265,7 @@ tlm::PulseView pulse_view(const tlm_ctx *c, int n)
     v.base = c->A;
     v.PB = c->PB;
     v.Pp = c->Pp;
+    v.mPp = tlm::magic_div((unsigned)c->Pp);
     v.pf = c->pf;
     v.slab = c->slab;
     v.h0 = c->h0;

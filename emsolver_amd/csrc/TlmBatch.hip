@@ -175,6 +175,7 @@ int rebuild(tlm_batch *b)
         a.rho = c->rho;
         a.nmat = c->nmat;
         a.mstrips = tlm::magic_div((unsigned)strips);
+        a.mPp = tlm::magic_div((unsigned)c->Pp);
         a.mnx = tlm::magic_div((unsigned)c->nx);
         d.buf[0] = M.buf[0];
         d.buf[1] = M.buf[1];

@@ -61,6 +61,7 @@ __device__ __forceinline__ PulseView member_view(const BatchMember &m, int n)
     v.base = m.buf[(n - m.n0) & 1];
     v.PB = m.st.PB;
     v.Pp = m.st.Pp;
+    v.mPp = m.st.mPp;
     v.pf = m.pf;
     v.slab = m.st.slab;
     v.h0 = m.st.h0;
@@ -124,10 +125,19 @@ __device__ __forceinline__ void monitor_batch_item(const BatchMember *mem, const
     if (n >= m.nend)
         return;
     const PulseView pv = member_view(m, n);
-    if (e.y < m.npr)
-        monitor_probe(pv, e.y, n, m.npr, m.prcell, m.inv_dl, m.prrec);
+    auto take = [&](auto pf) {
+        constexpr int PF = decltype(pf)::value;
+        if (e.y < m.npr)
+            monitor_probe<PF>(pv, e.y, n, m.npr, m.prcell, m.inv_dl, m.prrec);
+        else
+            monitor_port<PF>(pv, e.y - m.npr, n, m.np, m.pcells, m.poff, m.ppol, m.ploop, m.prec);
+    };
+    if (m.pf == PF_F32)
+        take(std::integral_constant<int, PF_F32>{});
+    else if (m.pf == PF_F16)
+        take(std::integral_constant<int, PF_F16>{});
     else
-        monitor_port(pv, e.y - m.npr, n, m.np, m.pcells, m.poff, m.ppol, m.ploop, m.prec);
+        take(std::integral_constant<int, PF_BF16>{});
 }
 
 // Fused scatter + connect for the members of one kind. gmem[g] is the member

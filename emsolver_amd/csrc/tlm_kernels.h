@@ -204,6 +204,7 @@ struct StepArgs
     float rho;
     int nmat;           // dielectric materials (props entries)
     Magic mstrips, mnx; // division by strips and by nx
+    Magic mPp;          // division by the slab pitch
     XcdMap xm;          // k_step's workgroup -> task-group mapping
     Fold fold; // FP32: soft sources added where the pulses are loaded
 };
@@ -951,6 +952,7 @@ struct PulseView
     char *base;
     long long PB;     // bytes per plane
     long long Pp;     // slab pitch (cells)
+    Magic mPp;        // division by it
     int pf;           // PF_*
     const uint2 *slab; // 16-bit formats: per slab (unused, 16-bit flag)
     int h0, h1;        // 16-bit formats: the FP32 slabs [h0, h1)
@@ -961,25 +963,68 @@ struct PulseView
 // FP32 contexts: 64-cell blocks of 12 ports per slab. 16-bit contexts: 64-cell
 // blocks of 6 pairs (pair p/2, half p&1), two codes per cell and pair in a
 // 16-bit slab, a float2 in an FP32 slab.
-__device__ __forceinline__ float pv_get(const PulseView &v, int p, long long c)
+// The 12 pulses of cell c for the injection and the monitors. What bounds
+// those is one chain of latencies, so the cell is split once (a multiply-high,
+// not a 64-bit division per port) and the format chosen once, ahead of loads
+// that are all in flight together: with a test of the format ahead of each
+// port's load, a 21 x 21 x 31 dipole's step (port, Huygens box) took 7.5 us, now
+// 5.5; the injection launch of 64 batched grids 13.9, now 9.0; a BF16 step of
+// 211 x 173 x 149 cells 91.9 with its injection, now 87.7. (Padded cell indices are below
+// 2^31: tlm_create limits a pulse plane to 32-bit byte offsets.)
+template <int PF>
+__device__ __forceinline__ void pv_get12(const PulseView &v, long long c, float x[12])
 {
-    const long long k = c / v.Pp, f = c - k * v.Pp;
+    const unsigned k = mdiv((unsigned)c, v.mPp), f = (unsigned)c - k * (unsigned)v.Pp;
+    if constexpr (PF == PF_F32)
+    {
+        const float *q = reinterpret_cast<const float *>(v.base + (size_t)k * (size_t)v.Pp * 48u + blk_off(f));
+#pragma unroll
+        for (int p = 0; p < 12; ++p)
+            x[p] = q[p * kWave];
+    }
+    else
+    {
+        const char *b = v.base + slab16_base(v.Pp, k, v.h0, v.h1);
+        if ((int)k >= v.h0 && (int)k < v.h1)
+        {
+            const float2 *q = reinterpret_cast<const float2 *>(b + blk16(f, 8u));
+#pragma unroll
+            for (int p = 0; p < 6; ++p)
+            {
+                const float2 w = q[p * kWave];
+                x[2 * p] = w.x;
+                x[2 * p + 1] = w.y;
+            }
+            return;
+        }
+        const unsigned *q = reinterpret_cast<const unsigned *>(b + blk16(f, 4u));
+        unsigned w[6];
+#pragma unroll
+        for (int p = 0; p < 6; ++p)
+            w[p] = q[p * kWave];
+        const float sc = v.sc[k];
+#pragma unroll
+        for (int p = 0; p < 6; ++p)
+        {
+            x[2 * p] = dec16<PF>(w[p] & 0xffffu) * sc;
+            x[2 * p + 1] = dec16<PF>(w[p] >> 16) * sc;
+        }
+    }
+}
+__device__ __forceinline__ void pv_get12(const PulseView &v, long long c, float x[12])
+{
     if (v.pf == PF_F32)
-        return *reinterpret_cast<const float *>(v.base + k * v.Pp * 48 + p * 256 +
-                                                blk_off((unsigned)f));
-    const uint2 s = v.slab[k];
-    const unsigned es = s.y ? 4u : 8u;
-    const char *q = v.base + slab16_base(v.Pp, k, v.h0, v.h1) + (size_t)(p >> 1) * 64u * es + blk16((unsigned)f, es);
-    if (!s.y)
-        return reinterpret_cast<const float *>(q)[p & 1];
-    const unsigned h = reinterpret_cast<const unsigned short *>(q)[p & 1];
-    return (v.pf == PF_F16 ? dec16<PF_F16>(h) : dec16<PF_BF16>(h)) * v.sc[k];
+        pv_get12<PF_F32>(v, c, x);
+    else if (v.pf == PF_F16)
+        pv_get12<PF_F16>(v, c, x);
+    else
+        pv_get12<PF_BF16>(v, c, x);
 }
 // Stores x; returns |x * 2^-E| for a 16-bit slot (0 for FP32) so callers can
 // check the range.
 __device__ __forceinline__ float pv_set(const PulseView &v, int p, long long c, float x)
 {
-    const long long k = c / v.Pp, f = c - k * v.Pp;
+    const long long k = mdiv((unsigned)c, v.mPp), f = c - k * v.Pp;
     if (v.pf == PF_F32)
     {
         *reinterpret_cast<float *>(v.base + k * v.Pp * 48 + p * 256 + blk_off((unsigned)f)) = x;
@@ -1002,7 +1047,7 @@ __device__ __forceinline__ float pv_set(const PulseView &v, int p, long long c, 
 // Stores a 16-bit code into a slot of a 16-bit slab.
 __device__ __forceinline__ void pv_set_code(const PulseView &v, int p, long long c, unsigned short h)
 {
-    const long long k = c / v.Pp, f = c - k * v.Pp;
+    const long long k = mdiv((unsigned)c, v.mPp), f = c - k * v.Pp;
     char *q = v.base + slab16_base(v.Pp, k, v.h0, v.h1) + (size_t)(p >> 1) * 64u * 4u + blk16((unsigned)f, 4u);
     reinterpret_cast<unsigned short *>(q)[p & 1] = h;
 }
@@ -1081,13 +1126,11 @@ __device__ __forceinline__ void plan_slab(const PlanArgs &p, int k)
 __device__ __forceinline__ float inject_cell(const PulseView &pv, long long c, int s0, int s1,
                                              const int *spol, const float *samp, float sv)
 {
-    const long long k = c / pv.Pp;
+    const unsigned k = mdiv((unsigned)c, pv.mPp);
     const bool h16 = pv.pf != PF_F32 && pv.slab[k].y != 0;
     const float sc = h16 ? pv.sc[k] : 1.0f, isc = h16 ? pv.isc[k] : 1.0f;
     float v[12];
-#pragma unroll
-    for (int p = 0; p < 12; ++p)
-        v[p] = pv_get(pv, p, c);
+    pv_get12(pv, c, v);
     unsigned short hc[12] = {};
     float over = 0.f;
     unsigned touched = 0u;
@@ -1161,12 +1204,11 @@ static __global__ void k_inject(PulseView pv, const long long *ucell, const int 
         pl.flag[0] = 1;
 }
 
+template <int PF>
 __device__ __forceinline__ void gather12(const PulseView &pv, long long c, float v[12])
 {
-#pragma unroll
-    for (int p = 0; p < 12; ++p)
-        v[p] = pv_get(pv, p, c);
-    if (pv.fold.ninj > 0)
+    pv_get12<PF>(pv, c, v);
+    if (PF == PF_F32 && pv.fold.ninj > 0)
         fold_sources(pv.fold, c, v);
 }
 
@@ -1182,6 +1224,13 @@ static __global__ void k_mark_fold(const long long *cell, int n, uint8_t *flags)
 
 // Port record of step n (TlmSolver.cpp:677-703): sequential float sum of
 // V_j over the port cells and I from Ampere's loop round the middle cell.
+__device__ __forceinline__ void port_record(float vsum, float ival, int id, int n, int np, float *prec)
+{
+    float *rec = prec + ((size_t)n * np + id) * 2;
+    rec[0] = vsum;
+    rec[1] = ival;
+}
+template <int PF>
 __device__ __forceinline__ void monitor_port(const PulseView &pv, int id, int n, int np,
                                              const long long *pcells, const int *poff,
                                              const int *ppol, const long long *ploop, float *prec)
@@ -1192,7 +1241,7 @@ __device__ __forceinline__ void monitor_port(const PulseView &pv, int id, int n,
     for (int s = b; s < e; ++s)
     {
         float v[12];
-        gather12(pv, pcells[s], v);
+        gather12<PF>(pv, pcells[s], v);
         vsum += scn::vj(v, pol);
     }
     if (e > b)
@@ -1201,31 +1250,35 @@ __device__ __forceinline__ void monitor_port(const PulseView &pv, int id, int n,
         const int t1 = (pol + 1) % 3, t2 = (pol + 2) % 3; // CYC_I, CYC_J
         const long long *L = ploop + 4 * (size_t)id;
         float v[12], zsum = 0.0f;
-        gather12(pv, L[0], v);
+        gather12<PF>(pv, L[0], v);
         zsum += scn::zi(v, t2);
-        gather12(pv, L[1], v);
+        gather12<PF>(pv, L[1], v);
         zsum -= scn::zi(v, t2);
-        gather12(pv, L[2], v);
+        gather12<PF>(pv, L[2], v);
         zsum -= scn::zi(v, t1);
-        gather12(pv, L[3], v);
+        gather12<PF>(pv, L[3], v);
         zsum += scn::zi(v, t1);
         ival = -2.0f * zsum / ETA0;
     }
-    float *rec = prec + ((size_t)n * np + id) * 2;
-    rec[0] = vsum;
-    rec[1] = ival;
+    port_record(vsum, ival, id, n, np, prec);
 }
 
 // E probe record of step n: (-1/dl) * V_j (TlmSolver.cpp:705-713).
-__device__ __forceinline__ void monitor_probe(const PulseView &pv, int id, int n, int npr,
-                                              const long long *prcell, float inv_dl, float *prrec)
+__device__ __forceinline__ void probe_record(const float v[12], int id, int n, int npr, float inv_dl,
+                                             float *prrec)
 {
-    float v[12];
-    gather12(pv, prcell[id], v);
     float *rec = prrec + ((size_t)n * npr + id) * 3;
     rec[0] = inv_dl * scn::vj(v, 0);
     rec[1] = inv_dl * scn::vj(v, 1);
     rec[2] = inv_dl * scn::vj(v, 2);
+}
+template <int PF>
+__device__ __forceinline__ void monitor_probe(const PulseView &pv, int id, int n, int npr,
+                                              const long long *prcell, float inv_dl, float *prrec)
+{
+    float v[12];
+    gather12<PF>(pv, prcell[id], v);
+    probe_record(v, id, n, npr, inv_dl, prrec);
 }
 
 struct MonitorArgs
@@ -1262,90 +1315,108 @@ struct MonitorArgs
     float *plane;
 };
 
+// |Js| and its DFT at one face (TlmSolver.cpp:627-649), from the pulses v of
+// its air cell at step n.
+__device__ __forceinline__ void js_record(const MonitorArgs &a, int id, int n, const float v[12])
+{
+    const int ax = a.faxis[id];
+    const float h1 = scn::zi(v, scn::pol_axis(ax, 0)), h2 = scn::zi(v, scn::pol_axis(ax, 1));
+    a.js_inst[id] = sqrtf(h1 * h1 + h2 * h2);
+    if (n >= a.settle)
+    {
+        const float cph = a.cph[n], sph = a.sph[n];
+        float *d = a.js_dft4 + 4 * (size_t)id;
+        d[0] += h1 * cph;
+        d[1] -= h1 * sph;
+        d[2] += h2 * cph;
+        d[3] -= h2 * sph;
+    }
+}
+
+// Huygens face DFT (TlmSolver.cpp:651-675); n >= settle.
+__device__ __forceinline__ void huy_record(const MonitorArgs &a, int id, int n, const float v[12])
+{
+    const int ax = a.haxis[id];
+    const int t1 = scn::pol_axis(ax, 0), t2 = scn::pol_axis(ax, 1);
+    const float e1 = -scn::vj(v, t1), e2 = -scn::vj(v, t2);
+    const float m1 = -scn::zi(v, t1), m2 = -scn::zi(v, t2);
+    const float cph = a.cph[n], sph = a.sph[n];
+    float *d = a.huy8 + 8 * (size_t)id;
+    d[0] += e1 * cph;
+    d[1] -= e1 * sph;
+    d[2] += e2 * cph;
+    d[3] -= e2 * sph;
+    d[4] += m1 * cph;
+    d[5] -= m1 * sph;
+    d[6] += m2 * cph;
+    d[7] -= m2 * sph;
+}
+
+// |E| = sqrt(sum_j V_j^2) at cell id of the plane, PEC cells 0
+// (TlmSolver.cpp:715-745).
+template <int PF>
+__device__ __forceinline__ void plane_item(const MonitorArgs &a, int id)
+{
+    const int q1 = id % a.pn1, q2 = id / a.pn1;
+    // (q1, q2) are the other two coordinates in ascending axis order
+    const int i = a.pa == 0 ? a.pidx : q1;
+    const int j = a.pa == 0 ? q1 : a.pa == 1 ? a.pidx : q2;
+    const int k = a.pa == 2 ? a.pidx : q2;
+    const long long c = (long long)k * a.Pp + (long long)j * a.nx + i;
+    float e = 0.0f;
+    if ((a.code[c] & 0xFFu) != 1u)
+    {
+        float v[12];
+        gather12<PF>(a.pv, c, v);
+        float e2 = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+        {
+            const float vj = scn::vj(v, q);
+            e2 += vj * vj;
+        }
+        e = sqrtf(e2);
+    }
+    a.plane[id] = e;
+}
+
 // Monitors on the post-injection incident pulses (TlmSolver::monitors,
 // TlmSolver.cpp:616-713), one thread per face / port / probe.
+template <int PF>
 __device__ __forceinline__ void monitor_item(const MonitorArgs &a, int id)
 {
-    const bool doDft = a.n >= a.settle;
     if (id < a.nf)
     {
         float v[12];
-        gather12(a.pv, a.fcell[id], v);
-        const int ax = a.faxis[id];
-        const float h1 = scn::zi(v, scn::pol_axis(ax, 0)), h2 = scn::zi(v, scn::pol_axis(ax, 1));
-        a.js_inst[id] = sqrtf(h1 * h1 + h2 * h2);
-        if (doDft)
-        {
-            const float cph = a.cph[a.n], sph = a.sph[a.n];
-            float *d = a.js_dft4 + 4 * (size_t)id;
-            d[0] += h1 * cph;
-            d[1] -= h1 * sph;
-            d[2] += h2 * cph;
-            d[3] -= h2 * sph;
-        }
+        gather12<PF>(a.pv, a.fcell[id], v);
+        js_record(a, id, a.n, v);
         return;
     }
     id -= a.nf;
     if (id < a.nh)
     {
-        if (!doDft)
+        if (a.n < a.settle)
             return;
         float v[12];
-        gather12(a.pv, a.hcell[id], v);
-        const int ax = a.haxis[id];
-        const int t1 = scn::pol_axis(ax, 0), t2 = scn::pol_axis(ax, 1);
-        const float e1 = -scn::vj(v, t1), e2 = -scn::vj(v, t2);
-        const float m1 = -scn::zi(v, t1), m2 = -scn::zi(v, t2);
-        const float cph = a.cph[a.n], sph = a.sph[a.n];
-        float *d = a.huy8 + 8 * (size_t)id;
-        d[0] += e1 * cph;
-        d[1] -= e1 * sph;
-        d[2] += e2 * cph;
-        d[3] -= e2 * sph;
-        d[4] += m1 * cph;
-        d[5] -= m1 * sph;
-        d[6] += m2 * cph;
-        d[7] -= m2 * sph;
+        gather12<PF>(a.pv, a.hcell[id], v);
+        huy_record(a, id, a.n, v);
         return;
     }
     id -= a.nh;
     if (id < a.np)
     {
-        monitor_port(a.pv, id, a.n, a.np, a.pcells, a.poff, a.ppol, a.ploop, a.prec);
+        monitor_port<PF>(a.pv, id, a.n, a.np, a.pcells, a.poff, a.ppol, a.ploop, a.prec);
         return;
     }
     id -= a.np;
     if (id < a.npr)
     {
-        monitor_probe(a.pv, id, a.n, a.npr, a.prcell, a.inv_dl, a.prrec);
+        monitor_probe<PF>(a.pv, id, a.n, a.npr, a.prcell, a.inv_dl, a.prrec);
         return;
     }
     id -= a.npr;
     if (id < a.pn)
-    {
-        // |E| = sqrt(sum_j V_j^2) on the plane, PEC cells 0 (TlmSolver.cpp:715-745)
-        const int q1 = id % a.pn1, q2 = id / a.pn1;
-        const int a1 = (a.pa == 0) ? 1 : 0, a2 = (a.pa == 2) ? 1 : 2;
-        int co[3];
-        co[a.pa] = a.pidx;
-        co[a1] = q1;
-        co[a2] = q2;
-        const long long c = (long long)co[2] * a.Pp + (long long)co[1] * a.nx + co[0];
-        float e = 0.0f;
-        if ((a.code[c] & 0xFFu) != 1u)
-        {
-            float v[12];
-            gather12(a.pv, c, v);
-            float e2 = 0.0f;
-            for (int j = 0; j < 3; ++j)
-            {
-                const float vj = scn::vj(v, j);
-                e2 += vj * vj;
-            }
-            e = sqrtf(e2);
-        }
-        a.plane[id] = e;
-    }
+        plane_item<PF>(a, id);
 }
 
 // The fused step: scatter + connect of every cell (strip_task / strip_task16)
@@ -1358,7 +1429,7 @@ __global__ void __launch_bounds__(256) k_step(StepArgs a, MonitorArgs m, int mon
     // alongside the step's workgroups instead of in a launch of their own)
     if ((int)blockIdx.x >= mon_from)
     {
-        monitor_item(m, ((int)blockIdx.x - mon_from) * (int)blockDim.x + (int)threadIdx.x);
+        monitor_item<PF>(m, ((int)blockIdx.x - mon_from) * (int)blockDim.x + (int)threadIdx.x);
         return;
     }
     const int lane = threadIdx.x & (kWave - 1);
@@ -1499,8 +1570,10 @@ static __global__ void k_pulses_out(PulseView pv, float *aos, long long nxy, lon
     const long long cell = c0 + id;
     const long long k = cell / nxy;
     const long long pc = k * pv.Pp + (cell - k * nxy);
+    float v[12];
+    pv_get12(pv, pc, v);
     for (int p = 0; p < 12; ++p)
-        aos[id * 12 + p] = pv_get(pv, p, pc);
+        aos[id * 12 + p] = v[p];
 }
 
 // Device rounding of the 16-bit formats (v * inv_scale), for checking the
