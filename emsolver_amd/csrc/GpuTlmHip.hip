@@ -91,6 +91,66 @@ size_t energy_parts(const tlm_ctx *c)
     return (size_t)c->blocks * c->wpb;
 }
 
+// ---- two steps a launch (k_step2) ----
+
+// Tile of a workgroup (one 64-cell block per wave and `cells`): C blocks per
+// wave, tb blocks of the tile, hb = ceil(nx / 64) blocks of rim on either
+// side, marched over zc slabs. Measured on 20 grids (us a step, tiles of one
+// / two blocks per wave): below ~6 M cells one block per wave leaves more
+// workgroups and shorter slabs (96^3 12.0 / 13.4, 128^3 21.2 / 22.5), above
+// it two reread less of the rim (256^3 182 / 171, 384^3 966 / 612). Few
+// blocks a tile where the grid is too small to fill the chip otherwise (24^3
+// 2.98 at 1 block, 3.24 at 8; 64^3 5.5 at 4, 6.1 at 8). A slab count that
+// gives every CU the same number of workgroups beats a longer march (160^3:
+// 46.7 at 250 workgroups of 32 slabs, 56 at 400 of 24).
+// The rim is 2 hb blocks of step n done twice: a tile of tb >= 8 blocks pays
+// up to hb = 12 (768 x 128 x 256: 318 against 414 us a step for two k_step
+// launches), one of 2 blocks at hb = 15 does not (606 against 263 us), so
+// grids wider than 768 cells keep single steps.
+constexpr int kPairMaxRim = 12, kPairWaves = 16, kCus = 256;
+void choose_pair(tlm_ctx *c)
+{
+    auto &p = c->pair;
+    p.hb = (c->nx + tlm::kWave - 1) / tlm::kWave;
+    p.ok = c->pf == TLM_PULSE_F32 && p.hb <= kPairMaxRim;
+    if (!p.ok)
+        return;
+    const long long ncell = (long long)c->nx * c->ny * c->nz;
+    p.cells = ncell >= (6LL << 20) || p.hb > 4 ? 2 : 1;
+    if (p.cells == 2)
+        p.tb = std::min(16, 2 * (kPairWaves - p.hb));
+    else
+        p.tb = ncell < 50000 ? 2 : ncell < 400000 ? 4 : 8;
+    p.tb = std::min(p.tb, (c->strips + p.cells - 1) / p.cells * p.cells);
+    p.ntile = (c->strips + p.tb - 1) / p.tb;
+    if (p.ntile == 1)
+        p.hb = 0; // the tile is the slab
+    p.nt = (p.tb + 2 * p.hb) / p.cells * tlm::kWave;
+    // slabs per tile: the fewest slab iterations (zc and the two beside them)
+    // over the rounds that the CUs take
+    long long best = 0;
+    for (int nzc = (c->nz + 63) / 64; nzc <= c->nz; ++nzc)
+    {
+        const int z = (c->nz + nzc - 1) / nzc;
+        const long long cost = ((long long)p.ntile * ((c->nz + z - 1) / z) + kCus - 1) / kCus * (z + 2);
+        if (best == 0 || cost < best)
+        {
+            best = cost;
+            p.zc = z;
+        }
+    }
+    p.groups = p.ntile * ((c->nz + p.zc - 1) / p.zc);
+    // equal shares for the XCDs: 8 m chunks of at most a slab's tiles (chunks
+    // of a whole slab left XCDs idle: 192^3 96 against 80 us a step)
+    const int m = (p.groups + 8 * p.ntile - 1) / (8 * p.ntile);
+    p.chunk = (p.groups + 8 * m - 1) / (8 * m);
+    p.blocks = 8 * tlm::xcd_chunk_map(p.groups, p.chunk).cpx;
+}
+size_t pair_energy_parts(const tlm_ctx *c)
+{
+    return c->pair.ok ? (size_t)c->pair.blocks * (c->pair.nt / tlm::kWave) : 0;
+}
+
 // The fused step launch; nmon > 0 appends the workgroups that take the
 // step's monitor records. With events e0 / e1 the launch carries them as its
 // own start / end timestamps (hipExtLaunchKernel): a marker recorded on the
@@ -180,19 +240,20 @@ bool fold_active(const tlm_ctx *c)
                                  step_occupancy(c) > 0);
 }
 
-tlm::Fold fold_of(const tlm_ctx *c, int n)
+tlm::Fold fold_at(const tlm_ctx *c, int n)
 {
     tlm::Fold f;
-    if (fold_active(c))
-    {
-        f.cell = c->ucell;
-        f.beg = c->ubeg;
-        f.pol = c->spol;
-        f.amp = c->samp;
-        f.ninj = c->nuniq;
-        f.sv = c->sv_host[n];
-    }
+    f.cell = c->ucell;
+    f.beg = c->ubeg;
+    f.pol = c->spol;
+    f.amp = c->samp;
+    f.ninj = c->nuniq;
+    f.sv = c->sv_host[n];
     return f;
+}
+tlm::Fold fold_of(const tlm_ctx *c, int n)
+{
+    return fold_active(c) ? fold_at(c, n) : tlm::Fold();
 }
 
 int launch_step(tlm_ctx *c, int n, const tlm::MonitorArgs &m, int nmon, hipEvent_t e0, hipEvent_t e1)
@@ -246,6 +307,130 @@ int launch_step(tlm_ctx *c, int n, const tlm::MonitorArgs &m, int nmon, hipEvent
     if (c->pf != TLM_PULSE_F32)
         hipLaunchKernelGGL(tlm::k_slab_max, dim3(c->nz), dim3(256), 0, c->stream, c->mpart,
                            c->strips, c->mreg);
+    return TLM_OK;
+}
+
+// Whether pairs of steps may run as one launch: FP32 pulses, the sources few
+// enough to be added in the step, the launch shape automatic (a caller's own
+// shape is for k_step).
+bool pair_active(const tlm_ctx *c)
+{
+    static const tlm_tuning automatic = tlm_ctx().tune;
+    return c->pair.ok && c->nuniq <= tlm::kFoldMax &&
+           std::memcmp(&c->tune, &automatic, sizeof(automatic)) == 0;
+}
+
+// Whether steps n and n+1 may be one pair: the energy, the cut plane and the
+// frames are taken from pulses in memory, so of a pair only step n has them.
+bool pair_ok(const tlm_ctx *c, int n, int end)
+{
+    return n + 1 < end && !(c->every > 0 && (n + 1) % c->every == 0) &&
+           !(c->pa >= 0 && (n + 1) % 2 == 0) &&
+           !(c->frame_every > 0 && (n % c->frame_every == 0 || (n + 1) % c->frame_every == 0));
+}
+
+// The kernel for the context's tile, with its LDS.
+struct PairKernel
+{
+    const void *f;
+    int lds;
+};
+template <bool S, bool E> PairKernel pair_kernel_of(const tlm_ctx *c)
+{
+    // an id is a byte: at most 254 dielectrics
+    constexpr int nmat = S ? 254 : 0;
+    if (c->pair.cells == 2)
+        return {(const void *)tlm::k_step2<S, E, 2, 1024>, tlm::pair_lds<2, 1024>(nmat)};
+    if (c->pair.nt <= 256)
+        return {(const void *)tlm::k_step2<S, E, 1, 256>, tlm::pair_lds<1, 256>(nmat)};
+    if (c->pair.nt <= 512)
+        return {(const void *)tlm::k_step2<S, E, 1, 512>, tlm::pair_lds<1, 512>(nmat)};
+    return {(const void *)tlm::k_step2<S, E, 1, 1024>, tlm::pair_lds<1, 1024>(nmat)};
+}
+PairKernel pair_kernel(const tlm_ctx *c, bool energy)
+{
+    if (c->stubs)
+        return energy ? pair_kernel_of<true, true>(c) : pair_kernel_of<true, false>(c);
+    return energy ? pair_kernel_of<false, true>(c) : pair_kernel_of<false, false>(c);
+}
+
+// First pair after an upload: the second stub buffer (all zero, as the stubs
+// are outside dielectric cells) and the kernels' LDS limit. A context without
+// room for the buffer (it takes at most a quarter of what is free) keeps
+// single steps.
+int prepare_pair(tlm_ctx *c)
+{
+    c->pair_ready = true;
+    for (bool energy : {false, true})
+    {
+        const PairKernel k = pair_kernel(c, energy);
+        if (k.lds > kLdsPerCu || hipFuncSetAttribute(k.f, hipFuncAttributeMaxDynamicSharedMemorySize, k.lds) != hipSuccess)
+        {
+            (void)hipGetLastError();
+            c->pair.ok = false;
+            return TLM_OK;
+        }
+    }
+    if (!c->stubs)
+        return TLM_OK;
+    const size_t n = (size_t)c->P * 3;
+    if (!c->Vs2)
+    {
+        size_t fr = 0, tot = 0;
+        if (hipMemGetInfo(&fr, &tot) != hipSuccess || n * sizeof(float) > fr / 4 ||
+            dalloc(c, &c->Vs2, n) != TLM_OK)
+        {
+            (void)hipGetLastError();
+            c->pair.ok = false;
+            return TLM_OK;
+        }
+    }
+    HIPCHK(c, hipMemsetAsync(c->Vs2, 0, n * sizeof(float), c->stream));
+    return TLM_OK;
+}
+
+int launch_pair(tlm_ctx *c, int n, const tlm::MonitorArgs &m0, hipEvent_t e0, hipEvent_t e1)
+{
+    tlm::PairArgs a = {};
+    a.A = c->A;
+    a.B = c->B;
+    a.Vs = c->Vs;
+    a.Vs2 = c->Vs2;
+    a.code = c->code;
+    a.uair = c->uair;
+    a.props = c->props;
+    a.epart = c->epart;
+    a.nx = c->nx;
+    a.ny = c->ny;
+    a.nz = c->nz;
+    a.Pp = c->Pp;
+    a.rho = c->rho;
+    a.nmat = std::min(c->nmat, 254);
+    a.strips = c->strips;
+    a.tb = c->pair.tb;
+    a.hb = c->pair.hb;
+    a.ntile = c->pair.ntile;
+    a.zc = c->pair.zc;
+    a.xm = tlm::xcd_chunk_map(c->pair.groups, c->pair.chunk);
+    a.mPp = tlm::magic_div((unsigned)c->Pp);
+    a.mnx = tlm::magic_div((unsigned)c->nx);
+    if (c->nuniq > 0)
+    {
+        a.fold = fold_at(c, n);
+        a.sv1 = c->sv_host[n + 1];
+    }
+    tlm::MonitorArgs m = m0;
+    m.pv.fold = a.fold;
+    const int wpb = c->pair.nt / tlm::kWave;
+    int mon_from = c->pair.blocks, mon_plane = (tlm::pair_face_waves(m) + m.np + wpb - 1) / wpb;
+    dim3 grid(mon_from + mon_plane + (m.pn + c->pair.nt - 1) / c->pair.nt), block(c->pair.nt);
+    const PairKernel k = pair_kernel(c, c->every > 0 && (n % c->every) == 0);
+    void *args[] = {&a, &m, &mon_from, &mon_plane};
+    if (e0)
+        HIPCHK(c, hipExtLaunchKernel(k.f, grid, block, args, k.lds, c->stream, e0, e1, 0));
+    else
+        HIPCHK(c, hipLaunchKernel(k.f, grid, block, args, k.lds, c->stream));
+    std::swap(c->Vs, c->Vs2);
     return TLM_OK;
 }
 
@@ -310,10 +495,17 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
             return fail(c, TLM_ERR_STATE, "16-bit pulse storage runs contiguous step blocks");
     }
     const bool fold = fold_active(c);
-    if (fold && !c->fold_marked)
+    if (pair_active(c) && !c->pair_ready)
+    {
+        int rc = prepare_pair(c);
+        if (rc)
+            return rc;
+    }
+    const bool pairs = pair_active(c);
+    if ((fold || (pairs && c->nuniq > 0)) && !c->fold_marked)
     {
         hipLaunchKernelGGL(tlm::k_mark_fold, dim3(1), dim3(64), 0, c->stream, c->ucell, c->nuniq,
-                           c->uair);
+                           c->uair, c->code);
         c->fold_marked = true;
     }
     const int nmon0 = c->nf + c->nh + c->np + c->npr;
@@ -330,8 +522,12 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
             c->kev.push_back(ev);
         }
     }
-    for (int n = step0; n < step0 + nsteps; ++n)
+    const int end = step0 + nsteps;
+    int per = 1; // steps of the launch
+    int nev = 0, timed_steps = 0; // timed launches and their steps
+    for (int n = step0; n < end; n += per)
     {
+        per = pairs && pair_ok(c, n, end) ? 2 : 1;
         const tlm::PulseView pv = pulse_view(c, n);
         tlm::PlanArgs pl = {};
         if (c->pf != TLM_PULSE_F32)
@@ -351,7 +547,7 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
             pl.isc_next = c->iscl[cur ^ 1];
             pl.flag = c->flag;
         }
-        if ((fold ? 0 : c->nuniq) + pl.nz > 0)
+        if ((fold || per == 2 ? 0 : c->nuniq) + pl.nz > 0)
         {
             int b = 128, g = (c->nuniq + pl.nz + b - 1) / b;
             hipLaunchKernelGGL(tlm::k_inject, dim3(g), dim3(b), 0, c->stream, pv, c->ucell,
@@ -402,11 +598,25 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
                 c->plane_step = n;
         }
         // the monitor records of step n run in the step launch's extra workgroups
+        // a launch is timed if one of its steps is among the sampled ones
         const int ti = n - step0;
-        if (time_kernel && ti % kernel_every == 0)
-            launch_step(c, n, m, nmon, c->kev[2 * (ti / kernel_every)], c->kev[2 * (ti / kernel_every) + 1]);
+        const bool timed = time_kernel && (ti + per - 1) / kernel_every * kernel_every >= ti;
+        hipEvent_t e0 = nullptr, e1 = nullptr;
+        if (timed)
+        {
+            e0 = c->kev[2 * nev];
+            e1 = c->kev[2 * nev + 1];
+            ++nev;
+            timed_steps += per;
+        }
+        if (per == 2)
+        {
+            int rc = launch_pair(c, n, m, e0, e1);
+            if (rc)
+                return rc;
+        }
         else
-            launch_step(c, n, m, nmon, nullptr, nullptr);
+            launch_step(c, n, m, nmon, e0, e1);
         if (c->frame_every > 0 && (n % c->frame_every) == 0 &&
             (int)c->frame_steps.size() < c->frame_max)
         {
@@ -425,7 +635,7 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
         if (c->every > 0 && (n % c->every) == 0)
         {
             const int idx = n / c->every;
-            const long long np = (long long)energy_parts(c);
+            const long long np = (long long)(per == 2 ? pair_energy_parts(c) : energy_parts(c));
             if (np > 8192)
             {
                 // two stages: 1024 fixed chunks, then one block
@@ -458,8 +668,8 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
     if (time_kernel && ms_kernel)
     {
         float kern_ms = 0.f;
-        HIPCHK(c, hipEventSynchronize(c->kev[2 * ntimed - 1]));
-        for (int s = 0; s < ntimed; ++s)
+        HIPCHK(c, hipEventSynchronize(c->kev[2 * nev - 1]));
+        for (int s = 0; s < nev; ++s)
         {
             float ms = 0.f;
             HIPCHK(c, hipEventElapsedTime(&ms, c->kev[2 * s], c->kev[2 * s + 1]));
@@ -467,7 +677,7 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
         }
         *ms_kernel = kern_ms;
         if (nkernel)
-            *nkernel = ntimed;
+            *nkernel = timed_steps;
     }
     HIPCHK(c, hipGetLastError());
     return TLM_OK;
@@ -727,7 +937,8 @@ int tlm_create(const tlm_grid_desc *d, tlm_ctx **out)
         if ((e = hipEventCreate(ev)) != hipSuccess)
             return bail(hip_fail(c, e, "hipEventCreate"));
     int rc;
-    c->epart_cap = energy_parts(c);
+    choose_pair(c);
+    c->epart_cap = std::max(energy_parts(c), pair_energy_parts(c));
     if (c->pf == TLM_PULSE_F32 &&
         ((rc = dalloc(c, &c->A, (size_t)c->PB * 12)) || (rc = dalloc(c, &c->B, (size_t)c->PB * 12))))
         return bail(rc);
@@ -873,6 +1084,7 @@ int install_material(tlm_ctx *c, bool any_diel, const float *yhat, const float *
         HIPCHK(c, hipMemsetAsync(c->B, 0, (size_t)c->PB * 12, c->stream));
     }
     dfree(c, c->Vs);
+    c->pair_ready = false;
     if (c->stubs)
     {
         if ((rc = dalloc(c, &c->Vs, (size_t)c->P * 3)))

@@ -5,6 +5,7 @@
 
 #include "../../include/GpuTlmHip.h"
 #include "tlm_kernels.h"
+#include "tlm_step2.h"
 
 #include <hip/hip_runtime.h>
 
@@ -26,6 +27,16 @@ struct tlm_ctx
     int strips = 0, zc = 0, nzc = 0, tasks = 0, groups = 0, blocks = 0, wpb = 4;
     int xchunk = 0; // > 0: groups per chunk of the XCD-interleaved map (choose_shape)
     size_t epart_cap = 0;
+    // two steps a launch (k_step2): tiles of tb blocks with hb blocks of rim on
+    // either side (ntile of them in a slab), marched over zc slabs by nt threads,
+    // a wave holding `cells` blocks; ok: the context may run pairs
+    struct
+    {
+        bool ok = false;
+        int tb = 0, hb = 0, ntile = 0, zc = 0, nt = 0, cells = 0, groups = 0, blocks = 0, chunk = 0;
+    } pair;
+    bool pair_ready = false; // prepared since the last upload
+    float *Vs2 = nullptr;    // the stubs a pair of steps writes (allocated at the first one)
     // state
     int pf = TLM_PULSE_F32; // pulse storage format
     int halo = 8;           // 16-bit formats: FP32 slabs on each side of a source slab

@@ -17,8 +17,9 @@
 //   * cell code: 16 bits per cell address: material id in bits 0-7 (0 air,
 //     1 PEC, >= 2 dielectric), then one bit per face telling whether the
 //     neighbour across it is PEC (bit 8 x-, 9 x+, 10 y-, 11 y+, 12 z-,
-//     13 z+; 0 on outer faces). Built once at upload, so a cell needs a
-//     single 2-byte load and never reads its neighbours' materials.
+//     13 z+; 0 on outer faces), bit 14 kCodeSource. Built once at
+//     upload, so a cell needs a single 2-byte load and never reads its
+//     neighbours' materials.
 //
 // One step is (TlmSolver::step, TlmSolver.cpp:485-513):
 //   k_inject  : soft sources add 0.5*amp*sv(n) into A        (:487-505)
@@ -236,6 +237,10 @@ enum : unsigned
     NB_ZM = 1u << 12,
     NB_ZP = 1u << 13
 };
+
+// One more bit of the cell code, read by the two-step kernel (tlm_step2.h):
+// the cell holds a folded soft source (set by k_mark_fold).
+constexpr unsigned kCodeSource = 1u << 14;
 
 // Block flag bit 5: every cell code of the 64-cell block has a material id
 // other than PEC (1) and no neighbour-PEC bit. The slab padding is coded PEC,
@@ -1212,14 +1217,19 @@ __device__ __forceinline__ void gather12(const PulseView &pv, long long c, float
         fold_sources(pv.fold, c, v);
 }
 
-// Marks the blocks holding folded source cells (flag bit 1); one thread, so
-// two cells of one block cannot race on the flag byte.
-static __global__ void k_mark_fold(const long long *cell, int n, uint8_t *flags)
+// Marks the blocks holding folded source cells (flag bit 1) and the cells
+// themselves (kCodeSource); one thread, so two cells of one block cannot race
+// on the flag byte. A mark left by an earlier source list only costs a look
+// at the list.
+static __global__ void k_mark_fold(const long long *cell, int n, uint8_t *flags, uint16_t *code)
 {
     if (blockIdx.x != 0 || threadIdx.x != 0)
         return;
     for (int u = 0; u < n; ++u)
+    {
         flags[cell[u] / kWave] |= 2u;
+        code[cell[u]] |= (uint16_t)kCodeSource;
+    }
 }
 
 // Port record of step n (TlmSolver.cpp:677-703): sequential float sum of

@@ -200,7 +200,7 @@ int tlm_read_frames(tlm_ctx *ctx, int32_t *steps, float *js, float *planes, int 
  * kernel_every = k > 0 (and ms_kernel not NULL) the fused scatter/connect
  * launches of the steps step0, step0+k, step0+2k, ... carry their own start
  * and end events: *ms_kernel is their summed duration and *nkernel (may be
- * NULL) their count. Events on a launch cost host time (~4 us per launch at
+ * NULL) the number of steps they took (a launch may take two). Events on a launch cost host time (~4 us per launch at
  * 256^3, ~20 us at 64^3), so a sample (k > 1) perturbs the run less than
  * k = 1; k = 0 measures no launch. */
 int tlm_time_steps(tlm_ctx *ctx, int step0, int nsteps, int kernel_every, float *ms_total,
@@ -213,7 +213,10 @@ int tlm_time_steps(tlm_ctx *ctx, int step0, int nsteps, int kernel_every, float 
 int tlm_copy_bandwidth(int device, size_t bytes, int iters, float *gbps, float *ms_per_copy);
 
 /* Tuning of the fused scatter/connect kernel (no effect on results, which
- * are bit-identical for every setting). No counterpart in the reference. */
+ * are bit-identical for every setting). No counterpart in the reference.
+ * With the default settings an FP32 context takes two steps a launch where it
+ * can; any other setting is the shape of the launch of a single step, and
+ * every step is then one. */
 typedef struct tlm_tuning {
     int32_t kernel;      /* 0: one cell per lane, 64-cell strips per wavefront (only variant) */
     int32_t planes;      /* z slabs marched per wave task; 0 = automatic. Default 1 with FP32
@@ -329,7 +332,10 @@ int tlm_batch_autotune(tlm_batch *b, int ticks_per_candidate, tlm_batch_tuning *
 /* Free and total device memory (admission control of a serving loop). */
 int tlm_device_memory(int device, size_t *free_bytes, size_t *total_bytes);
 /* Device bytes a context of this shape allocates (pulses, stubs if any
- * dielectric, cell codes and per-step work buffers; monitors excluded). */
+ * dielectric, cell codes and per-step work buffers; monitors excluded). An
+ * FP32 context with dielectric cells that is run by tlm_run takes a second
+ * stub buffer (12 bytes per cell) if that is at most a quarter of what is
+ * free, and steps without it otherwise. */
 int64_t tlm_estimate_bytes(const tlm_grid_desc *desc, int has_stubs);
 
 /* ---------------------------------------------------------------------
