@@ -1459,11 +1459,27 @@ int64_t tlm_huygens_mat(tlm_ctx *c, int o)
     dfree(c, c->haxis);
     c->hcell = hc;
     c->haxis = ha;
+    c->hlat = HuyLattice{};
     dfree(c, c->huy8);
     if ((rc = dalloc(c, &c->huy8, 8 * (size_t)std::max(1LL, n))))
         return rc;
     HIPCHK(c, hipMemset(c->huy8, 0, 8 * (size_t)std::max(1LL, n) * sizeof(float)));
     c->nh = (int)n;
+    if (on)
+    {
+        const int dims[3] = {c->nx, c->ny, c->nz};
+        for (int q = 0; q < 3; ++q)
+        {
+            c->hlat.lo[q] = o;
+            c->hlat.n[q] = dims[q] - 2 * o;
+            for (int side = 0; side < 2; ++side)
+            {
+                c->hlat.axis[c->hlat.nplane] = q;
+                c->hlat.coord[c->hlat.nplane++] = side ? dims[q] - 1 - o : o;
+            }
+        }
+        c->hlat.ok = huy_lattice_fits(c->hlat, c->nh);
+    }
     return n;
 }
 

@@ -13,6 +13,33 @@
 #include <string>
 #include <vector>
 
+namespace tlmi {
+
+// The Huygens faces as places of planes of a box: cell coordinates lo..lo+n-1
+// per axis, planes by normal axis and coordinate. ok: every face has a place of
+// its own there.
+constexpr int kHuyPlanes = 6;
+constexpr int kHuyLatticeMin = 4096; // faces
+struct HuyLattice
+{
+    bool ok = false;
+    int lo[3] = {0, 0, 0}, n[3] = {0, 0, 0};
+    int nplane = 0;
+    int axis[kHuyPlanes] = {}, coord[kHuyPlanes] = {};
+};
+
+// Worth a transform over all places of the planes: their rows padded to
+// 8, at most 1.5 places a face; phase tables of 32 directions stay below 24 MiB.
+inline bool huy_lattice_fits(const HuyLattice &h, int nf)
+{
+    long long places = 0;
+    for (int p = 0; p < h.nplane; ++p)
+        places += (long long)h.n[h.axis[p] == 0 ? 1 : 0] * ((h.n[h.axis[p] == 2 ? 1 : 2] + 7) / 8 * 8);
+    return nf >= kHuyLatticeMin && 2 * places <= 3LL * nf && h.n[0] + h.n[1] + h.n[2] <= 65536;
+}
+
+} // namespace tlmi
+
 struct tlm_ctx
 {
     int dev = 0;
@@ -69,6 +96,9 @@ struct tlm_ctx
     int *haxis = nullptr;
     float *huy8 = nullptr;
     int nh = 0;
+    tlmi::HuyLattice hlat;           // of the faces, for the far field
+    unsigned char *ff_ws = nullptr; // far-field workspace kept between calls
+    size_t ff_bytes = 0;
     long long *pcells = nullptr, *ploop = nullptr;
     int *poff = nullptr, *ppol = nullptr;
     float *prec = nullptr;
@@ -112,6 +142,9 @@ struct tlm_ctx
 };
 
 namespace tlmi {
+
+// Sets hlat from the context's list of faces (TlmFarField.hip).
+int huy_lattice_scan(tlm_ctx *c);
 
 // Records the message on the context (or the thread's create error) and
 // returns the code.

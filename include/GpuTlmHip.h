@@ -423,15 +423,16 @@ int tlm_far_field(int device, int nfaces, const float *pos, const int32_t *axis,
 /* From a context's own Huygens faces and accumulators (no readback of the
  * DFTs): positions cellCenter - domain centre for the given grid origin
  * (TlmSolver.cpp:323-334), outward signs from the side of the grid the face
- * is on. samples = the DFT sample count (0: no data). */
+ * is on. samples = the DFT sample count (0: no data). The context keeps its
+ * workspace for the next call if that is at most 64 MiB. */
 int tlm_far_field_ctx(tlm_ctx *ctx, const float origin[3], int samples, float f0, int n_theta,
                       int n_phi, float *U, tlm_far_field_summary *out);
 
 /* tlm_far_field_ctx without device allocation: no counterpart in the
  * reference. For callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc). The
- * transform's workspace (64-byte face records, direction tables, partial sums,
- * U) comes from a fixed 128 MiB device array that the library holds on each
+ * transform's workspace (face records or currents, phase tables, partial sums,
+ * U) comes from a fixed device array of 130 MiB that the library holds on each
  * GPU it runs on until the process ends: up to about 2 million Huygens faces
  * on the default 37 x 73 grid. Larger inputs are refused with
  * TLM_ERR_UNSUPPORTED. Calls on one GPU share that array: calls that overlap
