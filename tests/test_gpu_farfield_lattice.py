@@ -3,13 +3,13 @@
 directions taken together (an odd or even number of phi samples).
 
 Tolerance: that of test_gpu_ntff.py, 2e-5 of U_max against sums in double
-(torch's here, test_gpu_ntff.py holds the plain lists to the oracle's): float
+(numpy's here, over some of the directions; over all of them the two device
+paths are held to each other, to twice that): float
 products and sums of at most some 1e4 terms a direction, random
 rounding errors of 6e-8 each, of which the peak takes about sqrt(1e4) * 6e-8 =
 6e-6."""
 import numpy as np
 import pytest
-import torch
 
 from emsolver_amd import scenes, tlm
 from oracle import oracle_tlm as ot
@@ -44,28 +44,33 @@ def _accumulated(dims, offset, keep=None, pec=None, listed=False, V0=None):
     return sc, dev
 
 
-def _far64(pos, axes, sg, d8, f0, nt, nph):
-    """Intensity from face currents, in doubles on the device."""
-    pos, d8, sg = (torch.as_tensor(np.asarray(x, np.float64), device="cuda") for x in (pos, d8, sg))
-    e = torch.view_as_complex(d8.reshape(-1, 4, 2).contiguous())  # E1, E2, eta0 H1, eta0 H2
-    ax = torch.as_tensor(np.asarray(axes), device="cuda")
-    S = torch.zeros((len(ax), 6), dtype=torch.complex128, device="cuda")
+def _far64(pos, axes, sg, d8, f0, nt, nph, d):
+    """Intensity from face currents in directions d of the grid, in doubles."""
+    e = np.asarray(d8, np.float64).reshape(-1, 4, 2) @ np.array([1, 1j])  # E1, E2, eta0 H1, eta0 H2
+    S = np.zeros((len(e), 6), complex)
     for a, (t1, t2) in enumerate(((1, 2), (0, 2), (0, 1))):
-        w = torch.nonzero(ax == a)[:, 0]
-        s = (sg[w] * (-1.0 if a == 1 else 1.0))[:, None]
-        cols = torch.tensor([[t2, t1, 3 + t2, 3 + t1]], device="cuda")
-        S[w[:, None], cols] = torch.stack([e[w, 2], -e[w, 3], -e[w, 0], e[w, 1]], 1) * s
-    th = torch.arange(nt, dtype=torch.float64, device="cuda") * (np.pi / (nt - 1))
-    ph = torch.arange(nph, dtype=torch.float64, device="cuda") * (2 * np.pi / (nph - 1))
-    th, ph = (x.reshape(-1) for x in torch.meshgrid(th, ph, indexing="ij"))
-    r = torch.stack([th.sin() * ph.cos(), th.sin() * ph.sin(), th.cos()], 1)
-    k = 2 * np.pi * f0 / 299792458.0
-    V = torch.cat([torch.polar(torch.ones((len(x), len(ax)), dtype=torch.float64, device="cuda"), k * (x @ pos.T)) @ S
-                   for x in r.split(512)])
-    t = torch.stack([th.cos() * ph.cos(), th.cos() * ph.sin(), -th.sin()], 1).to(V.dtype)
-    p = torch.stack([-ph.sin(), ph.cos(), 0 * ph], 1).to(V.dtype)
-    nt_, np_, lt, lp = ((V[:, a:a + 3] * q).sum(1) for a, q in ((0, t), (0, p), (3, t), (3, p)))
-    return ((lp + nt_).abs() ** 2 + (lt - np_).abs() ** 2).reshape(nt, nph).cpu().numpy()
+        w = np.nonzero(np.asarray(axes) == a)[0]
+        s = sg[w] * (-1.0 if a == 1 else 1.0)
+        for col, x in ((t2, e[w, 2]), (t1, -e[w, 3]), (3 + t2, -e[w, 0]), (3 + t1, e[w, 1])):
+            S[w, col] = s * x
+    th, ph = np.pi * (d // nph) / (nt - 1), 2 * np.pi * (d % nph) / (nph - 1)
+    r = np.stack([np.sin(th) * np.cos(ph), np.sin(th) * np.sin(ph), np.cos(th)], 1)
+    V = np.exp(2j * np.pi * f0 / 299792458.0 * (r @ np.asarray(pos, np.float64).T)) @ S
+    t = np.stack([np.cos(th) * np.cos(ph), np.cos(th) * np.sin(ph), -np.sin(th)], 1)
+    p = np.stack([-np.sin(ph), np.cos(ph), 0 * ph], 1)
+    Nt, Np, Lt, Lp = ((V[:, a:a + 3] * q).sum(1) for a, q in ((0, t), (0, p), (3, t), (3, p)))
+    return np.abs(Lp + Nt) ** 2 + np.abs(Lt - Np) ** 2
+
+
+def _check(got, plain, geometry, f0, grid):
+    """Both results against doubles in the peak's and 400 other directions."""
+    n = grid[0] * grid[1]
+    d = np.unique(np.r_[0, n - 1, got.U.argmax(), plain.U.argmax(), np.random.default_rng(n).integers(0, n, 400)])
+    U = _far64(*geometry, f0, *grid, d)
+    for r in (got, plain):
+        assert np.abs(r.U.reshape(-1)[d] - U).max() < 2e-5 * U.max()
+        assert abs(r.u_max - U.max()) < 2e-5 * U.max()
+    assert np.abs(got.U - plain.U).max() < 4e-5 * U.max()
 
 
 @pytest.mark.parametrize("dims,offset,listed,pec", [
@@ -88,10 +93,7 @@ def test_lattice_matches_doubles(dims, offset, listed, pec, grid):
         assert np.array_equal(got.U, again.U)
         pos, sg = ot.huygens_geometry(dims, sc.origin, sc.dl, cells, axes)
         plain = tlm.far_field(pos, axes, sg, d8, sc.f0, *grid)
-        U = _far64(pos, axes, sg, d8, sc.f0, *grid)
-        for r in (got, plain):
-            assert np.abs(r.U - U).max() < 2e-5 * U.max()
-            assert abs(r.u_max - U.max()) < 2e-5 * U.max()
+        _check(got, plain, (pos, axes, sg, d8), sc.f0, grid)
 
 
 def test_lists_that_are_no_box():
@@ -107,9 +109,9 @@ def test_lists_that_are_no_box():
         d8 = dev.read_huygens()
         pos, sg = ot.huygens_geometry(dims, sc.origin, sc.dl, cells, axes)
         got = tlm.far_field_ctx(dev, sc.origin, 1, sc.f0, *GRID)
-        assert np.array_equal(got.U, tlm.far_field(pos, axes, sg, d8, sc.f0, *GRID).U)
-        U = _far64(pos, axes, sg, d8, sc.f0, *GRID)
-        assert np.abs(got.U - U).max() < 2e-5 * U.max()
+        plain = tlm.far_field(pos, axes, sg, d8, sc.f0, *GRID)
+        assert np.array_equal(got.U, plain.U)
+        _check(got, plain, (pos, axes, sg, d8), sc.f0, GRID)
 
 
 def test_infinite_field_takes_plain_sums():
