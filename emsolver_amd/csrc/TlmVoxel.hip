@@ -1018,6 +1018,40 @@ bool grid_ok(const tlm_voxel_grid *g)
 
 } // namespace
 
+namespace tlmi {
+
+int build_codes(tlm_ctx *c, const uint8_t *mat, int nmat, int *max_id)
+{
+    const long long ncell = (long long)c->nx * c->ny * c->nz;
+    Scratch s;
+    int *dmax, rc;
+    if ((rc = s.get(c, &dmax, 1)))
+        return rc;
+    const int m1 = -1;
+    HIPCHK(c, hipMemcpyAsync(dmax, &m1, sizeof(int), hipMemcpyHostToDevice, c->stream));
+    k_max_diel<<<grid_for(ncell, 4096), kThreads, 0, c->stream>>>(mat, ncell, dmax);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipMemcpyAsync(max_id, dmax, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (*max_id >= nmat)
+        return fail(c, TLM_ERR_ARG, "material id without a yhat/ghat entry");
+    k_codes<<<(unsigned)(c->ny * c->nz + c->nz), 128, 0, c->stream>>>(mat, c->nx, c->ny, c->nz, c->nxy, c->Pp,
+                                                                       c->code);
+    HIPCHK(c, hipGetLastError());
+    const long long nblk = c->P / tlm::kWave;
+    // padded to a multiple of 4 bytes for the step's dword loads of the flags
+    if ((rc = upload(c, &c->uair, (const uint8_t *)nullptr, (size_t)((nblk + 3) / 4 * 4))))
+        return rc;
+    c->fold_marked = false;
+    k_uair<<<(unsigned)((nblk + kThreads - 1) / kThreads), kThreads, 0, c->stream>>>(c->code, nblk,
+                                                                                     c->uair);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return TLM_OK;
+}
+
+} // namespace tlmi
+
 extern "C" {
 
 int tlm_mat_fill(tlm_ctx *c, uint8_t id)
@@ -1341,32 +1375,9 @@ int tlm_upload_mat(tlm_ctx *c, const float *yhat, const float *ghat, int nmat)
         return rc;
     if (nmat < 0 || (nmat > 0 && (!yhat || !ghat)))
         return fail(c, TLM_ERR_ARG, "tlm_upload_mat: bad arguments");
-    const long long ncell = (long long)c->nx * c->ny * c->nz;
-    Scratch s;
-    int *dmax;
-    if ((rc = s.get(c, &dmax, 1)))
-        return rc;
-    const int m1 = -1;
-    HIPCHK(c, hipMemcpyAsync(dmax, &m1, sizeof(int), hipMemcpyHostToDevice, c->stream));
-    k_max_diel<<<grid_for(ncell, 4096), kThreads, 0, c->stream>>>(c->mat, ncell, dmax);
-    HIPCHK(c, hipGetLastError());
     int max_id = -1;
-    HIPCHK(c, hipMemcpyAsync(&max_id, dmax, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (max_id >= nmat)
-        return fail(c, TLM_ERR_ARG, "material id without a yhat/ghat entry");
-    k_codes<<<(unsigned)(c->ny * c->nz + c->nz), 128, 0, c->stream>>>(c->mat, c->nx, c->ny, c->nz,
-                                                                       c->nxy, c->Pp, c->code);
-    HIPCHK(c, hipGetLastError());
-    const long long nblk = c->P / tlm::kWave;
-    // padded to a multiple of 4 bytes for the step's dword loads of the flags
-    if ((rc = upload(c, &c->uair, (const uint8_t *)nullptr, (size_t)((nblk + 3) / 4 * 4))))
+    if ((rc = build_codes(c, c->mat, nmat, &max_id)))
         return rc;
-    c->fold_marked = false;
-    k_uair<<<(unsigned)((nblk + kThreads - 1) / kThreads), kThreads, 0, c->stream>>>(c->code, nblk,
-                                                                                     c->uair);
-    HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     return install_material(c, max_id >= 0, yhat, ghat, nmat, nullptr, nullptr);
 }
 

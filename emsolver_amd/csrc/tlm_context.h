@@ -143,6 +143,11 @@ struct tlm_ctx
 
 namespace tlmi {
 
+// Cell codes and block flags of a device map (cellIndex order, 16-byte aligned);
+// *max_id: its largest dielectric index, -1 if none. Refuses one without an
+// entry among nmat (TlmVoxel.hip).
+int build_codes(tlm_ctx *c, const uint8_t *mat, int nmat, int *max_id);
+
 // Sets hlat from the context's list of faces (TlmFarField.hip).
 int huy_lattice_scan(tlm_ctx *c);
 
