@@ -243,6 +243,14 @@ bool fold_active(const tlm_ctx *c)
                                  step_occupancy(c) > 0);
 }
 
+void mark_fold(tlm_ctx *c, hipStream_t s)
+{
+    if (c->fold_marked)
+        return;
+    hipLaunchKernelGGL(tlm::k_mark_fold, dim3(1), dim3(64), 0, s, c->ucell, c->nuniq, c->uair, c->code);
+    c->fold_marked = true;
+}
+
 tlm::Fold fold_at(const tlm_ctx *c, int n)
 {
     tlm::Fold f;
@@ -505,12 +513,8 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
             return rc;
     }
     const bool pairs = pair_active(c);
-    if ((fold || (pairs && c->nuniq > 0)) && !c->fold_marked)
-    {
-        hipLaunchKernelGGL(tlm::k_mark_fold, dim3(1), dim3(64), 0, c->stream, c->ucell, c->nuniq,
-                           c->uair, c->code);
-        c->fold_marked = true;
-    }
+    if (fold || (pairs && c->nuniq > 0))
+        mark_fold(c, c->stream);
     const int nmon0 = c->nf + c->nh + c->np + c->npr;
     const bool time_kernel = kernel_every > 0;
     const int ntimed = time_kernel ? (nsteps + kernel_every - 1) / kernel_every : 0;

@@ -6,7 +6,8 @@
 // grid gives the same bits alone and in a batch: the per-cell arithmetic and
 // every monitor write are the single-grid code paths, only the launch that
 // drives them differs. A tick advances every active member by one step (see
-// tlm_batch_kernels.h); blocks of ticks are captured in a HIP graph.
+// tlm_batch_kernels.h), two ticks the FP32 members that can by a pair of
+// steps; blocks of ticks are captured in a HIP graph.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Wunused-function" // single-grid kernels of the shared header
 #include "tlm_batch_kernels.h"
@@ -31,8 +32,10 @@ struct Member
 {
     tlm_ctx *c = nullptr;
     int n0 = 0, nend = 0;
-    long long tick0 = 0;
+    tlm::BatchClock c0 = {}, end = {}; // clock at step n0, and after the last step
+    bool pairs = false;                // takes pairs of steps (tlm::BatchMember)
     char *buf[2] = {nullptr, nullptr};
+    float *vs[2] = {nullptr, nullptr};
     long long cells = 0;
     bool range_err = false; // 16-bit storage: a value outgrew its slab scale
 };
@@ -46,8 +49,8 @@ struct tlm_batch
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::string err = "no error";
     std::vector<Member> mem;
-    long long tick = 0; // ticks queued so far (the device counter after they ran)
-    long long *d_tick = nullptr;
+    tlm::BatchClock now = {}; // what is queued so far (the device clock after it ran)
+    tlm::BatchClock *d_now = nullptr;
     tlm_batch_tuning tune = {1, 4, 0, 32, 4};
     bool dirty = true;
     // device tables, rebuilt when the membership or the tuning changes
@@ -59,10 +62,20 @@ struct tlm_batch
     int2 *d_inj = nullptr, *d_mon = nullptr, *d_smax = nullptr;
     size_t inj_cap = 0, mon_cap = 0, smax_cap = 0;
     int ninj = 0, nplan = 0, nmon = 0, nsmax = 0;
+    // the parts of members that take pairs: first entries of inj, last ones of
+    // mon and gmem
+    int ninj_pair = 0, nmon_pair = 0, ngroups_pair[kKinds] = {};
+    tlm::PairGroup *d_pgrp[2] = {}; // without and with stubs
+    size_t pgrp_cap[2] = {};
+    int npgrp[2] = {};
+    int2 *d_pmon = nullptr;
+    size_t pmon_cap = 0;
+    int npmon = 0;
+    bool pair_ready = false;
     int wpb = 4;
-    // captured block of ticks
-    hipGraphExec_t gexec = nullptr;
-    int glen = 0;
+    // captured blocks of ticks, one by one and in pairs
+    hipGraphExec_t gexec[2] = {};
+    int glen[2] = {};
 };
 
 namespace {
@@ -106,10 +119,13 @@ template <class T> int grow(tlm_batch *b, T **p, size_t *cap, size_t n)
 
 void drop_graph(tlm_batch *b)
 {
-    if (b->gexec)
-        (void)hipGraphExecDestroy(b->gexec);
-    b->gexec = nullptr;
-    b->glen = 0;
+    for (int k = 0; k < 2; ++k)
+    {
+        if (b->gexec[k])
+            (void)hipGraphExecDestroy(b->gexec[k]);
+        b->gexec[k] = nullptr;
+        b->glen[k] = 0;
+    }
 }
 
 int kind_of(const tlm_ctx *c)
@@ -120,7 +136,159 @@ int kind_of(const tlm_ctx *c)
 // Current step of a member (clamped to its end).
 int member_now(const tlm_batch *b, const Member &m)
 {
-    return (int)std::min<long long>(m.nend, m.n0 + (b->tick - m.tick0));
+    return (int)std::min<long long>(m.nend, m.n0 + (b->now.tick - m.c0.tick));
+}
+
+// Its current buffers: pulses and stubs by what was queued while it ran.
+void member_bufs(const tlm_batch *b, const Member &m, int *buf, int *vs)
+{
+    const int n = member_now(b, m);
+    const tlm::BatchClock &t = n < m.nend ? b->now : m.end;
+    *buf = (m.pairs ? (int)(t.launch - m.c0.launch) : n - m.n0) & 1;
+    *vs = m.pairs ? (int)(t.pair - m.c0.pair) & 1 : 0;
+}
+
+// Queued: `count` launches of one tick each, or of two (pairs).
+void advance(tlm_batch *b, int count, bool pairs)
+{
+    const int per = pairs ? 2 : 1;
+    for (Member &m : b->mem)
+    {
+        const int left = m.nend - member_now(b, m);
+        if (left > 0 && left <= count * per)
+        {
+            const int k = left / per; // launches to its end: no pair straddles it
+            m.end = {b->now.tick + left, b->now.launch + k, b->now.pair + (pairs ? k : 0)};
+        }
+    }
+    b->now.tick += count * per;
+    b->now.launch += count;
+    b->now.pair += pairs ? count : 0;
+}
+
+// ---- pairs of steps ----
+
+// Whether the batch's launch shape is its own to choose (as pair_active).
+bool pairs_wanted(const tlm_batch *b)
+{
+    const tlm_batch_tuning d = tlm_batch().tune, &t = b->tune;
+    return t.planes == d.planes && t.block_waves == d.block_waves && t.grid_blocks == d.grid_blocks;
+}
+
+// Makes a member ready for pairs if it can take them.
+int member_pairs(tlm_batch *b, Member &m, bool *ok)
+{
+    tlm_ctx *c = m.c;
+    *ok = false;
+    if (!b->pair_ready || !pairs_wanted(b) || c->pf != TLM_PULSE_F32 || !c->pair.ok || c->nuniq > tlm::kFoldMax ||
+        m.nend - member_now(b, m) < 2)
+        return TLM_OK;
+    int rc = c->pair_ready ? (int)TLM_OK : tlmi::prepare_pair(c);
+    if (rc)
+        return bfail(b, rc, c->err);
+    if (!c->pair.ok || (c->stubs && !c->Vs2))
+        return TLM_OK;
+    if (c->nuniq > 0)
+        tlmi::mark_fold(c, c->stream);
+    BCHK(b, hipStreamSynchronize(c->stream));
+    *ok = true;
+    return TLM_OK;
+}
+
+// Tiles of a member: tb blocks beside the rim, as many as a workgroup's waves
+// hold, marched over some `slabs` slabs.
+void pair_shape(const tlm_ctx *c, int slabs, tlm::PairArgs &a)
+{
+    constexpr int C = tlm::kPairBatchCells, waves = tlm::kPairBatchThreads / tlm::kWave;
+    a = {};
+    a.code = c->code;
+    a.uair = c->uair;
+    a.props = c->props;
+    a.nx = c->nx;
+    a.ny = c->ny;
+    a.nz = c->nz;
+    a.Pp = c->Pp;
+    a.rho = c->rho;
+    a.nmat = std::min(c->nmat, 254);
+    a.strips = (int)(c->Pp / tlm::kWave);
+    a.hb = (c->nx + tlm::kWave - 1) / tlm::kWave;
+    if (a.strips <= C * waves)
+        a.hb = 0; // the tile is the slab
+    const int most = std::max(C * waves - 2 * a.hb, C), nt = (a.strips + most - 1) / most;
+    a.tb = ((a.strips + nt - 1) / nt + C - 1) / C * C;
+    a.ntile = (a.strips + a.tb - 1) / a.tb;
+    const int nzc = std::max(1, (c->nz + slabs / 2) / slabs);
+    a.zc = (c->nz + nzc - 1) / nzc;
+    a.mPp = tlm::magic_div((unsigned)c->Pp);
+    a.mnx = tlm::magic_div((unsigned)c->nx);
+    if (c->nuniq > 0)
+        a.fold = tlmi::fold_at(c, 0);
+}
+
+// Slabs per tile: 16 where that leaves two tiles a CU or more, else 8 or 4, in
+// batches of the smallest grids 2. Us a tick at 16 / by this rule: one grid of
+// 64^3 25.2 / 8.7, four of 32 to 64 cells an axis 26.0 / 12.6 (13.2 at 2), 64
+// of 16 to 40 62 / 50, 64 of 32 to 128 264 / 264 (10 slabs 262, 32 270).
+int pair_slabs(const tlm_batch *b)
+{
+    int slabs = 16;
+    for (; slabs > 2; slabs /= 2)
+    {
+        long long n = 0;
+        for (const Member &m : b->mem)
+            if (m.pairs)
+            {
+                tlm::PairArgs a;
+                pair_shape(m.c, slabs, a);
+                n += (long long)a.ntile * ((a.nz + a.zc - 1) / a.zc);
+            }
+        if (n >= (slabs == 4 ? 128 : 512))
+            break;
+    }
+    return slabs;
+}
+
+// The tiles in launch order: workgroup w runs on XCD w % 8, so the members'
+// tiles of a slab range go together to the XCD with the least to do, largest
+// first, and an XCD's list is every eighth entry.
+std::vector<tlm::PairGroup> pair_order(const std::vector<tlm::BatchMember> &hm, bool stubs)
+{
+    struct Unit
+    {
+        int mem, tz;
+        long long cost;
+    };
+    std::vector<Unit> unit;
+    for (size_t i = 0; i < hm.size(); ++i)
+    {
+        const tlm::PairArgs &a = hm[i].pa;
+        if (!hm[i].pairs || (hm[i].vs[0] != nullptr) != stubs)
+            continue;
+        for (int z = 0; z * a.zc < a.nz; ++z)
+            unit.push_back({(int)i, z, (long long)a.ntile * (a.tb + 2 * a.hb) * (std::min(a.zc, a.nz - z * a.zc) + 2)});
+    }
+    std::stable_sort(unit.begin(), unit.end(), [](const Unit &x, const Unit &y) { return x.cost > y.cost; });
+    std::vector<tlm::PairGroup> list[tlm::kNumXcd];
+    long long load[tlm::kNumXcd] = {};
+    size_t most = 0;
+    for (const Unit &u : unit)
+    {
+        const int x = (int)(std::min_element(load, load + tlm::kNumXcd) - load);
+        load[x] += u.cost;
+        for (int t = 0; t < hm[u.mem].pa.ntile; ++t)
+            list[x].push_back({u.mem, u.tz, t});
+        most = std::max(most, list[x].size());
+    }
+    std::vector<tlm::PairGroup> out(most * tlm::kNumXcd, tlm::PairGroup{-1, 0, 0});
+    for (int x = 0; x < tlm::kNumXcd; ++x)
+        for (size_t l = 0; l < list[x].size(); ++l)
+            out[l * tlm::kNumXcd + x] = list[x][l];
+    return out;
+}
+
+constexpr int pair_batch_lds(bool stubs)
+{
+    return tlm::pair_lds<tlm::kPairBatchCells, tlm::kPairBatchThreads>(stubs ? 254 : 0);
 }
 
 // Rebuilds the member descriptors, the group tables and the monitor entry
@@ -133,13 +301,50 @@ int rebuild(tlm_batch *b)
     const int wpb = b->wpb;
     std::vector<tlm::BatchMember> hm(b->mem.size());
     std::vector<int> gm[kKinds];
-    std::vector<int2> inj, plan, mon, smax;
-    for (size_t i = 0; i < b->mem.size(); ++i)
+    std::vector<int2> inj, inj1, plan, mon, pmon, smax;
+    // first the members that take single steps, then those that take pairs
+    std::vector<size_t> order;
+    for (bool pairs : {false, true})
+        for (size_t i = 0; i < b->mem.size(); ++i)
+        {
+            Member &M = b->mem[i];
+            if (!pairs)
+            {
+                // from here on the member counts from its present step
+                int s = 0, v = 0;
+                member_bufs(b, M, &s, &v);
+                if (s)
+                    std::swap(M.buf[0], M.buf[1]);
+                if (v)
+                    std::swap(M.vs[0], M.vs[1]);
+                M.n0 = member_now(b, M);
+                M.c0 = M.end = b->now;
+                M.c->A = M.buf[0];
+                M.c->B = M.buf[1];
+                if (M.pairs)
+                {
+                    M.c->Vs = M.vs[0];
+                    M.c->Vs2 = M.vs[1];
+                }
+                int rc = member_pairs(b, M, &M.pairs);
+                if (rc)
+                    return rc;
+                M.vs[0] = M.c->Vs;
+                M.vs[1] = M.pairs ? M.c->Vs2 : nullptr;
+            }
+            if (M.pairs == pairs)
+                order.push_back(i);
+        }
+    for (int k = 0; k < kKinds; ++k)
+        b->ngroups_pair[k] = 0;
+    b->nmon_pair = 0;
+    const int slabs = pair_slabs(b);
+    for (size_t i : order)
     {
         const Member &M = b->mem[i];
         tlm_ctx *c = M.c;
         tlm::BatchMember &d = hm[i];
-        std::memset(&d, 0, sizeof(d));
+        d = {};
         const int pl = c->pf == TLM_PULSE_F32 ? b->tune.planes : b->tune.planes16;
         const int zc = pl > 0 ? std::min(pl, c->nz) : c->nz;
         const int nzc = (c->nz + zc - 1) / zc;
@@ -179,7 +384,12 @@ int rebuild(tlm_batch *b)
         a.mnx = tlm::magic_div((unsigned)c->nx);
         d.buf[0] = M.buf[0];
         d.buf[1] = M.buf[1];
-        d.tick0 = M.tick0;
+        d.vs[0] = M.vs[0];
+        d.vs[1] = M.vs[1];
+        d.c0 = M.c0;
+        d.pairs = M.pairs;
+        if (M.pairs)
+            pair_shape(c, slabs, d.pa);
         d.n0 = M.n0;
         d.nend = M.nend;
         d.pf = c->pf;
@@ -214,7 +424,14 @@ int rebuild(tlm_batch *b)
         d.group0 = (int)gm[k].size();
         gm[k].insert(gm[k].end(), groups, (int)i);
         for (int u = 0; u < c->nuniq; ++u)
-            inj.push_back(make_int2((int)i, u));
+            (M.pairs ? inj : inj1).push_back(make_int2((int)i, u));
+        if (M.pairs)
+        {
+            b->ngroups_pair[k] += groups;
+            b->nmon_pair += c->npr + c->np;
+            for (int w = 0; w < (c->npr + 7) / 8 + c->np; ++w)
+                pmon.push_back(make_int2((int)i, w));
+        }
         if (c->pf != TLM_PULSE_F32)
             for (int z = 0; z < c->nz; ++z)
             {
@@ -224,6 +441,8 @@ int rebuild(tlm_batch *b)
         for (int p = 0; p < c->npr + c->np; ++p)
             mon.push_back(make_int2((int)i, p));
     }
+    b->ninj_pair = (int)inj.size();
+    inj.insert(inj.end(), inj1.begin(), inj1.end());
     b->ninj = (int)inj.size();
     b->nplan = (int)plan.size();
     inj.insert(inj.end(), plan.begin(), plan.end());
@@ -254,55 +473,148 @@ int rebuild(tlm_batch *b)
         BCHK(b, hipMemcpy(b->d_gmem[k], gm[k].data(), gm[k].size() * sizeof(int),
                           hipMemcpyHostToDevice));
     }
+    for (int k = 0; k < 2; ++k)
+    {
+        const std::vector<tlm::PairGroup> g = pair_order(hm, k != 0);
+        b->npgrp[k] = (int)g.size();
+        if (g.empty())
+            continue;
+        if ((rc = grow(b, &b->d_pgrp[k], &b->pgrp_cap[k], g.size())))
+            return rc;
+        BCHK(b, hipMemcpy(b->d_pgrp[k], g.data(), g.size() * sizeof(g[0]), hipMemcpyHostToDevice));
+    }
+    b->npmon = (int)pmon.size();
+    if (!pmon.empty())
+    {
+        if ((rc = grow(b, &b->d_pmon, &b->pmon_cap, pmon.size())))
+            return rc;
+        BCHK(b, hipMemcpy(b->d_pmon, pmon.data(), pmon.size() * sizeof(int2), hipMemcpyHostToDevice));
+    }
     b->dirty = false;
     return TLM_OK;
 }
 
-// One kind's step launch; with_mon appends the workgroups that take the
-// tick's probe and port records.
-template <bool S, int PF> void launch_kind(tlm_batch *b, int k, bool with_mon)
+// One kind's step launch over its first ng groups; nmon > 0 appends the
+// workgroups that take the first nmon records of the tick.
+template <bool S, int PF> void launch_kind(tlm_batch *b, int k, int ng, int nmon)
 {
-    const int ng = b->ngroups[k];
     const int blocks = b->tune.grid_blocks > 0 ? std::min(ng, b->tune.grid_blocks) : ng;
     const int bt = b->wpb * tlm::kWave;
-    const int mon_blocks = with_mon && b->nmon > 0 ? (b->nmon + bt - 1) / bt : 0;
+    const int mon_blocks = (nmon + bt - 1) / bt;
     hipLaunchKernelGGL((tlm::k_step_batch<S, PF>), dim3(blocks + mon_blocks), dim3(bt), 0,
-                       b->stream, b->d_mem, b->d_gmem[k], ng, b->d_tick, b->d_mon, b->nmon,
+                       b->stream, b->d_mem, b->d_gmem[k], ng, b->d_now, b->d_mon, nmon,
                        blocks);
 }
 
-void queue_tick(tlm_batch *b)
+// One tick of all members, or of those that do not take pairs; the clock goes
+// on by `by`.
+void queue_tick(tlm_batch *b, bool all, tlm::BatchClock by)
 {
-    if (b->ninj + b->nplan > 0)
+    const int skip = all ? 0 : b->ninj_pair, ninj = b->ninj - skip;
+    if (ninj + b->nplan > 0)
     {
-        const int n = b->ninj + b->nplan, t = 128;
+        const int n = ninj + b->nplan, t = 128;
         hipLaunchKernelGGL(tlm::k_inject_batch, dim3((n + t - 1) / t), dim3(t), 0, b->stream,
-                           b->d_mem, b->d_inj, b->ninj, b->nplan, b->d_tick);
+                           b->d_mem, b->d_inj + skip, ninj, b->nplan, b->d_now);
     }
     // the records ride with the first kind that has members
-    bool mon = true;
+    int mon = b->nmon - (all ? 0 : b->nmon_pair);
     auto kind = [&](int k, auto launch) {
-        if (!b->ngroups[k])
+        const int ng = b->ngroups[k] - (all ? 0 : b->ngroups_pair[k]);
+        if (!ng)
             return;
-        launch(k, mon);
-        mon = false;
+        launch(k, ng, mon);
+        mon = 0;
     };
-    kind(0, [&](int k, bool m) { launch_kind<false, tlm::PF_F32>(b, k, m); });
-    kind(1, [&](int k, bool m) { launch_kind<false, tlm::PF_F16>(b, k, m); });
-    kind(2, [&](int k, bool m) { launch_kind<false, tlm::PF_BF16>(b, k, m); });
-    kind(3, [&](int k, bool m) { launch_kind<true, tlm::PF_F32>(b, k, m); });
-    kind(4, [&](int k, bool m) { launch_kind<true, tlm::PF_F16>(b, k, m); });
-    kind(5, [&](int k, bool m) { launch_kind<true, tlm::PF_BF16>(b, k, m); });
-    if (mon && b->nmon > 0)
+    kind(0, [&](int k, int ng, int m) { launch_kind<false, tlm::PF_F32>(b, k, ng, m); });
+    kind(1, [&](int k, int ng, int m) { launch_kind<false, tlm::PF_F16>(b, k, ng, m); });
+    kind(2, [&](int k, int ng, int m) { launch_kind<false, tlm::PF_BF16>(b, k, ng, m); });
+    kind(3, [&](int k, int ng, int m) { launch_kind<true, tlm::PF_F32>(b, k, ng, m); });
+    kind(4, [&](int k, int ng, int m) { launch_kind<true, tlm::PF_F16>(b, k, ng, m); });
+    kind(5, [&](int k, int ng, int m) { launch_kind<true, tlm::PF_BF16>(b, k, ng, m); });
+    if (mon > 0)
     {
         // no member with step groups (cannot happen with active members):
         // the records alone, through an empty step grid
-        launch_kind<false, tlm::PF_F32>(b, 0, true);
+        launch_kind<false, tlm::PF_F32>(b, 0, 0, mon);
     }
     if (b->nsmax > 0)
         hipLaunchKernelGGL(tlm::k_slab_max_batch, dim3(b->nsmax), dim3(256), 0, b->stream,
-                           b->d_mem, b->d_smax, b->d_tick);
-    hipLaunchKernelGGL(tlm::k_tick, dim3(1), dim3(64), 0, b->stream, b->d_tick);
+                           b->d_mem, b->d_smax, b->d_now);
+    hipLaunchKernelGGL(tlm::k_tick, dim3(1), dim3(64), 0, b->stream, b->d_now, by);
+}
+
+// Two ticks: the members that take pairs in one launch, then the others' two.
+void queue_pair(tlm_batch *b)
+{
+    constexpr int NT = tlm::kPairBatchThreads;
+    int mon = b->npmon;
+    for (int k = 0; k < 2; ++k)
+    {
+        if (!b->npgrp[k])
+            continue;
+        hipLaunchKernelGGL((k ? tlm::k_step2_batch<true, NT> : tlm::k_step2_batch<false, NT>),
+                           dim3(b->npgrp[k] + (mon + NT / tlm::kWave - 1) / (NT / tlm::kWave)), dim3(NT),
+                           pair_batch_lds(k != 0), b->stream, b->d_mem, b->d_pgrp[k], b->d_now, b->d_pmon, mon,
+                           b->npgrp[k]);
+        mon = 0;
+    }
+    int single = b->ninj - b->ninj_pair + b->nplan;
+    for (int k = 0; k < kKinds; ++k)
+        single += b->ngroups[k] - b->ngroups_pair[k];
+    if (!single)
+    {
+        hipLaunchKernelGGL(tlm::k_tick, dim3(1), dim3(64), 0, b->stream, b->d_now, tlm::BatchClock{2, 1, 1});
+        return;
+    }
+    queue_tick(b, false, {1, 0, 0});
+    queue_tick(b, false, {1, 1, 1});
+}
+
+// Queues `count` ticks, or pairs of ticks, in captured blocks of the tuning's
+// length as far as they go.
+int queue_blocks(tlm_batch *b, int count, bool pairs)
+{
+    auto one = [&] {
+        if (pairs)
+            queue_pair(b);
+        else
+            queue_tick(b, true, {1, 1, 0});
+    };
+    const int k = pairs ? 1 : 0, L = pairs ? b->tune.graph_ticks / 2 : b->tune.graph_ticks;
+    int left = count;
+    if (L > 0 && left >= L)
+    {
+        if (!b->gexec[k] || b->glen[k] != L)
+        {
+            if (b->gexec[k])
+                (void)hipGraphExecDestroy(b->gexec[k]);
+            b->gexec[k] = nullptr;
+            hipGraph_t g = nullptr;
+            BCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
+            for (int t = 0; t < L; ++t)
+                one();
+            BCHK(b, hipStreamEndCapture(b->stream, &g));
+            hipError_t e = hipGraphInstantiate(&b->gexec[k], g, nullptr, nullptr, 0);
+            (void)hipGraphDestroy(g);
+            if (e != hipSuccess)
+            {
+                b->gexec[k] = nullptr;
+                return bhip(b, e, "hipGraphInstantiate");
+            }
+            b->glen[k] = L;
+        }
+        while (left >= L)
+        {
+            BCHK(b, hipGraphLaunch(b->gexec[k], b->stream));
+            left -= L;
+        }
+    }
+    for (; left > 0; --left)
+        one();
+    BCHK(b, hipGetLastError());
+    advance(b, count, pairs);
+    return TLM_OK;
 }
 
 int queue_ticks(tlm_batch *b, int nticks)
@@ -313,37 +625,29 @@ int queue_ticks(tlm_batch *b, int nticks)
         if (rc)
             return rc;
     }
-    int left = nticks;
-    const int L = b->tune.graph_ticks;
-    if (L > 0 && left >= L)
+    for (int left = nticks; left > 0;)
     {
-        if (!b->gexec || b->glen != L)
+        // as many pairs as end at no member's odd step; with none, a single
+        // tick; without members that take pairs, single ticks throughout
+        int count = left / 2;
+        bool any = false;
+        for (const Member &m : b->mem)
         {
-            drop_graph(b);
-            hipGraph_t g = nullptr;
-            BCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-            for (int t = 0; t < L; ++t)
-                queue_tick(b);
-            BCHK(b, hipStreamEndCapture(b->stream, &g));
-            hipError_t e = hipGraphInstantiate(&b->gexec, g, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(g);
-            if (e != hipSuccess)
-            {
-                b->gexec = nullptr;
-                return bhip(b, e, "hipGraphInstantiate");
-            }
-            b->glen = L;
+            const int r = m.nend - member_now(b, m);
+            if (!m.pairs || r <= 0)
+                continue;
+            any = true;
+            if (r % 2)
+                count = std::min(count, r / 2);
         }
-        while (left >= L)
-        {
-            BCHK(b, hipGraphLaunch(b->gexec, b->stream));
-            left -= L;
-        }
+        const bool pairs = any && count > 0;
+        if (!pairs)
+            count = any ? 1 : left;
+        int rc = queue_blocks(b, count, pairs);
+        if (rc)
+            return rc;
+        left -= pairs ? 2 * count : count;
     }
-    for (; left > 0; --left)
-        queue_tick(b);
-    BCHK(b, hipGetLastError());
-    b->tick += nticks;
     return TLM_OK;
 }
 
@@ -359,9 +663,15 @@ int sync_members(tlm_batch *b)
     {
         tlm_ctx *c = m.c;
         const int now = member_now(b, m);
-        const int s = (now - m.n0) & 1;
+        int s = 0, v = 0;
+        member_bufs(b, m, &s, &v);
         c->A = m.buf[s];
         c->B = m.buf[s ^ 1];
+        if (m.pairs)
+        {
+            c->Vs = m.vs[v];
+            c->Vs2 = m.vs[v ^ 1];
+        }
         c->next_step = now;
         c->steps_run_hi = std::max(c->steps_run_hi, now);
         if (c->npr > 0 && c->nfreq > 0 && c->dft_done < now)
@@ -412,10 +722,19 @@ int tlm_batch_create(int device, tlm_batch **out)
         return bail(e, "hipStreamCreate");
     if ((e = hipEventCreate(&b->ev0)) != hipSuccess || (e = hipEventCreate(&b->ev1)) != hipSuccess)
         return bail(e, "hipEventCreate");
-    if ((e = hipMalloc((void **)&b->d_tick, sizeof(long long))) != hipSuccess)
+    if ((e = hipMalloc((void **)&b->d_now, sizeof(tlm::BatchClock))) != hipSuccess)
         return bail(e, "hipMalloc");
-    if ((e = hipMemset(b->d_tick, 0, sizeof(long long))) != hipSuccess)
+    if ((e = hipMemset(b->d_now, 0, sizeof(tlm::BatchClock))) != hipSuccess)
         return bail(e, "hipMemset");
+    b->pair_ready = true;
+    for (int k = 0; k < 2; ++k)
+        if (hipFuncSetAttribute(k ? (const void *)tlm::k_step2_batch<true, tlm::kPairBatchThreads>
+                                  : (const void *)tlm::k_step2_batch<false, tlm::kPairBatchThreads>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, pair_batch_lds(k != 0)) != hipSuccess)
+        {
+            (void)hipGetLastError();
+            b->pair_ready = false;
+        }
     *out = b;
     return TLM_OK;
 }
@@ -431,8 +750,8 @@ void tlm_batch_destroy(tlm_batch *b)
         m.c->batch = nullptr;
     b->mem.clear();
     drop_graph(b);
-    for (void *p : {(void *)b->d_tick, (void *)b->d_mem, (void *)b->d_inj, (void *)b->d_mon,
-                    (void *)b->d_smax})
+    for (void *p : {(void *)b->d_now, (void *)b->d_mem, (void *)b->d_inj, (void *)b->d_mon,
+                    (void *)b->d_smax, (void *)b->d_pmon, (void *)b->d_pgrp[0], (void *)b->d_pgrp[1]})
         if (p)
             (void)hipFree(p);
     for (int k = 0; k < kKinds; ++k)
@@ -484,9 +803,10 @@ int tlm_batch_add(tlm_batch *b, tlm_ctx *c, int nsteps)
     m.c = c;
     m.n0 = n0;
     m.nend = n0 + nsteps;
-    m.tick0 = b->tick;
+    m.c0 = m.end = b->now;
     m.buf[0] = c->A;
     m.buf[1] = c->B;
+    m.vs[0] = c->Vs;
     m.cells = (long long)c->nx * c->ny * c->nz;
     b->mem.push_back(m);
     c->batch = b;

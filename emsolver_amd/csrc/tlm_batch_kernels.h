@@ -8,20 +8,31 @@
 // over the concatenated task groups of its members (the first of them also
 // taking every member's probe and port records in extra workgroups), one
 // slab-maximum launch for the 16-bit members and a one-thread launch that
-// advances the device tick. Every launch reads the
-// tick from device memory, so a block of ticks can be captured once in a
-// HIP graph and replayed.
+// advances the device clock. Every launch reads the
+// clock from device memory, so a block of ticks can be captured once in a
+// HIP graph and replayed. FP32 members take two ticks in one launch
+// (k_step2_batch), in which their sources are added, where they can.
 #pragma once
 
 #include "tlm_kernels.h"
+#include "tlm_step2.h"
 
 namespace tlm {
+
+// Ticks done, step launches done (a pair of ticks is one), pairs among them.
+struct BatchClock
+{
+    long long tick, launch, pair;
+};
 
 struct BatchMember
 {
     StepArgs st;        // geometry and pointers; A/B and the scales are picked per tick
-    char *buf[2];       // pulse buffers: buf[0] holds the incident pulses of step n0
-    long long tick0;    // batch tick at which the member runs its step n0
+    PairArgs pa;        // the same for pairs of steps
+    int pairs;          // the member takes pairs: its buffers alternate by launches
+    BatchClock c0;      // the clock at which the member runs its step n0 ...
+    char *buf[2];       // ... and pulse buffers: buf[0] holds the incident pulses of that step
+    float *vs[2];       // its stubs likewise, by pairs
     int n0, nend;       // the member runs steps [n0, nend) in the batch
     int pf;             // PF_*
     int sbase;          // 16-bit: step whose scales are in buffer 0
@@ -49,16 +60,25 @@ struct BatchMember
     int group0;         // first task group of the member in its kind's table
 };
 
-// Step of member m at batch tick `tick`; >= nend once it has finished.
-__device__ __forceinline__ int member_step(const BatchMember &m, long long tick)
+// Step of member m at batch time t; >= nend once it has finished.
+__device__ __forceinline__ int member_step(const BatchMember &m, const BatchClock &t)
 {
-    return m.n0 + (int)(tick - m.tick0);
+    return m.n0 + (int)(t.tick - m.c0.tick);
+}
+// Buffer with the incident pulses of step n.
+__device__ __forceinline__ int member_buf(const BatchMember &m, int n, const BatchClock &t)
+{
+    return (m.pairs ? (int)(t.launch - m.c0.launch) : n - m.n0) & 1;
+}
+__device__ __forceinline__ int member_vs(const BatchMember &m, const BatchClock &t)
+{
+    return m.pairs ? (int)(t.pair - m.c0.pair) & 1 : 0;
 }
 
-__device__ __forceinline__ PulseView member_view(const BatchMember &m, int n)
+__device__ __forceinline__ PulseView member_view(const BatchMember &m, int n, const BatchClock &t)
 {
     PulseView v;
-    v.base = m.buf[(n - m.n0) & 1];
+    v.base = m.buf[member_buf(m, n, t)];
     v.PB = m.st.PB;
     v.Pp = m.st.Pp;
     v.mPp = m.st.mPp;
@@ -75,19 +95,19 @@ __device__ __forceinline__ PulseView member_view(const BatchMember &m, int n)
 // Injection of every member's soft sources (entries (member, unique cell)),
 // then the 16-bit scale planning (entries (member, slab)).
 static __global__ void k_inject_batch(const BatchMember *mem, const int2 *ent, int ninj, int nplan,
-                               const long long *tick_p)
+                               const BatchClock *now)
 {
     const int id = blockIdx.x * blockDim.x + threadIdx.x;
     if (id >= ninj + nplan)
         return;
     const int2 e = ent[id];
     const BatchMember &m = mem[e.x];
-    const int n = member_step(m, *tick_p);
+    const int n = member_step(m, *now);
     if (n >= m.nend)
         return;
     if (id < ninj)
     {
-        const PulseView pv = member_view(m, n);
+        const PulseView pv = member_view(m, n, *now);
         const float over =
             inject_cell(pv, m.ucell[e.y], m.ubeg[e.y], m.ubeg[e.y + 1], m.spol, m.samp, m.sv[n]);
         if (m.pf != PF_F32 && over > m.fmax)
@@ -115,16 +135,16 @@ static __global__ void k_inject_batch(const BatchMember *mem, const int2 *ent, i
 // Probe and port records of every member (entries (member, index): index <
 // npr is a probe, the rest ports).
 __device__ __forceinline__ void monitor_batch_item(const BatchMember *mem, const int2 *ent, int nent,
-                                                   const long long *tick_p, int id)
+                                                   const BatchClock *now, int id)
 {
     if (id >= nent)
         return;
     const int2 e = ent[id];
     const BatchMember &m = mem[e.x];
-    const int n = member_step(m, *tick_p);
+    const int n = member_step(m, *now);
     if (n >= m.nend)
         return;
-    const PulseView pv = member_view(m, n);
+    const PulseView pv = member_view(m, n, *now);
     auto take = [&](auto pf) {
         constexpr int PF = decltype(pf)::value;
         if (e.y < m.npr)
@@ -147,35 +167,36 @@ __device__ __forceinline__ void monitor_batch_item(const BatchMember *mem, const
 // members (they read the incident pulses, which the step only reads).
 template <bool STUBS, int PF>
 __global__ void __launch_bounds__(256) k_step_batch(const BatchMember *mem, const int *gmem,
-                                                    int ngroups, const long long *tick_p,
+                                                    int ngroups, const BatchClock *now,
                                                     const int2 *ment, int nment, int mon_from)
 {
     if ((int)blockIdx.x >= mon_from)
     {
-        monitor_batch_item(mem, ment, nment, tick_p,
+        monitor_batch_item(mem, ment, nment, now,
                            ((int)blockIdx.x - mon_from) * (int)blockDim.x + (int)threadIdx.x);
         return;
     }
     const int lane = threadIdx.x & (kWave - 1);
     const int wpb = blockDim.x / kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const long long tick = *tick_p;
+    const BatchClock t = *now;
     const XcdRange gr = xcd_range(blockIdx.x, mon_from, ngroups);
     double esum = 0.0;
     for (int g = gr.first; g < gr.end; g += gr.step)
     {
         const int mi = gmem[g];
         const BatchMember &m = mem[mi];
-        const int n = member_step(m, tick);
+        const int n = member_step(m, t);
         if (n >= m.nend)
             continue;
         const int task = (g - m.group0) * wpb + wave;
         if (task >= m.st.tasks)
             continue;
         StepArgs a = m.st;
-        const int s = (n - m.n0) & 1;
+        const int s = member_buf(m, n, t);
         a.A = m.buf[s];
         a.B = m.buf[s ^ 1];
+        a.Vs = m.vs[member_vs(m, t)];
         if (PF != PF_F32)
         {
             const int cur = (n - m.sbase) & 1;
@@ -189,12 +210,87 @@ __global__ void __launch_bounds__(256) k_step_batch(const BatchMember *mem, cons
     }
 }
 
+// Blocks per wave and threads of the pairs' tiles. 64 grids of 32 to 128 cells
+// an axis (21.2 M cells), us a tick: 264 with one block in each of 16 waves,
+// 277 of 8 waves; two blocks 295 of 16 waves and 297 of 8.
+constexpr int kPairBatchCells = 1, kPairBatchThreads = 1024;
+
+// A place in the launch of pairs: tile (tz, tt) of a member; member -1: none.
+struct PairGroup
+{
+    int mem, tz, tt;
+};
+
+// Steps n and n+1 of the FP32 members of one kind that take pairs, one tile
+// per workgroup (k_step2). Workgroups from mon_from on take both steps'
+// probe and port records, a wave each (ment: member, wave).
+template <bool STUBS, int NT>
+__global__ void __launch_bounds__(NT, kPairOcc)
+    k_step2_batch(const BatchMember *mem, const PairGroup *grp, const BatchClock *now, const int2 *ment, int nment,
+                  int mon_from)
+{
+    extern __shared__ float lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const bool mon = (int)blockIdx.x >= mon_from;
+    int mi, sub = 0;
+    PairGroup g = {-1, 0, 0};
+    if (mon)
+    {
+        const int id = ((int)blockIdx.x - mon_from) * (NT / kWave) + wave;
+        if (id >= nment)
+            return;
+        const int2 e = ment[id];
+        mi = e.x;
+        sub = e.y;
+    }
+    else
+    {
+        g = grp[blockIdx.x];
+        mi = g.mem;
+    }
+    if (mi < 0)
+        return;
+    const BatchMember &m = mem[mi];
+    const BatchClock t = *now;
+    const int n = member_step(m, t);
+    if (n + 1 >= m.nend)
+        return;
+    PairArgs a = m.pa;
+    const int s = member_buf(m, n, t), vs = member_vs(m, t);
+    a.A = m.buf[s];
+    a.B = m.buf[s ^ 1];
+    a.Vs = m.vs[vs];
+    a.Vs2 = m.vs[vs ^ 1];
+    a.fold.sv = m.sv[n];
+    a.sv1 = m.sv[n + 1];
+    if (mon)
+    {
+        MonitorArgs o = {};
+        o.pv = member_view(m, n, t);
+        o.pv.fold = a.fold;
+        o.n = n;
+        o.np = m.np;
+        o.pcells = m.pcells;
+        o.poff = m.poff;
+        o.ppol = m.ppol;
+        o.ploop = m.ploop;
+        o.prec = m.prec;
+        o.npr = m.npr;
+        o.prcell = m.prcell;
+        o.inv_dl = m.inv_dl;
+        o.prrec = m.prrec;
+        monitor_pair(o, a, sub);
+        return;
+    }
+    pair_tile<STUBS, false, kPairBatchCells, NT>(a, g.tz, g.tt, (a.tb + 2 * a.hb) / kPairBatchCells, lds);
+}
+
 // Per-slab maxima of the 16-bit members (one workgroup per (member, slab)).
-static __global__ void k_slab_max_batch(const BatchMember *mem, const int2 *ent, const long long *tick_p)
+static __global__ void k_slab_max_batch(const BatchMember *mem, const int2 *ent, const BatchClock *now)
 {
     const int2 e = ent[blockIdx.x];
     const BatchMember &m = mem[e.x];
-    const int n = member_step(m, *tick_p);
+    const int n = member_step(m, *now);
     if (n >= m.nend)
         return;
     __shared__ float s[256];
@@ -214,11 +310,15 @@ static __global__ void k_slab_max_batch(const BatchMember *mem, const int2 *ent,
         m.mreg[e.y] = s[0];
 }
 
-// End of a tick.
-static __global__ void k_tick(long long *tick_p)
+// Advances the clock.
+static __global__ void k_tick(BatchClock *now, BatchClock by)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0)
-        *tick_p += 1;
+    {
+        now->tick += by.tick;
+        now->launch += by.launch;
+        now->pair += by.pair;
+    }
 }
 
 } // namespace tlm

@@ -148,6 +148,14 @@ namespace tlmi {
 // entry among nmat (TlmVoxel.hip).
 int build_codes(tlm_ctx *c, const uint8_t *mat, int nmat, int *max_id);
 
+// First pair of steps after an upload: the second stub buffer and the kernels'
+// limits. Clears pair.ok where there is no room.
+int prepare_pair(tlm_ctx *c);
+// Marks the blocks and cells of the sources that the step adds itself.
+void mark_fold(tlm_ctx *c, hipStream_t s);
+// Those sources at step n.
+tlm::Fold fold_at(const tlm_ctx *c, int n);
+
 // Sets hlat from the context's list of faces (TlmFarField.hip).
 int huy_lattice_scan(tlm_ctx *c);
 

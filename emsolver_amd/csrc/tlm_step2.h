@@ -282,32 +282,15 @@ template <int C, int NT> constexpr int pair_lds(int nmat)
     return 2 * C * NT * 32 + nmat * 8;
 }
 
+// Tile tt of the slabs' tiles from slab tz * zc on, by the workgroup's first
+// nw waves (tb + 2 hb blocks, C to a wave).
 template <bool STUBS, bool ENERGY, int C, int NT>
-__global__ void __launch_bounds__(NT, kPairOcc) k_step2(PairArgs a, MonitorArgs m, int mon_from, int mon_plane)
+__device__ __forceinline__ void pair_tile(const PairArgs &a, int tz, int tt, int nw, float *lds)
 {
-    extern __shared__ float lds[];
     const int nt = (int)blockDim.x;
-    if ((int)blockIdx.x >= mon_from)
-    {
-        // the faces, probes and ports of both steps, then the plane of step n
-        const int b = (int)blockIdx.x - mon_from;
-        if (b < mon_plane)
-            monitor_pair(m, a, (b * nt + (int)threadIdx.x) / kWave);
-        else if ((b - mon_plane) * nt + (int)threadIdx.x < m.pn)
-            plane_item<PF_F32>(m, (b - mon_plane) * nt + (int)threadIdx.x);
-        return;
-    }
     constexpr int em = C * NT;
     const int lane = threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), nw = nt / kWave;
-    const XcdRange gr = xcd_range_map(blockIdx.x, a.xm);
-    if (gr.first >= gr.end)
-    {
-        if (ENERGY && lane == 0)
-            a.epart[blockIdx.x * nw + wave] = 0.0;
-        return;
-    }
-    const int tz = gr.first / a.ntile, tt = gr.first - tz * a.ntile;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int b0 = tt * a.tb, b1 = min(a.strips, b0 + a.tb); // blocks of the tile
     const int k0 = tz * a.zc, k1 = min(a.nz, k0 + a.zc);
     const int ka = max(0, k0 - 1), klast = min(k1, a.nz - 1); // slabs read
@@ -325,6 +308,8 @@ __global__ void __launch_bounds__(NT, kPairOcc) k_step2(PairArgs a, MonitorArgs 
         }
         __syncthreads();
     }
+    if (wave >= nw)
+        return;
 
     // A wave holds C blocks, all of the tile (waves below ni) or all of the rim.
     const int ni = a.tb / C;
@@ -603,6 +588,32 @@ __global__ void __launch_bounds__(NT, kPairOcc) k_step2(PairArgs a, MonitorArgs 
         if (lane == 0)
             a.epart[blockIdx.x * nw + wave] = esum;
     }
+}
+
+template <bool STUBS, bool ENERGY, int C, int NT>
+__global__ void __launch_bounds__(NT, kPairOcc) k_step2(PairArgs a, MonitorArgs m, int mon_from, int mon_plane)
+{
+    extern __shared__ float lds[];
+    const int nt = (int)blockDim.x, nw = nt / kWave;
+    if ((int)blockIdx.x >= mon_from)
+    {
+        // the faces, probes and ports of both steps, then the plane of step n
+        const int b = (int)blockIdx.x - mon_from;
+        if (b < mon_plane)
+            monitor_pair(m, a, (b * nt + (int)threadIdx.x) / kWave);
+        else if ((b - mon_plane) * nt + (int)threadIdx.x < m.pn)
+            plane_item<PF_F32>(m, (b - mon_plane) * nt + (int)threadIdx.x);
+        return;
+    }
+    const XcdRange gr = xcd_range_map(blockIdx.x, a.xm);
+    if (gr.first >= gr.end)
+    {
+        if (ENERGY && (threadIdx.x & (kWave - 1)) == 0)
+            a.epart[blockIdx.x * nw + threadIdx.x / kWave] = 0.0;
+        return;
+    }
+    const int tz = gr.first / a.ntile;
+    pair_tile<STUBS, ENERGY, C, NT>(a, tz, gr.first - tz * a.ntile, nw, lds);
 }
 
 } // namespace tlm
