@@ -267,7 +267,8 @@ tlm::Fold fold_of(const tlm_ctx *c, int n)
     return fold_active(c) ? fold_at(c, n) : tlm::Fold();
 }
 
-int launch_step(tlm_ctx *c, int n, const tlm::MonitorArgs &m, int nmon, hipEvent_t e0, hipEvent_t e1)
+// last: of a run; before any other step k_plan_inject takes the 16-bit slab maxima.
+int launch_step(tlm_ctx *c, int n, bool last, const tlm::MonitorArgs &m, int nmon, hipEvent_t e0, hipEvent_t e1)
 {
     const bool energy = c->every > 0 && (n % c->every) == 0;
     tlm::StepArgs a;
@@ -315,7 +316,7 @@ int launch_step(tlm_ctx *c, int n, const tlm::MonitorArgs &m, int nmon, hipEvent
         launch_pf<tlm::PF_BF16>(c, a, energy, m, nmon, e0, e1);
     else
         launch_pf<tlm::PF_F32>(c, a, energy, m, nmon, e0, e1);
-    if (c->pf != TLM_PULSE_F32)
+    if (last && c->pf != TLM_PULSE_F32)
         hipLaunchKernelGGL(tlm::k_slab_max, dim3(c->nz), dim3(256), 0, c->stream, c->mpart,
                            c->strips, c->mreg);
     return TLM_OK;
@@ -554,7 +555,13 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
             pl.isc_next = c->iscl[cur ^ 1];
             pl.flag = c->flag;
         }
-        if ((fold || per == 2 ? 0 : c->nuniq) + pl.nz > 0)
+        if (pl.nz > 0 && n > step0)
+        {
+            const int np = (c->nz + tlm::kPlanSlabs - 1) / tlm::kPlanSlabs, g = (c->nuniq + 255) / 256;
+            hipLaunchKernelGGL(tlm::k_plan_inject, dim3(np + g), dim3(256), 0, c->stream, pv, c->ucell, c->ubeg,
+                               c->spol, c->samp, c->nuniq, c->sv, n, pl, c->mpart, c->strips, c->mreg, np);
+        }
+        else if ((fold || per == 2 ? 0 : c->nuniq) + pl.nz > 0)
         {
             int b = 128, g = (c->nuniq + pl.nz + b - 1) / b;
             hipLaunchKernelGGL(tlm::k_inject, dim3(g), dim3(b), 0, c->stream, pv, c->ucell,
@@ -623,7 +630,7 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
                 return rc;
         }
         else
-            launch_step(c, n, m, nmon, e0, e1);
+            launch_step(c, n, n + 1 == end, m, nmon, e0, e1);
         if (c->frame_every > 0 && (n % c->frame_every) == 0 &&
             (int)c->frame_steps.size() < c->frame_max)
         {

@@ -129,7 +129,7 @@ static __global__ void k_inject_batch(const BatchMember *mem, const int2 *ent, i
     pl.sc_next = m.scl[cur ^ 1];
     pl.isc_next = m.iscl[cur ^ 1];
     pl.flag = m.flag;
-    plan_slab(pl, e.y);
+    plan_slab(pl, e.y, pl.mreg + e.y);
 }
 
 // Probe and port records of every member (entries (member, index): index <
