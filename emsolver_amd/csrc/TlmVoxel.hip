@@ -623,74 +623,123 @@ __global__ void k_set_cells(uint8_t *mat, const long long *cells, int n, uint8_t
         mat[cells[t]] = id;
 }
 
-// Cell codes of the padded layout: material id | neighbour-PEC bits; the
-// slab padding is coded PEC (the host build in tlm_upload, on the device).
-// Block r < ny*nz codes row (j, k) = (r % ny, r / ny); block ny*nz + k the
-// padding of slab k.
-__global__ void k_codes(const uint8_t *mat, int nx, int ny, int nz, long long nxy, long long Pp,
-                        uint16_t *code)
+// 0x80 in every byte of x that is 1 (PEC).
+__device__ __forceinline__ unsigned long long pec_bytes(unsigned long long x)
 {
-    const int r = blockIdx.x;
-    if (r >= ny * nz)
-    {
-        const long long base = (long long)(r - ny * nz) * Pp;
-        for (long long p = nxy + threadIdx.x; p < Pp; p += blockDim.x)
-            code[base + p] = 1;
-        return;
-    }
-    const int k = r / ny, j = r - k * ny;
-    const uint8_t *row = mat + (long long)k * nxy + (long long)j * nx;
-    uint16_t *out = code + (long long)k * Pp + (long long)j * nx;
-    for (int i = threadIdx.x; i < nx; i += blockDim.x)
-    {
-        unsigned v = row[i];
-        if (i > 0 && row[i - 1] == 1)
-            v |= tlm::NB_XM;
-        if (i < nx - 1 && row[i + 1] == 1)
-            v |= tlm::NB_XP;
-        if (j > 0 && row[i - nx] == 1)
-            v |= tlm::NB_YM;
-        if (j < ny - 1 && row[i + nx] == 1)
-            v |= tlm::NB_YP;
-        if (k > 0 && row[i - nxy] == 1)
-            v |= tlm::NB_ZM;
-        if (k < nz - 1 && row[i + nxy] == 1)
-            v |= tlm::NB_ZP;
-        out[i] = (uint16_t)v;
-    }
+    constexpr unsigned long long k7f = 0x7f7f7f7f7f7f7f7full;
+    const unsigned long long t = x ^ 0x0101010101010101ull;
+    return ~(((t & k7f) + k7f) | t | k7f);
 }
 
-// Per 64-cell block: bit 0 if all codes are 0 (air with no PEC neighbour),
-// bit 2 if a cell is dielectric (material id >= 2 in the low byte of its
-// code), bits 3 and 4 if one of cells 0-31 / 32-63 is, bit 5 (kBlockClean)
-// if no code is PEC (padding included) or has a neighbour-PEC bit.
-__global__ void k_uair(const uint16_t *code, long long nblk, uint8_t *uair)
+// Cell codes of the padded layout: material id | neighbour-PEC bits; the
+// slab padding is coded PEC. Flags per 64-cell block: bit 0 if all codes are 0
+// (air with no PEC neighbour; a block with padding never qualifies), bit 2 if a
+// cell is dielectric (such blocks load their stubs with their pulses), bits 3
+// and 4 if one of cells 0-31 / 32-63 is, bit 5 (kBlockClean) if no code is PEC
+// (padding included) or has a neighbour-PEC bit.
+// A thread codes eight cells of a slab from seven 8-byte loads (of any
+// alignment), eight threads join for a block's flags. 256^3: 31 us; a cell per
+// thread from seven byte loads took 70, the flags in a pass of their own 14.
+__global__ void k_codes(const uint8_t *mat, int nx, int ny, int nz, long long nxy, long long Pp, tlm::Magic mPp,
+                        tlm::Magic mnx, long long nblk, uint16_t *code, uint8_t *uair)
 {
-    const long long b = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nblk)
+    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= nblk * 8)
         return;
-    const uint4 *q = reinterpret_cast<const uint4 *>(code + b * tlm::kWave);
-    unsigned any = 0, half = 0;
-    bool clean = true;
-    for (int r = 0; r < tlm::kWave / 8; ++r)
+    const long long p = q * 8, k = tlm::mdiv((unsigned)p, mPp), r = p - k * Pp, ncell = nxy * nz, c = k * nxy + r;
+    unsigned w[8];
+    if (r + 8 <= nxy && c >= 8 && c + 16 <= ncell)
     {
-        const uint4 v = q[r];
-        any |= v.x | v.y | v.z | v.w;
-        bool diel = false;
-        for (unsigned w : {v.x, v.y, v.z, v.w})
+        auto at = [&](long long d, bool on) {
+            unsigned long long x = 0;
+            if (on)
+                __builtin_memcpy(&x, mat + c + d, 8);
+            return x;
+        };
+        // a row or slab whose eight bytes reach past the map is read byte by byte below
+        const unsigned long long m = at(0, true), xm = pec_bytes(at(-1, true)), xp = pec_bytes(at(1, true));
+        auto far = [&](long long d) {
+            if (c + d >= 0 && c + d + 8 <= ncell)
+                return pec_bytes(at(d, true));
+            unsigned long long x = 0;
+            for (int e = 0; e < 8; ++e)
+                if (c + d + e >= 0 && c + d + e < ncell && mat[c + d + e] == 1)
+                    x |= 0x80ull << (8 * e);
+            return x;
+        };
+        const unsigned long long ym = far(-nx), yp = far(nx), zm = far(-nxy), zp = far(nxy);
+        int j = (int)tlm::mdiv((unsigned)r, mnx), i = (int)r - j * nx;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
         {
-            diel = diel || (w & 0xFFu) >= 2u || ((w >> 16) & 0xFFu) >= 2u;
-            clean = clean && tlm::code_is_clean(w & 0xFFFFu) && tlm::code_is_clean(w >> 16);
+            auto bit = [&](unsigned long long x) { return (x >> (8 * e + 7)) & 1u; };
+            unsigned v = (unsigned)(m >> (8 * e)) & 0xffu;
+            v |= i > 0 && bit(xm) ? tlm::NB_XM : 0u;
+            v |= i < nx - 1 && bit(xp) ? tlm::NB_XP : 0u;
+            v |= j > 0 && bit(ym) ? tlm::NB_YM : 0u;
+            v |= j < ny - 1 && bit(yp) ? tlm::NB_YP : 0u;
+            v |= k > 0 && bit(zm) ? tlm::NB_ZM : 0u;
+            v |= k < nz - 1 && bit(zp) ? tlm::NB_ZP : 0u;
+            w[e] = v;
+            if (++i == nx)
+            {
+                i = 0;
+                ++j;
+            }
         }
-        if (diel)
-            half |= 8u << (r >> 2); // uint4 r holds cells 8r .. 8r+7
     }
-    uair[b] = (uint8_t)((any == 0 ? 1u : 0u) | (half ? 4u : 0u) | half |
-                        (clean ? tlm::kBlockClean : 0u));
+    else
+    {
+        // the ends of a slab and of the map
+        for (int e = 0; e < 8; ++e)
+        {
+            const long long f = r + e;
+            if (f >= nxy)
+            {
+                w[e] = 1;
+                continue;
+            }
+            const uint8_t *at = mat + c + e;
+            const int j = (int)(f / nx), i = (int)(f - (long long)j * nx);
+            unsigned v = *at;
+            if (i > 0 && at[-1] == 1)
+                v |= tlm::NB_XM;
+            if (i < nx - 1 && at[1] == 1)
+                v |= tlm::NB_XP;
+            if (j > 0 && at[-nx] == 1)
+                v |= tlm::NB_YM;
+            if (j < ny - 1 && at[nx] == 1)
+                v |= tlm::NB_YP;
+            if (k > 0 && at[-nxy] == 1)
+                v |= tlm::NB_ZM;
+            if (k < nz - 1 && at[nxy] == 1)
+                v |= tlm::NB_ZP;
+            w[e] = v;
+        }
+    }
+    unsigned any = 0, diel = 0, dirty = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+    {
+        any |= w[e];
+        diel |= (w[e] & 0xffu) >= 2u;
+        dirty |= !tlm::code_is_clean(w[e]);
+    }
+    *reinterpret_cast<uint4 *>(code + p) =
+        make_uint4(w[0] | w[1] << 16, w[2] | w[3] << 16, w[4] | w[5] << 16, w[6] | w[7] << 16);
+    // bits: 0 a code other than 0, 1 not clean, 2 and 3 a dielectric cell of either half
+    const int t = threadIdx.x & 7;
+    unsigned f = (any ? 1u : 0u) | dirty << 1 | diel << (t < 4 ? 2 : 3);
+    for (int o = 1; o < 8; o <<= 1)
+        f |= __shfl_xor(f, o, 8);
+    if (t == 0)
+        uair[q / 8] = (uint8_t)((f & 1u ? 0u : 1u) | (f & 12u ? 4u : 0u) | (f & 12u) << 1 |
+                                (f & 2u ? 0u : tlm::kBlockClean));
 }
 
 // Largest dielectric index (id - 2) of the map, -1 if none (16 cells per
-// load; the map is a 256-byte aligned allocation).
+// load; the map is a 256-byte aligned allocation). 256^3: 25 us, 38 with four
+// times the waves and an atomic by each.
 __global__ void k_max_diel(const uint8_t *mat, long long n, int *out)
 {
     unsigned m = 0; // largest id seen
@@ -709,8 +758,10 @@ __global__ void k_max_diel(const uint8_t *mat, long long n, int *out)
         for (long long q = n16 * 16 + threadIdx.x; q < n; q += blockDim.x)
             m = max(m, (unsigned)mat[q]);
     int d = m >= 2 ? (int)m - 2 : -1;
-    d = __reduce_max_sync(~0ull, d);
-    if ((threadIdx.x & (tlm::kWave - 1)) == 0 && d >= 0)
+    for (int o = tlm::kWave / 2; o > 0; o >>= 1)
+        d = max(d, __shfl_xor(d, o, tlm::kWave));
+    // most waves find their maximum there already
+    if ((threadIdx.x & (tlm::kWave - 1)) == 0 && d > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
         atomicMax(out, d);
 }
 
@@ -1029,22 +1080,20 @@ int build_codes(tlm_ctx *c, const uint8_t *mat, int nmat, int *max_id)
         return rc;
     const int m1 = -1;
     HIPCHK(c, hipMemcpyAsync(dmax, &m1, sizeof(int), hipMemcpyHostToDevice, c->stream));
-    k_max_diel<<<grid_for(ncell, 4096), kThreads, 0, c->stream>>>(mat, ncell, dmax);
+    k_max_diel<<<grid_for(ncell / 64, 1024), kThreads, 0, c->stream>>>(mat, ncell, dmax);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpyAsync(max_id, dmax, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (*max_id >= nmat)
         return fail(c, TLM_ERR_ARG, "material id without a yhat/ghat entry");
-    k_codes<<<(unsigned)(c->ny * c->nz + c->nz), 128, 0, c->stream>>>(mat, c->nx, c->ny, c->nz, c->nxy, c->Pp,
-                                                                       c->code);
-    HIPCHK(c, hipGetLastError());
     const long long nblk = c->P / tlm::kWave;
     // padded to a multiple of 4 bytes for the step's dword loads of the flags
     if ((rc = upload(c, &c->uair, (const uint8_t *)nullptr, (size_t)((nblk + 3) / 4 * 4))))
         return rc;
     c->fold_marked = false;
-    k_uair<<<(unsigned)((nblk + kThreads - 1) / kThreads), kThreads, 0, c->stream>>>(c->code, nblk,
-                                                                                     c->uair);
+    k_codes<<<(unsigned)((nblk * 8 + kThreads - 1) / kThreads), kThreads, 0, c->stream>>>(
+        mat, c->nx, c->ny, c->nz, c->nxy, c->Pp, tlm::magic_div((unsigned)c->Pp), tlm::magic_div((unsigned)c->nx), nblk,
+        c->code, c->uair);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return TLM_OK;
@@ -1494,6 +1543,18 @@ int64_t tlm_huygens_mat(tlm_ctx *c, int o)
     return n;
 }
 
+// Cells of a list in cellIndex order of the unpadded grid (on the host, through
+// an array of its own, 0.4 of the 3.9 ms in which a 256^3 mesh scene was set
+// up and its lists read).
+static __global__ void k_list_cells(const long long *pc, long long n, long long Pp, long long nxy, long long *out)
+{
+    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= n)
+        return;
+    const long long k = pc[q] / Pp;
+    out[q] = k * nxy + (pc[q] - k * Pp);
+}
+
 static int64_t read_list(tlm_ctx *c, const long long *dcell, const int *daxis, int n,
                          int64_t *cells, int32_t *axes, int64_t cap)
 {
@@ -1501,21 +1562,22 @@ static int64_t read_list(tlm_ctx *c, const long long *dcell, const int *daxis, i
         return fail(nullptr, TLM_ERR_ARG, "null context");
     HIPCHK(c, hipSetDevice(c->dev));
     const long long m = std::min<long long>(n, std::max<int64_t>(cap, 0));
-    if (m > 0)
+    if (m > 0 && cells)
     {
-        std::vector<long long> pc((size_t)m);
-        std::vector<int> pa((size_t)m);
-        HIPCHK(c, hipMemcpy(pc.data(), dcell, (size_t)m * sizeof(long long), hipMemcpyDeviceToHost));
-        HIPCHK(c, hipMemcpy(pa.data(), daxis, (size_t)m * sizeof(int), hipMemcpyDeviceToHost));
-        for (long long q = 0; q < m; ++q)
-        {
-            const long long k = pc[q] / c->Pp;
-            if (cells)
-                cells[q] = k * c->nxy + (pc[q] - k * c->Pp);
-            if (axes)
-                axes[q] = pa[q];
-        }
+        static_assert(sizeof(long long) == sizeof(int64_t), "one cell index");
+        Scratch s;
+        long long *out;
+        int rc = s.get(c, &out, (size_t)m);
+        if (rc)
+            return rc;
+        k_list_cells<<<(unsigned)((m + kThreads - 1) / kThreads), kThreads, 0, c->stream>>>(dcell, m, c->Pp, c->nxy,
+                                                                                           out);
+        HIPCHK(c, hipGetLastError());
+        HIPCHK(c, hipMemcpyAsync(cells, out, (size_t)m * sizeof(long long), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
     }
+    if (m > 0 && axes)
+        HIPCHK(c, hipMemcpy(axes, daxis, (size_t)m * sizeof(int), hipMemcpyDeviceToHost));
     return n;
 }
 
