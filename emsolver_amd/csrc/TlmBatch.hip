@@ -65,9 +65,9 @@ struct tlm_batch
     // the parts of members that take pairs: first entries of inj, last ones of
     // mon and gmem
     int ninj_pair = 0, nmon_pair = 0, ngroups_pair[kKinds] = {};
-    tlm::PairGroup *d_pgrp[2] = {}; // without and with stubs
-    size_t pgrp_cap[2] = {};
-    int npgrp[2] = {};
+    tlm::PairGroup *d_pgrp[4] = {}; // by stubs (0, 1) and 2 (cells - 1)
+    size_t pgrp_cap[4] = {};
+    int npgrp[4] = {};
     int2 *d_pmon = nullptr;
     size_t pmon_cap = 0;
     int npmon = 0;
@@ -199,7 +199,8 @@ int member_pairs(tlm_batch *b, Member &m, bool *ok)
 // hold, marched over some `slabs` slabs.
 void pair_shape(const tlm_ctx *c, int slabs, tlm::PairArgs &a)
 {
-    constexpr int C = tlm::kPairBatchCells, waves = tlm::kPairBatchThreads / tlm::kWave;
+    constexpr int waves = tlm::kPairBatchThreads / tlm::kWave;
+    const int C = tlm::pair_batch_cells(c->nx);
     a = {};
     a.code = c->code;
     a.uair = c->uair;
@@ -228,7 +229,8 @@ void pair_shape(const tlm_ctx *c, int slabs, tlm::PairArgs &a)
 // Slabs per tile: 16 where that leaves two tiles a CU or more, else 8 or 4, in
 // batches of the smallest grids 2. Us a tick at 16 / by this rule: one grid of
 // 64^3 25.2 / 8.7, four of 32 to 64 cells an axis 26.0 / 12.6 (13.2 at 2), 64
-// of 16 to 40 62 / 50, 64 of 32 to 128 264 / 264 (10 slabs 262, 32 270).
+// of 16 to 40 62 / 50, 64 of 32 to 128 264 / 264 (10 slabs 262, 32 270); longer
+// marches lose in large batches too (six of 200 to 256 806, 863 at 32).
 int pair_slabs(const tlm_batch *b)
 {
     int slabs = 16;
@@ -251,7 +253,7 @@ int pair_slabs(const tlm_batch *b)
 // The tiles in launch order: workgroup w runs on XCD w % 8, so the members'
 // tiles of a slab range go together to the XCD with the least to do, largest
 // first, and an XCD's list is every eighth entry.
-std::vector<tlm::PairGroup> pair_order(const std::vector<tlm::BatchMember> &hm, bool stubs)
+std::vector<tlm::PairGroup> pair_order(const std::vector<tlm::BatchMember> &hm, bool stubs, int cells)
 {
     struct Unit
     {
@@ -262,7 +264,7 @@ std::vector<tlm::PairGroup> pair_order(const std::vector<tlm::BatchMember> &hm, 
     for (size_t i = 0; i < hm.size(); ++i)
     {
         const tlm::PairArgs &a = hm[i].pa;
-        if (!hm[i].pairs || (hm[i].vs[0] != nullptr) != stubs)
+        if (!hm[i].pairs || (hm[i].vs[0] != nullptr) != stubs || tlm::pair_batch_cells(a.nx) != cells)
             continue;
         for (int z = 0; z * a.zc < a.nz; ++z)
             unit.push_back({(int)i, z, (long long)a.ntile * (a.tb + 2 * a.hb) * (std::min(a.zc, a.nz - z * a.zc) + 2)});
@@ -286,9 +288,22 @@ std::vector<tlm::PairGroup> pair_order(const std::vector<tlm::BatchMember> &hm, 
     return out;
 }
 
-constexpr int pair_batch_lds(bool stubs)
+// The kernel of a list (tlm_batch::d_pgrp) and its LDS.
+using PairKernel = void (*)(const tlm::BatchMember *, const tlm::PairGroup *, const tlm::BatchClock *, const int2 *,
+                            int, int);
+PairKernel pair_kernel(int k)
 {
-    return tlm::pair_lds<tlm::kPairBatchCells, tlm::kPairBatchThreads>(stubs ? 254 : 0);
+    constexpr int NT = tlm::kPairBatchThreads;
+    return k == 0   ? tlm::k_step2_batch<false, 1, NT>
+           : k == 1 ? tlm::k_step2_batch<true, 1, NT>
+           : k == 2 ? tlm::k_step2_batch<false, 2, NT>
+                    : tlm::k_step2_batch<true, 2, NT>;
+}
+int pair_lds(int k)
+{
+    constexpr int NT = tlm::kPairBatchThreads;
+    const int nmat = k & 1 ? 254 : 0;
+    return k < 2 ? tlm::pair_lds<1, NT>(nmat) : tlm::pair_lds<2, NT>(nmat);
 }
 
 // Rebuilds the member descriptors, the group tables and the monitor entry
@@ -473,9 +488,9 @@ int rebuild(tlm_batch *b)
         BCHK(b, hipMemcpy(b->d_gmem[k], gm[k].data(), gm[k].size() * sizeof(int),
                           hipMemcpyHostToDevice));
     }
-    for (int k = 0; k < 2; ++k)
+    for (int k = 0; k < 4; ++k)
     {
-        const std::vector<tlm::PairGroup> g = pair_order(hm, k != 0);
+        const std::vector<tlm::PairGroup> g = pair_order(hm, k & 1, 1 + k / 2);
         b->npgrp[k] = (int)g.size();
         if (g.empty())
             continue;
@@ -549,13 +564,13 @@ void queue_pair(tlm_batch *b)
 {
     constexpr int NT = tlm::kPairBatchThreads;
     int mon = b->npmon;
-    for (int k = 0; k < 2; ++k)
+    for (int k = 0; k < 4; ++k)
     {
         if (!b->npgrp[k])
             continue;
-        hipLaunchKernelGGL((k ? tlm::k_step2_batch<true, NT> : tlm::k_step2_batch<false, NT>),
+        hipLaunchKernelGGL(pair_kernel(k),
                            dim3(b->npgrp[k] + (mon + NT / tlm::kWave - 1) / (NT / tlm::kWave)), dim3(NT),
-                           pair_batch_lds(k != 0), b->stream, b->d_mem, b->d_pgrp[k], b->d_now, b->d_pmon, mon,
+                           pair_lds(k), b->stream, b->d_mem, b->d_pgrp[k], b->d_now, b->d_pmon, mon,
                            b->npgrp[k]);
         mon = 0;
     }
@@ -727,10 +742,9 @@ int tlm_batch_create(int device, tlm_batch **out)
     if ((e = hipMemset(b->d_now, 0, sizeof(tlm::BatchClock))) != hipSuccess)
         return bail(e, "hipMemset");
     b->pair_ready = true;
-    for (int k = 0; k < 2; ++k)
-        if (hipFuncSetAttribute(k ? (const void *)tlm::k_step2_batch<true, tlm::kPairBatchThreads>
-                                  : (const void *)tlm::k_step2_batch<false, tlm::kPairBatchThreads>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, pair_batch_lds(k != 0)) != hipSuccess)
+    for (int k = 0; k < 4; ++k)
+        if (hipFuncSetAttribute((const void *)pair_kernel(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                pair_lds(k)) != hipSuccess)
         {
             (void)hipGetLastError();
             b->pair_ready = false;
@@ -751,7 +765,8 @@ void tlm_batch_destroy(tlm_batch *b)
     b->mem.clear();
     drop_graph(b);
     for (void *p : {(void *)b->d_now, (void *)b->d_mem, (void *)b->d_inj, (void *)b->d_mon,
-                    (void *)b->d_smax, (void *)b->d_pmon, (void *)b->d_pgrp[0], (void *)b->d_pgrp[1]})
+                    (void *)b->d_smax, (void *)b->d_pmon, (void *)b->d_pgrp[0], (void *)b->d_pgrp[1],
+                    (void *)b->d_pgrp[2], (void *)b->d_pgrp[3]})
         if (p)
             (void)hipFree(p);
     for (int k = 0; k < kKinds; ++k)

@@ -210,10 +210,16 @@ __global__ void __launch_bounds__(256) k_step_batch(const BatchMember *mem, cons
     }
 }
 
-// Blocks per wave and threads of the pairs' tiles. 64 grids of 32 to 128 cells
-// an axis (21.2 M cells), us a tick: 264 with one block in each of 16 waves,
-// 277 of 8 waves; two blocks 295 of 16 waves and 297 of 8.
-constexpr int kPairBatchCells = 1, kPairBatchThreads = 1024;
+// Threads of the pairs' tiles; blocks per wave (C): one, two where the rim of
+// one row on either side is wide. 64 grids of 32 to 128 cells an axis (21.2 M
+// cells), us a tick: 264 with one block in each of 16 waves, 277 of 8 waves;
+// two blocks 295 of 16 waves and 297 of 8. One / two blocks: 24 grids of 128 to
+// 200 1078 / 1106, six of 200 to 256 806 / 773, four of 300 to 330 1959 / 1374.
+constexpr int kPairBatchThreads = 1024;
+__host__ __device__ inline int pair_batch_cells(int nx)
+{
+    return nx > 192 ? 2 : 1;
+}
 
 // A place in the launch of pairs: tile (tz, tt) of a member; member -1: none.
 struct PairGroup
@@ -224,7 +230,7 @@ struct PairGroup
 // Steps n and n+1 of the FP32 members of one kind that take pairs, one tile
 // per workgroup (k_step2). Workgroups from mon_from on take both steps'
 // probe and port records, a wave each (ment: member, wave).
-template <bool STUBS, int NT>
+template <bool STUBS, int C, int NT>
 __global__ void __launch_bounds__(NT, kPairOcc)
     k_step2_batch(const BatchMember *mem, const PairGroup *grp, const BatchClock *now, const int2 *ment, int nment,
                   int mon_from)
@@ -282,7 +288,7 @@ __global__ void __launch_bounds__(NT, kPairOcc)
         monitor_pair(o, a, sub);
         return;
     }
-    pair_tile<STUBS, false, kPairBatchCells, NT>(a, g.tz, g.tt, (a.tb + 2 * a.hb) / kPairBatchCells, lds);
+    pair_tile<STUBS, false, C, NT>(a, g.tz, g.tt, (a.tb + 2 * a.hb) / C, lds);
 }
 
 // Per-slab maxima of the 16-bit members (one workgroup per (member, slab)).

@@ -15,12 +15,13 @@ pytestmark = pytest.mark.gpu
 
 
 def _members():
-    """Tiles of one and of several a slab (nx to 70: a rim of two blocks), one
+    """Tiles of one and of several a slab, one and two blocks a wave (nx > 192), one
     slab and many, with and without stubs, ends of both parities, a 16-bit
     member and one with more sources than a step adds itself."""
     out = []
     for q, (dims, steps, diel) in enumerate([((70, 41, 9), 33, True), ((64, 20, 40), 40, False), ((33, 35, 18), 7, True),
-                                             ((5, 3, 1), 16, True), ((130, 17, 6), 25, False), ((9, 9, 35), 1, True)]):
+                                             ((5, 3, 1), 16, True), ((130, 17, 6), 25, False), ((9, 9, 35), 1, True),
+                                             ((200, 30, 7), 18, True), ((259, 25, 5), 17, False)]):
         s = _random_scene(*dims, seed=20 + q, diel=diel, rho=(0.0, -1.0, 0.4)[q % 3], steps=steps)
         s.faces, s.energy_every = False, 0
         out.append(s)
