@@ -13,8 +13,9 @@ are resident in HBM before the timed region.
 
 Prints ONE JSON line. `value` is Gcell-updates/s of the timed K steps
 (wall clock between two stream synchronisations). `roofline` prices the
-fused scatter/connect kernel: algorithmic bytes per launch
-(cells * (97 + 24 * f_diel) B for FP32 pulses) over its average launch
+fused scatter/connect kernel, which takes two steps a launch on FP32 grids:
+algorithmic bytes per launch (cells * (97 + 24 * f_diel) B for FP32 pulses,
+each input read once and each output written once) over its average launch
 time, measured with HIP events carried by the step launches of the timed
 region on the context stream, against the 8 TB/s HBM peak. `cpu_baseline`
 times the CPU restatement of the reference algorithm (oracle/, the
@@ -75,6 +76,13 @@ def fp32_slab_fraction(scene):
     return float(hot.mean())
 
 
+def steps_per_launch(scene):
+    """Steps the fused kernel takes in one launch: two for FP32 pulses on grids
+    up to 768 cells wide with at most 32 source cells, else one."""
+    src = {int(c) for c, _, _ in scene.sources} | {int(c) for pc, _, _ in scene.ports for c in pc}
+    return 2 if scene.pulse == "f32" and scene.nx <= 768 and len(src) <= 32 else 1
+
+
 def read_traffic(workload):
     """HBM bytes per launch of the fused kernel from the committed rocprofv3
     PMC summary of this workload, if present (line 'traffic_bytes_per_launch:')."""
@@ -116,8 +124,9 @@ def gpu_run(scene, warmup, steps, tag, plain=False, kernel_every=None):
         "wall_s": wall,
         "gcells": cells * steps / wall / 1e9,
         "ms_per_step": wall * 1e3 / steps,
-        "kernel_ms_avg": ms_kernel,
-        "kernel_launches_timed": len(range(0, steps, kernel_every)),
+        "steps_per_launch": steps_per_launch(sc),
+        "kernel_ms_avg": ms_kernel * steps_per_launch(sc),  # ms_kernel: per step
+        "kernel_launches_timed": len({s // steps_per_launch(sc) for s in range(0, steps, kernel_every)}),
         "kernel_every": kernel_every,
     }
     if plain:
@@ -226,9 +235,10 @@ def batched_run(count=256, sample_every=4):
         "port_absmax": probe_absmax,
     }
     out["speedup_vs_one_at_a_time"] = round(out["gcell_s"] / out["one_at_a_time_gcell_s"], 3)
-    # the mix's algorithmic bytes per cell-update; the rate above covers the
+    # the mix's algorithmic bytes per cell-update (a launch's over its steps); the rate above covers the
     # whole run, the tail where few members are left included
-    bpc = sum(sc.ncell * scene_alg_bytes(sc) for sc in scs) / sum(sc.ncell for sc in scs)
+    bpc = (sum(sc.ncell * scene_alg_bytes(sc) / steps_per_launch(sc) for sc in scs)
+           / sum(sc.ncell for sc in scs))
     out["alg_bytes_per_cell"] = round(bpc, 3)
     out["roofline_frac"] = round(out["gcell_s"] * bpc / HBM_PEAK_GBS, 4)
     path = os.path.join(ROOT, "profiles", f"k_step_batch_{count}.md")
@@ -308,14 +318,14 @@ def served_run(count=200, rate=50.0, baseline_sample=20, seed=5, max_cells=int(2
     summ["one_at_a_time_sample"] = f"first {baseline_sample} requests, FP32, alone"
     summ["speedup_vs_one_at_a_time"] = round(summ["gcell_s"] / summ["one_at_a_time_fp32_gcell_s"], 3)
     # the HBM roofline of this mix: every request's cell-updates at its own
-    # algorithmic bytes (FP16 requests: 16-bit slabs outside the FP32 band)
-    # moved at 8 TB/s; no schedule of the same requests can beat it
+    # algorithmic bytes (FP16 requests: 16-bit slabs outside the FP32 band; FP32
+    # ones half a step's, two steps a launch) moved at 8 TB/s
     work = byts = f16_work = 0.0
     for r in reqs:
         sc = r.build()
         w = sc.ncell * sc.total_steps
         work += w
-        byts += w * scene_alg_bytes(sc)
+        byts += w * scene_alg_bytes(sc) / steps_per_launch(sc)
         f16_work += w if sc.pulse != "f32" else 0.0
     ceil = work / (byts / (HBM_PEAK_GBS * 1e9)) / 1e9
     summ["hbm_ceiling_gcell_s"] = round(ceil, 3)
@@ -527,11 +537,13 @@ def free_space_64_run(with_cpu=True):
     with tlm.open_scene(sc) as dev:
         _, ker = dev.time_steps(0, sc.total_steps, kernel_every=1)
     b = alg_bytes_per_cell(sc)
+    ker *= steps_per_launch(sc)
     out = {
         "grid": [64, 64, 64],
         "steps": sc.total_steps,
         "gcell_s": round(sc.ncell * sc.total_steps / wall / 1e9, 3),
         "kernel_us_avg": round(ker * 1e3, 2),
+        "steps_per_launch": steps_per_launch(sc),
         "achieved_gbs": round(sc.ncell * b / (ker * 1e-3) / 1e9, 1),
         "note": "state (25 MB) resident in the Infinity Cache: not an HBM roofline case; "
                 "gcell_s from 1000 steps with no launch events, kernel_us_avg from a second "
@@ -698,6 +710,7 @@ def main():
             "gcell_s": round(r["gcells"], 3),
             "kernel_ms_avg": round(r["kernel_ms_avg"], 4),
             "kernel_launches_timed": r["kernel_launches_timed"],
+            "steps_per_launch": r["steps_per_launch"],
             "achieved_gbs": round(r["achieved_gbs"], 1),
             "roofline_frac": round(r["achieved_gbs"] / HBM_PEAK_GBS, 4),
             "alg_bytes_per_cell": round(r["alg_bytes_per_cell"], 3),
@@ -787,9 +800,10 @@ def main():
             "unit": "GB/s",
             "frac": round(ach / HBM_PEAK_GBS, 4),
             "traffic": read_traffic(workload),
-            "kernel": "tlm::k_step (fused scatter+connect)",
+            "kernel": "tlm::k_step2 (fused scatter+connect, two steps a launch)",
             "kernel_ms_avg": round(main_run["kernel_ms_avg"], 5),
             "kernel_launches_timed": main_run["kernel_launches_timed"],
+            "steps_per_launch": main_run["steps_per_launch"],
             "alg_bytes_per_launch": int(round(scene.ncell * main_run["alg_bytes_per_cell"])),
         },
         "cpu_baseline": cpu,
