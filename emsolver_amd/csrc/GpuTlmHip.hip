@@ -4,8 +4,8 @@
 // (GpuTlm.cpp:532-884 in the reference) with HIP: one stream per context,
 // device-resident per-step tables, two launches per step (inject, then the
 // fused scatter/connect whose extra workgroups take the monitor records; one
-// where the step adds the sources itself) and no host synchronisation inside
-// a run.
+// where the step adds the sources itself, one for two steps of most FP32 grids)
+// and no host synchronisation inside a run.
 #include "tlm_context.h"
 
 #include <hip/hip_ext.h>
@@ -368,8 +368,8 @@ PairKernel pair_kernel(const tlm_ctx *c, bool energy)
 
 // First pair after an upload: the second stub buffer (all zero, as the stubs
 // are outside dielectric cells) and the kernels' LDS limit. A context without
-// room for the buffer (it takes at most a quarter of what is free) keeps
-// single steps.
+// room for the buffer (above 64 MB it takes at most a quarter of what is free)
+// keeps single steps.
 int prepare_pair(tlm_ctx *c)
 {
     c->pair_ready = true;
@@ -388,8 +388,10 @@ int prepare_pair(tlm_ctx *c)
     const size_t n = (size_t)c->P * 3;
     if (!c->Vs2)
     {
+        // (asking for the free memory takes longer than a small grid's first launches)
+        constexpr size_t kSmall = (size_t)64 << 20;
         size_t fr = 0, tot = 0;
-        if (hipMemGetInfo(&fr, &tot) != hipSuccess || n * sizeof(float) > fr / 4 ||
+        if ((n * sizeof(float) > kSmall && (hipMemGetInfo(&fr, &tot) != hipSuccess || n * sizeof(float) > fr / 4)) ||
             dalloc(c, &c->Vs2, n) != TLM_OK)
         {
             (void)hipGetLastError();
@@ -757,7 +759,12 @@ int read_back(tlm_ctx *c, float *host_out, const tlm::PulseView *pv, float *soa,
     int rc = dalloc(c, &stage, slot * n);
     if (rc)
         return rc;
-    hipError_t e = hipHostMalloc((void **)&pin, slot * n * sizeof(float), hipHostMallocDefault);
+    if (hipHostMalloc((void **)&pin, slot * n * sizeof(float), hipHostMallocDefault) != hipSuccess)
+    {
+        (void)hipGetLastError(); // without pinned memory straight to host_out
+        pin = nullptr;
+    }
+    hipError_t e = hipSuccess;
     std::vector<hipEvent_t> ev((size_t)n, nullptr);
     for (int w = 0; w < n && e == hipSuccess; ++w)
         e = hipEventCreateWithFlags(&ev[w], hipEventDisableTiming);
@@ -765,7 +772,7 @@ int read_back(tlm_ctx *c, float *host_out, const tlm::PulseView *pv, float *soa,
     std::atomic<int> bad{(int)e};
     if (e == hipSuccess)
         on_threads(n, [&](int w) {
-            float *d = stage + slot * w, *h = pin + slot * w;
+            float *d = stage + slot * w;
             hipError_t r = hipSetDevice(c->dev);
             for (long long i; r == hipSuccess && bad == hipSuccess && (i = next++) < nchunk;)
             {
@@ -777,10 +784,11 @@ int read_back(tlm_ctx *c, float *host_out, const tlm::PulseView *pv, float *soa,
                     hipLaunchKernelGGL(tlm::k_stubs_out, dim3(g), dim3(256), 0, c->stream, soa, d, c->nxy, c->Pp, c0,
                                        cnt);
                 const size_t bytes = (size_t)cnt * ncomp * sizeof(float);
+                float *h = pin ? pin + slot * w : host_out + c0 * ncomp;
                 if ((r = hipGetLastError()) == hipSuccess &&
                     (r = hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, c->stream)) == hipSuccess &&
                     (r = hipEventRecord(ev[w], c->stream)) == hipSuccess &&
-                    (r = hipEventSynchronize(ev[w])) == hipSuccess)
+                    (r = hipEventSynchronize(ev[w])) == hipSuccess && pin)
                     std::memcpy(host_out + c0 * ncomp, h, bytes);
             }
             if (r != hipSuccess)
@@ -1086,9 +1094,12 @@ int tlm_upload(tlm_ctx *c, const uint8_t *mat, const float *yhat, const float *g
     int rc = TLM_OK, max_id = -1;
     if (c->uploaded || !map)
     {
-        if ((rc = dalloc(c, &own, (size_t)ncell)))
+        if ((rc = dalloc(c, &own, (size_t)ncell)) == TLM_OK)
+            map = own;
+        else if (!map)
             return rc;
-        map = own;
+        else
+            (void)hipGetLastError(); // the plane that the next step writes: nothing else reads it
     }
     const hipError_t e = hipMemcpyAsync(map, mat, (size_t)ncell, hipMemcpyHostToDevice, c->stream);
     rc = e == hipSuccess ? build_codes(c, map, nmat, &max_id) : hip_fail(c, e, "hipMemcpyAsync");

@@ -435,7 +435,7 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 // Bound by the matrix cores and the loads behind them: 369024 faces x 37 x 73
 // directions 1932 us in the sums over faces, 180 with the mirror images
 // together, 102 with opposite directions too (50 at the matrix cores' FP32 peak,
-// 75 at the rate they reach here without any loads). Three waves a SIMD
+// 70 at the rate they reach here without any loads). Three waves a SIMD
 // and tiles of 32 entries: 179 against 203 with 64 entries and two waves, 194
 // with batches of two row pairs for four.
 template <bool OPP>

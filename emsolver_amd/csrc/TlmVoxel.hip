@@ -1602,14 +1602,22 @@ static int64_t read_list(tlm_ctx *c, const long long *dcell, const int *daxis, i
         static_assert(sizeof(long long) == sizeof(int64_t), "one cell index");
         Scratch s;
         long long *out;
-        int rc = s.get(c, &out, (size_t)m);
-        if (rc)
-            return rc;
-        k_list_cells<<<(unsigned)((m + kThreads - 1) / kThreads), kThreads, 0, c->stream>>>(dcell, m, c->Pp, c->nxy,
-                                                                                           out);
-        HIPCHK(c, hipGetLastError());
-        HIPCHK(c, hipMemcpyAsync(cells, out, (size_t)m * sizeof(long long), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
+        if (s.get(c, &out, (size_t)m) == TLM_OK)
+        {
+            k_list_cells<<<(unsigned)((m + kThreads - 1) / kThreads), kThreads, 0, c->stream>>>(dcell, m, c->Pp,
+                                                                                               c->nxy, out);
+            HIPCHK(c, hipGetLastError());
+            HIPCHK(c, hipMemcpyAsync(cells, out, (size_t)m * sizeof(long long), hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+        }
+        else
+        {
+            // no device memory: in the caller's own array
+            (void)hipGetLastError();
+            HIPCHK(c, hipMemcpy(cells, dcell, (size_t)m * sizeof(long long), hipMemcpyDeviceToHost));
+            for (long long q = 0; q < m; ++q)
+                cells[q] = cells[q] / c->Pp * c->nxy + cells[q] % c->Pp;
+        }
     }
     if (m > 0 && axes)
         HIPCHK(c, hipMemcpy(axes, daxis, (size_t)m * sizeof(int), hipMemcpyDeviceToHost));
