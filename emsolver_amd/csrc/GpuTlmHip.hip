@@ -368,8 +368,8 @@ PairKernel pair_kernel(const tlm_ctx *c, bool energy)
 
 // First pair after an upload: the second stub buffer (all zero, as the stubs
 // are outside dielectric cells) and the kernels' LDS limit. A context without
-// room for the buffer (above 64 MB it takes at most a quarter of what is free)
-// keeps single steps.
+// room for the buffer (it takes at most a quarter of what is free) keeps
+// single steps.
 int prepare_pair(tlm_ctx *c)
 {
     c->pair_ready = true;
@@ -388,10 +388,8 @@ int prepare_pair(tlm_ctx *c)
     const size_t n = (size_t)c->P * 3;
     if (!c->Vs2)
     {
-        // (asking for the free memory takes longer than a small grid's first launches)
-        constexpr size_t kSmall = (size_t)64 << 20;
         size_t fr = 0, tot = 0;
-        if ((n * sizeof(float) > kSmall && (hipMemGetInfo(&fr, &tot) != hipSuccess || n * sizeof(float) > fr / 4)) ||
+        if (hipMemGetInfo(&fr, &tot) != hipSuccess || n * sizeof(float) > fr / 4 ||
             dalloc(c, &c->Vs2, n) != TLM_OK)
         {
             (void)hipGetLastError();
