@@ -289,7 +289,7 @@ std::vector<tlm::PairGroup> pair_order(const std::vector<tlm::BatchMember> &hm, 
 }
 
 // The kernel of a list (tlm_batch::d_pgrp) and its LDS.
-using PairKernel = void (*)(const tlm::BatchMember *, const tlm::PairGroup *, const tlm::BatchClock *, const int2 *,
+using PairKernel = void (*)(const tlm::BatchMember *, const tlm::PairGroup *, tlm::BatchNow, const int2 *,
                             int, int);
 PairKernel pair_kernel(int k)
 {
@@ -511,26 +511,27 @@ int rebuild(tlm_batch *b)
 
 // One kind's step launch over its first ng groups; nmon > 0 appends the
 // workgroups that take the first nmon records of the tick.
-template <bool S, int PF> void launch_kind(tlm_batch *b, int k, int ng, int nmon)
+template <bool S, int PF> void launch_kind(tlm_batch *b, int k, int ng, int nmon, const tlm::BatchNow &now)
 {
     const int blocks = b->tune.grid_blocks > 0 ? std::min(ng, b->tune.grid_blocks) : ng;
     const int bt = b->wpb * tlm::kWave;
     const int mon_blocks = (nmon + bt - 1) / bt;
     hipLaunchKernelGGL((tlm::k_step_batch<S, PF>), dim3(blocks + mon_blocks), dim3(bt), 0,
-                       b->stream, b->d_mem, b->d_gmem[k], ng, b->d_now, b->d_mon, nmon,
+                       b->stream, b->d_mem, b->d_gmem[k], ng, now, b->d_mon, nmon,
                        blocks);
 }
 
-// One tick of all members, or of those that do not take pairs; the clock goes
-// on by `by`.
-void queue_tick(tlm_batch *b, bool all, tlm::BatchClock by)
+// One tick of all members, or of those that do not take pairs, `off` after the
+// device clock.
+void queue_tick(tlm_batch *b, bool all, tlm::BatchClock off)
 {
+    const tlm::BatchNow now{b->d_now, off};
     const int skip = all ? 0 : b->ninj_pair, ninj = b->ninj - skip;
     if (ninj + b->nplan > 0)
     {
         const int n = ninj + b->nplan, t = 128;
         hipLaunchKernelGGL(tlm::k_inject_batch, dim3((n + t - 1) / t), dim3(t), 0, b->stream,
-                           b->d_mem, b->d_inj + skip, ninj, b->nplan, b->d_now);
+                           b->d_mem, b->d_inj + skip, ninj, b->nplan, now);
     }
     // the records ride with the first kind that has members
     int mon = b->nmon - (all ? 0 : b->nmon_pair);
@@ -541,26 +542,25 @@ void queue_tick(tlm_batch *b, bool all, tlm::BatchClock by)
         launch(k, ng, mon);
         mon = 0;
     };
-    kind(0, [&](int k, int ng, int m) { launch_kind<false, tlm::PF_F32>(b, k, ng, m); });
-    kind(1, [&](int k, int ng, int m) { launch_kind<false, tlm::PF_F16>(b, k, ng, m); });
-    kind(2, [&](int k, int ng, int m) { launch_kind<false, tlm::PF_BF16>(b, k, ng, m); });
-    kind(3, [&](int k, int ng, int m) { launch_kind<true, tlm::PF_F32>(b, k, ng, m); });
-    kind(4, [&](int k, int ng, int m) { launch_kind<true, tlm::PF_F16>(b, k, ng, m); });
-    kind(5, [&](int k, int ng, int m) { launch_kind<true, tlm::PF_BF16>(b, k, ng, m); });
+    kind(0, [&](int k, int ng, int m) { launch_kind<false, tlm::PF_F32>(b, k, ng, m, now); });
+    kind(1, [&](int k, int ng, int m) { launch_kind<false, tlm::PF_F16>(b, k, ng, m, now); });
+    kind(2, [&](int k, int ng, int m) { launch_kind<false, tlm::PF_BF16>(b, k, ng, m, now); });
+    kind(3, [&](int k, int ng, int m) { launch_kind<true, tlm::PF_F32>(b, k, ng, m, now); });
+    kind(4, [&](int k, int ng, int m) { launch_kind<true, tlm::PF_F16>(b, k, ng, m, now); });
+    kind(5, [&](int k, int ng, int m) { launch_kind<true, tlm::PF_BF16>(b, k, ng, m, now); });
     if (mon > 0)
     {
         // no member with step groups (cannot happen with active members):
         // the records alone, through an empty step grid
-        launch_kind<false, tlm::PF_F32>(b, 0, 0, mon);
+        launch_kind<false, tlm::PF_F32>(b, 0, 0, mon, now);
     }
     if (b->nsmax > 0)
         hipLaunchKernelGGL(tlm::k_slab_max_batch, dim3(b->nsmax), dim3(256), 0, b->stream,
-                           b->d_mem, b->d_smax, b->d_now);
-    hipLaunchKernelGGL(tlm::k_tick, dim3(1), dim3(64), 0, b->stream, b->d_now, by);
+                           b->d_mem, b->d_smax, now);
 }
 
 // Two ticks: the members that take pairs in one launch, then the others' two.
-void queue_pair(tlm_batch *b)
+void queue_pair(tlm_batch *b, tlm::BatchClock off)
 {
     constexpr int NT = tlm::kPairBatchThreads;
     int mon = b->npmon;
@@ -570,7 +570,7 @@ void queue_pair(tlm_batch *b)
             continue;
         hipLaunchKernelGGL(pair_kernel(k),
                            dim3(b->npgrp[k] + (mon + NT / tlm::kWave - 1) / (NT / tlm::kWave)), dim3(NT),
-                           pair_lds(k), b->stream, b->d_mem, b->d_pgrp[k], b->d_now, b->d_pmon, mon,
+                           pair_lds(k), b->stream, b->d_mem, b->d_pgrp[k], tlm::BatchNow{b->d_now, off}, b->d_pmon, mon,
                            b->npgrp[k]);
         mon = 0;
     }
@@ -578,23 +578,25 @@ void queue_pair(tlm_batch *b)
     for (int k = 0; k < kKinds; ++k)
         single += b->ngroups[k] - b->ngroups_pair[k];
     if (!single)
-    {
-        hipLaunchKernelGGL(tlm::k_tick, dim3(1), dim3(64), 0, b->stream, b->d_now, tlm::BatchClock{2, 1, 1});
         return;
-    }
-    queue_tick(b, false, {1, 0, 0});
-    queue_tick(b, false, {1, 1, 1});
+    queue_tick(b, false, off);
+    ++off.tick;
+    queue_tick(b, false, off);
 }
 
 // Queues `count` ticks, or pairs of ticks, in captured blocks of the tuning's
 // length as far as they go.
 int queue_blocks(tlm_batch *b, int count, bool pairs)
 {
-    auto one = [&] {
-        if (pairs)
-            queue_pair(b);
-        else
-            queue_tick(b, true, {1, 1, 0});
+    const tlm::BatchClock per = pairs ? tlm::BatchClock{2, 1, 1} : tlm::BatchClock{1, 1, 0};
+    auto times = [&](int t) { return tlm::BatchClock{per.tick * t, per.launch * t, per.pair * t}; };
+    auto block = [&](int len) {
+        for (int t = 0; t < len; ++t)
+            if (pairs)
+                queue_pair(b, times(t));
+            else
+                queue_tick(b, true, times(t));
+        hipLaunchKernelGGL(tlm::k_tick, dim3(1), dim3(64), 0, b->stream, b->d_now, times(len));
     };
     const int k = pairs ? 1 : 0, L = pairs ? b->tune.graph_ticks / 2 : b->tune.graph_ticks;
     int left = count;
@@ -607,8 +609,7 @@ int queue_blocks(tlm_batch *b, int count, bool pairs)
             b->gexec[k] = nullptr;
             hipGraph_t g = nullptr;
             BCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-            for (int t = 0; t < L; ++t)
-                one();
+            block(L);
             BCHK(b, hipStreamEndCapture(b->stream, &g));
             hipError_t e = hipGraphInstantiate(&b->gexec[k], g, nullptr, nullptr, 0);
             (void)hipGraphDestroy(g);
@@ -625,8 +626,8 @@ int queue_blocks(tlm_batch *b, int count, bool pairs)
             left -= L;
         }
     }
-    for (; left > 0; --left)
-        one();
+    if (left > 0)
+        block(left);
     BCHK(b, hipGetLastError());
     advance(b, count, pairs);
     return TLM_OK;

@@ -7,8 +7,8 @@
 // planning), one fused step launch per member kind (stubs x storage format)
 // over the concatenated task groups of its members (the first of them also
 // taking every member's probe and port records in extra workgroups), one
-// slab-maximum launch for the 16-bit members and a one-thread launch that
-// advances the device clock. Every launch reads the
+// slab-maximum launch for the 16-bit members; a one-thread launch advances the
+// device clock at the end of a block of ticks. Every launch reads the
 // clock from device memory, so a block of ticks can be captured once in a
 // HIP graph and replayed. FP32 members take two ticks in one launch
 // (k_step2_batch), in which their sources are added, where they can.
@@ -23,6 +23,19 @@ namespace tlm {
 struct BatchClock
 {
     long long tick, launch, pair;
+};
+// Time of a launch: the device clock, and what the block of ticks it belongs to
+// did before it. The clock goes on once a block: with a k_tick after each pair of
+// ticks one grid of 64^3 took 17.8 us a pair, 15.9 so; 16 of 32 to 128 cells an
+// axis 151 and 148.
+struct BatchNow
+{
+    const BatchClock *base;
+    BatchClock off;
+    __device__ __forceinline__ BatchClock operator()() const
+    {
+        return {base->tick + off.tick, base->launch + off.launch, base->pair + off.pair};
+    }
 };
 
 struct BatchMember
@@ -95,19 +108,19 @@ __device__ __forceinline__ PulseView member_view(const BatchMember &m, int n, co
 // Injection of every member's soft sources (entries (member, unique cell)),
 // then the 16-bit scale planning (entries (member, slab)).
 static __global__ void k_inject_batch(const BatchMember *mem, const int2 *ent, int ninj, int nplan,
-                               const BatchClock *now)
+                               BatchNow now)
 {
     const int id = blockIdx.x * blockDim.x + threadIdx.x;
     if (id >= ninj + nplan)
         return;
     const int2 e = ent[id];
     const BatchMember &m = mem[e.x];
-    const int n = member_step(m, *now);
+    const int n = member_step(m, now());
     if (n >= m.nend)
         return;
     if (id < ninj)
     {
-        const PulseView pv = member_view(m, n, *now);
+        const PulseView pv = member_view(m, n, now());
         const float over =
             inject_cell(pv, m.ucell[e.y], m.ubeg[e.y], m.ubeg[e.y + 1], m.spol, m.samp, m.sv[n]);
         if (m.pf != PF_F32 && over > m.fmax)
@@ -135,16 +148,16 @@ static __global__ void k_inject_batch(const BatchMember *mem, const int2 *ent, i
 // Probe and port records of every member (entries (member, index): index <
 // npr is a probe, the rest ports).
 __device__ __forceinline__ void monitor_batch_item(const BatchMember *mem, const int2 *ent, int nent,
-                                                   const BatchClock *now, int id)
+                                                   BatchNow now, int id)
 {
     if (id >= nent)
         return;
     const int2 e = ent[id];
     const BatchMember &m = mem[e.x];
-    const int n = member_step(m, *now);
+    const int n = member_step(m, now());
     if (n >= m.nend)
         return;
-    const PulseView pv = member_view(m, n, *now);
+    const PulseView pv = member_view(m, n, now());
     auto take = [&](auto pf) {
         constexpr int PF = decltype(pf)::value;
         if (e.y < m.npr)
@@ -167,7 +180,7 @@ __device__ __forceinline__ void monitor_batch_item(const BatchMember *mem, const
 // members (they read the incident pulses, which the step only reads).
 template <bool STUBS, int PF>
 __global__ void __launch_bounds__(256) k_step_batch(const BatchMember *mem, const int *gmem,
-                                                    int ngroups, const BatchClock *now,
+                                                    int ngroups, BatchNow now,
                                                     const int2 *ment, int nment, int mon_from)
 {
     if ((int)blockIdx.x >= mon_from)
@@ -179,7 +192,7 @@ __global__ void __launch_bounds__(256) k_step_batch(const BatchMember *mem, cons
     const int lane = threadIdx.x & (kWave - 1);
     const int wpb = blockDim.x / kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const BatchClock t = *now;
+    const BatchClock t = now();
     const XcdRange gr = xcd_range(blockIdx.x, mon_from, ngroups);
     double esum = 0.0;
     for (int g = gr.first; g < gr.end; g += gr.step)
@@ -232,7 +245,7 @@ struct PairGroup
 // probe and port records, a wave each (ment: member, wave).
 template <bool STUBS, int C, int NT>
 __global__ void __launch_bounds__(NT, kPairOcc)
-    k_step2_batch(const BatchMember *mem, const PairGroup *grp, const BatchClock *now, const int2 *ment, int nment,
+    k_step2_batch(const BatchMember *mem, const PairGroup *grp, BatchNow now, const int2 *ment, int nment,
                   int mon_from)
 {
     extern __shared__ float lds[];
@@ -257,7 +270,7 @@ __global__ void __launch_bounds__(NT, kPairOcc)
     if (mi < 0)
         return;
     const BatchMember &m = mem[mi];
-    const BatchClock t = *now;
+    const BatchClock t = now();
     const int n = member_step(m, t);
     if (n + 1 >= m.nend)
         return;
@@ -292,11 +305,11 @@ __global__ void __launch_bounds__(NT, kPairOcc)
 }
 
 // Per-slab maxima of the 16-bit members (one workgroup per (member, slab)).
-static __global__ void k_slab_max_batch(const BatchMember *mem, const int2 *ent, const BatchClock *now)
+static __global__ void k_slab_max_batch(const BatchMember *mem, const int2 *ent, BatchNow now)
 {
     const int2 e = ent[blockIdx.x];
     const BatchMember &m = mem[e.x];
-    const int n = member_step(m, *now);
+    const int n = member_step(m, now());
     if (n >= m.nend)
         return;
     __shared__ float s[256];
