@@ -631,6 +631,8 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
         }
         else
             launch_step(c, n, n + 1 == end, m, nmon, e0, e1);
+        ++c->launches;
+        c->pairs += per == 2;
         if (c->frame_every > 0 && (n % c->frame_every) == 0 &&
             (int)c->frame_steps.size() < c->frame_max)
         {
@@ -1163,6 +1165,7 @@ int install_material(tlm_ctx *c, bool any_diel, const float *yhat, const float *
     if (Vs && c->stubs && (rc = convert(c, Vs, nullptr, c->Vs, 3)))
         return rc;
     c->uploaded = true;
+    c->launches = c->pairs = 0;
     c->energy_steps.clear();
     c->steps_run_hi = 0;
     c->dft_done = 0;
@@ -1659,6 +1662,17 @@ int tlm_time_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *m
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     if (ms_total)
         *ms_total = ms;
+    return TLM_OK;
+}
+
+int tlm_step_launches(const tlm_ctx *c, int64_t *launches, int64_t *pairs)
+{
+    if (!c)
+        return TLM_ERR_ARG;
+    if (launches)
+        *launches = c->launches;
+    if (pairs)
+        *pairs = c->pairs;
     return TLM_OK;
 }
 

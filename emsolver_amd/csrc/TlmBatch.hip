@@ -33,6 +33,7 @@ struct Member
     tlm_ctx *c = nullptr;
     int n0 = 0, nend = 0;
     tlm::BatchClock c0 = {}, end = {}; // clock at step n0, and after the last step
+    long long launches0 = 0, pairs0 = 0; // the context's counts at step n0
     bool pairs = false;                // takes pairs of steps (tlm::BatchMember)
     char *buf[2] = {nullptr, nullptr};
     float *vs[2] = {nullptr, nullptr};
@@ -146,6 +147,15 @@ void member_bufs(const tlm_batch *b, const Member &m, int *buf, int *vs)
     const tlm::BatchClock &t = n < m.nend ? b->now : m.end;
     *buf = (m.pairs ? (int)(t.launch - m.c0.launch) : n - m.n0) & 1;
     *vs = m.pairs ? (int)(t.pair - m.c0.pair) & 1 : 0;
+}
+
+// The context's counts of launches, as of what was queued.
+void member_counts(const tlm_batch *b, const Member &m)
+{
+    const int n = member_now(b, m);
+    const tlm::BatchClock &t = n < m.nend ? b->now : m.end;
+    m.c->launches = m.launches0 + (m.pairs ? t.launch - m.c0.launch : n - m.n0);
+    m.c->pairs = m.pairs0 + (m.pairs ? t.pair - m.c0.pair : 0);
 }
 
 // Queued: `count` launches of one tick each, or of two (pairs).
@@ -332,6 +342,9 @@ int rebuild(tlm_batch *b)
                     std::swap(M.buf[0], M.buf[1]);
                 if (v)
                     std::swap(M.vs[0], M.vs[1]);
+                member_counts(b, M);
+                M.launches0 = M.c->launches;
+                M.pairs0 = M.c->pairs;
                 M.n0 = member_now(b, M);
                 M.c0 = M.end = b->now;
                 M.c->A = M.buf[0];
@@ -688,6 +701,7 @@ int sync_members(tlm_batch *b)
             c->Vs = m.vs[v];
             c->Vs2 = m.vs[v ^ 1];
         }
+        member_counts(b, m);
         c->next_step = now;
         c->steps_run_hi = std::max(c->steps_run_hi, now);
         if (c->npr > 0 && c->nfreq > 0 && c->dft_done < now)
@@ -823,6 +837,8 @@ int tlm_batch_add(tlm_batch *b, tlm_ctx *c, int nsteps)
     m.buf[0] = c->A;
     m.buf[1] = c->B;
     m.vs[0] = c->Vs;
+    m.launches0 = c->launches;
+    m.pairs0 = c->pairs;
     m.cells = (long long)c->nx * c->ny * c->nz;
     b->mem.push_back(m);
     c->batch = b;

@@ -64,6 +64,7 @@ struct tlm_ctx
     } pair;
     bool pair_ready = false; // prepared since the last upload
     float *Vs2 = nullptr;    // the stubs a pair of steps writes (allocated at the first one)
+    long long launches = 0, pairs = 0; // step launches since the last upload, those of two steps
     // state
     int pf = TLM_PULSE_F32; // pulse storage format
     int halo = 8;           // 16-bit formats: FP32 slabs on each side of a source slab

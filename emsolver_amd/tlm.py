@@ -413,6 +413,13 @@ class TlmDevice:
         return {"strips_per_slab": r.value, "slabs_per_task": z.value, "groups": g.value,
                 "threads_per_group": t.value}
 
+    def step_launches(self):
+        """(launches, pairs): launches of the fused step since the last upload,
+        alone or in a batch, and how many of them took two steps."""
+        n, p = C.c_int64(0), C.c_int64(0)
+        self._chk(self.lib.tlm_step_launches(self.h, C.byref(n), C.byref(p)), "tlm_step_launches")
+        return int(n.value), int(p.value)
+
     # ---- readback ----
     def read_state(self):
         V = np.empty(12 * self.n, np.float32)

@@ -244,6 +244,11 @@ int tlm_get_tuning(const tlm_ctx *ctx, tlm_tuning *t);
 int tlm_launch_shape(const tlm_ctx *ctx, int *rows_per_group, int *planes_per_group,
                      int *groups, int *threads_per_group);
 
+/* Launches of the fused step that the context's steps took since its last
+ * upload, alone or (as of the last tlm_batch_sync or tlm_batch_remove) in a
+ * batch, and how many of them took two steps. Either may be NULL. */
+int tlm_step_launches(const tlm_ctx *ctx, int64_t *launches, int64_t *pairs);
+
 /* ScatterUnitarityError / DielScatterUnitarityError (TlmSolver.cpp:116-169)
  * evaluated with the device scatter: returns max |S^T W S - W| for the air
  * node (epsr <= 1) or the stub node with yhat = 4(epsr-1), or a negative

@@ -1,0 +1,88 @@
+"""How many launches the steps of a context took (tlm_step_launches): two steps
+a launch where the solver says so, and single steps where it says so."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from emsolver_amd import scenes, tlm
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(nx, ny, nz, steps, diel=True, sources=1, **kw):
+    mat = np.zeros(nx * ny * nz, np.uint8)
+    if diel:
+        mat[:(mat.size + 1) // 2] = 2
+    s = scenes.Scene(nx, ny, nz, mat, np.full(int(diel), 3.0, np.float32), np.zeros(int(diel), np.float32),
+                     total_steps=steps, name=f"launches_{nx}x{ny}x{nz}", **kw)
+    s.sources = [(int(c), 2, 1.0) for c in np.arange(sources)]
+    s.faces, s.energy_every = False, 0
+    s.probes = np.array([mat.size - 1], np.int64)
+    return s
+
+
+def _launches(sc, block=256, **tuning):
+    with tlm.open_scene(sc) as dev:
+        if tuning:
+            dev.set_tuning(**tuning)
+        for n in range(0, sc.total_steps, block):
+            dev.run(n, min(block, sc.total_steps - n))
+        dev.sync()
+        return dev.step_launches()
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (64, 9, 11), (65, 12, 10), (130, 21, 9), (257, 10, 9), (768, 9, 9),
+                                   (192, 192, 192)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("diel", [False, True])
+def test_fp32_steps_go_in_pairs(shape, diel):
+    assert _launches(_scene(*shape, steps=41, diel=diel, sources=1)) == (21, 20)
+
+
+def test_single_steps():
+    """Wider than 768 cells, more sources than a step adds itself, a launch
+    shape of the caller's, 16-bit pulses, blocks of one step."""
+    sc = _scene(64, 9, 11, steps=40)
+    assert _launches(_scene(769, 5, 4, steps=40)) == (40, 0)
+    assert _launches(_scene(64, 9, 11, steps=40, sources=32)) == (20, 20)
+    assert _launches(_scene(64, 9, 11, steps=40, sources=33)) == (40, 0)
+    assert _launches(sc, fold=1) == (40, 0)
+    assert _launches(dataclasses.replace(sc, pulse="f16")) == (40, 0)
+    assert _launches(sc, block=1) == (40, 0)
+
+
+def test_an_upload_counts_anew():
+    sc = _scene(64, 9, 11, steps=40)
+    with tlm.open_scene(sc) as dev:
+        dev.run(0, 40)
+        yh, gh = tlm.stub_admittances(sc.epsr, sc.sigma, sc.dl)
+        dev.upload(sc.mat, yh, gh)
+        assert dev.step_launches() == (0, 0)
+        dev.run(0, 30)
+        assert dev.step_launches() == (15, 15)
+
+
+def test_batch_members():
+    """Members count what they took part in: pairs while all have an even
+    number of steps left or more than one, single ticks at an odd end."""
+    scs = [_scene(64, 9, 11, steps=40), _scene(33, 20, 7, steps=31, diel=False),
+           dataclasses.replace(_scene(20, 20, 20, steps=24), pulse="f16")]
+    devs = [tlm.open_scene(s) for s in scs]
+    devs[0].run(0, 4)
+    first = devs[0].step_launches()
+    with tlm.TlmBatch() as b:
+        b.add(devs[0], 36)
+        b.add(devs[1], 31)
+        b.add(devs[2], 24)
+        b.run(10)
+        b.sync()
+        assert [d.step_launches() for d in devs] == [(first[0] + 5, first[1] + 5), (5, 5), (10, 0)]
+        b.set_tuning(graph_ticks=0)  # the tables are built again
+        b.run(30)
+        b.sync()
+        # 10 pairs, the odd member's last step, 2 pairs, the last step of 35, none of the rest
+        assert [d.step_launches() for d in devs] == [(first[0] + 19, first[1] + 17), (16, 15), (24, 0)]
+        for d in devs:
+            b.remove(d)
+    for d in devs:
+        d.close()
