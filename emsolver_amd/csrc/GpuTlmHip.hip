@@ -366,8 +366,10 @@ PairKernel pair_kernel(const tlm_ctx *c, bool energy)
     return energy ? pair_kernel_of<false, true>(c) : pair_kernel_of<false, false>(c);
 }
 
-// First pair after an upload: the second stub buffer (all zero, as the stubs
-// are outside dielectric cells) and the kernels' LDS limit. A context without
+// First pair after an upload: the second stub buffer and the kernels' LDS
+// limit. The buffer starts as a copy: no step touches the stubs of the 32-cell
+// halves of a block without a dielectric cell, and a caller may have uploaded
+// some there, which both buffers then hold for good. A context without
 // room for the buffer (it takes at most a quarter of what is free) keeps
 // single steps.
 int prepare_pair(tlm_ctx *c)
@@ -397,7 +399,7 @@ int prepare_pair(tlm_ctx *c)
             return TLM_OK;
         }
     }
-    HIPCHK(c, hipMemsetAsync(c->Vs2, 0, n * sizeof(float), c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->Vs2, c->Vs, n * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
     return TLM_OK;
 }
 
