@@ -322,14 +322,35 @@ int launch_step(tlm_ctx *c, int n, bool last, const tlm::MonitorArgs &m, int nmo
     return TLM_OK;
 }
 
-// Whether pairs of steps may run as one launch: FP32 pulses, the sources few
-// enough to be added in the step, the launch shape automatic (a caller's own
-// shape is for k_step).
+// Whether the context's sources can be added in a pair of steps, and whether a
+// pair is worth it with its monitors. A record of step n+1 takes the loads and
+// scatters of seven cells (PairPulses), which costs more than the pair saves
+// where most of the work are records. Per cell a face costs most when it lies
+// beside others along x (a single step's loads are then whole lines), a face
+// of the Huygens box less, a probe anywhere in the grid more; below 16384 faces the
+// saved launch is worth more than any of them. Us a step, single / pairs:
+//   PEC plates along x and y, 128^3 with 0.05, 0.06, 0.13, 0.5 faces a cell
+//   31.6 / 31.0, 31.5 / 34.6, 32.0 / 50.0, 42.2 / 148; 48^3 with 0.13 and
+//   0.17 6.0 / 5.3 and 6.0 / 6.7, 32^3 with 0.5 5.5 / 4.5;
+//   scattered PEC cells, 128^3 with 0.06, 0.12, 0.28: 54.1 / 41.6, 62.2 / 52.4,
+//   84.5 / 90.4;
+//   a Huygens box, 64^3 with 0.07 and 96^3 with 0.05 11.3 / 8.6 and 22.0 / 18.6;
+//   scattered probes, 128^3 with 0.015, 0.02 and 0.03 39.0 / 34.9, 41.8 / 40.2
+//   and 46.7 / 52.1.
+bool pair_suits(const tlm_ctx *c)
+{
+    const long long ncell = (long long)c->nx * c->ny * c->nz;
+    return c->nuniq <= tlm::kFoldMax &&
+           5LL * c->nf + 3LL * c->nh + 12LL * c->npr <= std::max(5 * 16384LL, ncell / 4);
+}
+
+// Whether pairs of steps may run as one launch: FP32 pulses, the sources and
+// records few enough (pair_suits), the launch shape automatic (a
+// caller's own shape is for k_step).
 bool pair_active(const tlm_ctx *c)
 {
     static const tlm_tuning automatic = tlm_ctx().tune;
-    return c->pair.ok && c->nuniq <= tlm::kFoldMax &&
-           std::memcmp(&c->tune, &automatic, sizeof(automatic)) == 0;
+    return c->pair.ok && pair_suits(c) && std::memcmp(&c->tune, &automatic, sizeof(automatic)) == 0;
 }
 
 // Whether steps n and n+1 may be one pair: the energy, the cut plane and the

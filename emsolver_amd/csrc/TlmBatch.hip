@@ -190,7 +190,7 @@ int member_pairs(tlm_batch *b, Member &m, bool *ok)
 {
     tlm_ctx *c = m.c;
     *ok = false;
-    if (!b->pair_ready || !pairs_wanted(b) || c->pf != TLM_PULSE_F32 || !c->pair.ok || c->nuniq > tlm::kFoldMax ||
+    if (!b->pair_ready || !pairs_wanted(b) || c->pf != TLM_PULSE_F32 || !c->pair.ok || !tlmi::pair_suits(c) ||
         m.nend - member_now(b, m) < 2)
         return TLM_OK;
     int rc = c->pair_ready ? (int)TLM_OK : tlmi::prepare_pair(c);

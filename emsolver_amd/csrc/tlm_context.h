@@ -149,6 +149,9 @@ namespace tlmi {
 // entry among nmat (TlmVoxel.hip).
 int build_codes(tlm_ctx *c, const uint8_t *mat, int nmat, int *max_id);
 
+// Whether a pair of steps can add the context's sources and is worth it with
+// its monitors.
+bool pair_suits(const tlm_ctx *c);
 // First pair of steps after an upload: the second stub buffer and the kernels'
 // limits. Clears pair.ok where there is no room.
 int prepare_pair(tlm_ctx *c);

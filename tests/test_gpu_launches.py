@@ -86,3 +86,40 @@ def test_batch_members():
             b.remove(d)
     for d in devs:
         d.close()
+
+
+def _plates(n, every, probes=1):
+    """PEC plates across z, one every so many slabs: n^2 faces on either side of each."""
+    s = _scene(n, n, n, steps=20, diel=False)
+    v = s.mat.reshape(n, n, n)
+    if every:
+        v[1:n - 1:every] = scenes.MAT_PEC
+    s.faces = True
+    s.probes = np.sort(np.random.default_rng(1).choice(n ** 3, probes, replace=False)).astype(np.int64)
+    return s
+
+
+@pytest.mark.parametrize("n,every,probes,huy,pairs", [
+    (16, 2, 4096, 0, True),                           # a small grid full of them
+    (64, 31, 0, 0, True), (64, 31, 1, 0, False),      # 16384 faces, and one record more
+    (64, 0, 0, 4, True),                              # a Huygens box of 18816
+    (96, 24, 0, 0, False),                            # 73728 faces: 0.08 a cell
+    (96, 95, 10752, 0, True), (96, 95, 10753, 0, False)])
+def test_many_records_take_single_steps(n, every, probes, huy, pairs):
+    sc = _plates(n, every, probes)
+    sc.huy_offset = huy
+    assert _launches(sc) == ((10, 10) if pairs else (20, 0))
+
+
+def test_many_probes_in_a_batch_take_single_steps():
+    few, many = _scene(20, 20, 20, steps=20), _scene(20, 20, 20, steps=20)
+    many.probes = np.arange(6827, dtype=np.int64)  # 12 each: above 81920
+    devs = [tlm.open_scene(s) for s in (few, many)]
+    with tlm.TlmBatch() as b:
+        for d in devs:
+            b.add(d, 20)
+        b.run(20)
+        b.sync()
+        assert [d.step_launches() for d in devs] == [(10, 10), (20, 0)]
+    for d in devs:
+        d.close()
