@@ -4,8 +4,8 @@
 
 compiles ``emsolver_amd/lib/libemsolver_tlm.so`` from the HIP sources under
 ``csrc/`` and the C++ drop-in glue under ``host/`` (TlmSolver facade and
-RunGpuTlm), plus the test programs ``tests/selftest/tlm_selftest`` and
-``tests/selftest/tlm_stop``.
+RunGpuTlm), plus the test programs ``tests/selftest/tlm_selftest``,
+``tests/selftest/tlm_stop`` and ``tests/selftest/tlm_scarce``.
 
 Flags that matter:
   -ffp-contract=off  no fused multiply-add: every a*b+c rounds twice, as the
@@ -56,8 +56,8 @@ def build(verbose: bool = False) -> str:
     tmp = lib + ".tmp"
     _run([HIPCC, *DEVICE, *COMMON, "-shared", "-o", tmp, *srcs], verbose)
     os.replace(tmp, lib)
-    # the self-test and cancellation programs (test infrastructure, live with the tests)
-    for name in ("tlm_selftest", "tlm_stop"):
+    # the self-test, cancellation and scarce-memory programs (test infrastructure, live with the tests)
+    for name in ("tlm_selftest", "tlm_stop", "tlm_scarce"):
         st = os.path.join(ROOT, "tests", "selftest", name + ".cpp")
         if os.path.exists(st):
             exe = os.path.join(ROOT, "tests", "selftest", name)

@@ -350,7 +350,7 @@ bool pair_suits(const tlm_ctx *c)
 bool pair_active(const tlm_ctx *c)
 {
     static const tlm_tuning automatic = tlm_ctx().tune;
-    return c->pair.ok && pair_suits(c) && std::memcmp(&c->tune, &automatic, sizeof(automatic)) == 0;
+    return c->pair.ok && !c->pair_refused && pair_suits(c) && std::memcmp(&c->tune, &automatic, sizeof(automatic)) == 0;
 }
 
 // Whether steps n and n+1 may be one pair: the energy, the cut plane and the
@@ -392,35 +392,36 @@ PairKernel pair_kernel(const tlm_ctx *c, bool energy)
 // halves of a block without a dielectric cell, and a caller may have uploaded
 // some there, which both buffers then hold for good. A context without
 // room for the buffer (it takes at most a quarter of what is free) keeps
-// single steps.
+// single steps until the next upload.
 int prepare_pair(tlm_ctx *c)
 {
     c->pair_ready = true;
+    c->pair_refused = true;
     for (bool energy : {false, true})
     {
         const PairKernel k = pair_kernel(c, energy);
         if (k.lds > kLdsPerCu || hipFuncSetAttribute(k.f, hipFuncAttributeMaxDynamicSharedMemorySize, k.lds) != hipSuccess)
         {
             (void)hipGetLastError();
-            c->pair.ok = false;
             return TLM_OK;
         }
     }
-    if (!c->stubs)
-        return TLM_OK;
     const size_t n = (size_t)c->P * 3;
-    if (!c->Vs2)
+    if (c->stubs && !c->Vs2)
     {
         size_t fr = 0, tot = 0;
         if (hipMemGetInfo(&fr, &tot) != hipSuccess || n * sizeof(float) > fr / 4 ||
-            dalloc(c, &c->Vs2, n) != TLM_OK)
+            hipMalloc((void **)&c->Vs2, n * sizeof(float)) != hipSuccess)
         {
             (void)hipGetLastError();
-            c->pair.ok = false;
+            c->Vs2 = nullptr;
             return TLM_OK;
         }
+        c->owned.push_back(c->Vs2);
     }
-    HIPCHK(c, hipMemcpyAsync(c->Vs2, c->Vs, n * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
+    if (c->stubs)
+        HIPCHK(c, hipMemcpyAsync(c->Vs2, c->Vs, n * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
+    c->pair_refused = false;
     return TLM_OK;
 }
 
@@ -1157,7 +1158,7 @@ int install_material(tlm_ctx *c, bool any_diel, const float *yhat, const float *
         HIPCHK(c, hipMemsetAsync(c->B, 0, (size_t)c->PB * 12, c->stream));
     }
     dfree(c, c->Vs);
-    c->pair_ready = false;
+    c->pair_ready = c->pair_refused = false;
     if (c->stubs)
     {
         if ((rc = dalloc(c, &c->Vs, (size_t)c->P * 3)))

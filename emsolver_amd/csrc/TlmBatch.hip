@@ -196,7 +196,7 @@ int member_pairs(tlm_batch *b, Member &m, bool *ok)
     int rc = c->pair_ready ? (int)TLM_OK : tlmi::prepare_pair(c);
     if (rc)
         return bfail(b, rc, c->err);
-    if (!c->pair.ok || (c->stubs && !c->Vs2))
+    if (c->pair_refused)
         return TLM_OK;
     if (c->nuniq > 0)
         tlmi::mark_fold(c, c->stream);

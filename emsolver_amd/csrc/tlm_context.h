@@ -56,13 +56,14 @@ struct tlm_ctx
     size_t epart_cap = 0;
     // two steps a launch (k_step2): tiles of tb blocks with hb blocks of rim on
     // either side (ntile of them in a slab), marched over zc slabs by nt threads,
-    // a wave holding `cells` blocks; ok: the context may run pairs
+    // a wave holding `cells` blocks; ok: the grid may run pairs
     struct
     {
         bool ok = false;
         int tb = 0, hb = 0, ntile = 0, zc = 0, nt = 0, cells = 0, groups = 0, blocks = 0, chunk = 0;
     } pair;
-    bool pair_ready = false; // prepared since the last upload
+    bool pair_ready = false;   // prepared since the last upload ...
+    bool pair_refused = false; // ... without room for the second stub buffer
     float *Vs2 = nullptr;    // the stubs a pair of steps writes (allocated at the first one)
     long long launches = 0, pairs = 0; // step launches since the last upload, those of two steps
     // state
@@ -153,7 +154,7 @@ int build_codes(tlm_ctx *c, const uint8_t *mat, int nmat, int *max_id);
 // its monitors.
 bool pair_suits(const tlm_ctx *c);
 // First pair of steps after an upload: the second stub buffer and the kernels'
-// limits. Clears pair.ok where there is no room.
+// limits. Sets pair_refused where there is no room.
 int prepare_pair(tlm_ctx *c);
 // Marks the blocks and cells of the sources that the step adds itself.
 void mark_fold(tlm_ctx *c, hipStream_t s);
