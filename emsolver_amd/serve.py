@@ -112,8 +112,17 @@ class TlmServer:
         self.max_cells = int(max_cells)
         self.stats = {}
 
+    @staticmethod
+    def _pair_bytes(sc) -> int:
+        """The second stub buffer that an FP32 member with dielectric cells may
+        take at its first block of ticks: as large as its stubs."""
+        if sc.pulse != "f32" or not sc.has_diel:
+            return 0
+        return (tlm.estimate_bytes(sc.nx, sc.ny, sc.nz, sc.pulse, True)
+                - tlm.estimate_bytes(sc.nx, sc.ny, sc.nz, sc.pulse, False))
+
     def _need_bytes(self, sc) -> int:
-        b = tlm.estimate_bytes(sc.nx, sc.ny, sc.nz, sc.pulse, sc.has_diel)
+        b = tlm.estimate_bytes(sc.nx, sc.ny, sc.nz, sc.pulse, sc.has_diel) + self._pair_bytes(sc)
         if sc.ops is not None:
             b += sc.ncell  # the device material map of a device-built scene
         if sc.pulse != "f32" and sc.fp32_halo >= 0:
@@ -177,6 +186,7 @@ class TlmServer:
                 sc = take(r.rid)
                 need = self._need_bytes(sc)
                 free, _ = tlm.device_memory(self.device)
+                free -= sum(self._pair_bytes(p[2]) for p in pending)  # not taken yet
                 cells = sum(v[1].ncell for v in live.values()) + sum(p[2].ncell for p in pending)
                 over = self.max_cells > 0 and cells + sc.ncell > self.max_cells
                 if (live or pending) and (need + self.hbm_reserve > free or over):
