@@ -1165,6 +1165,8 @@ int install_material(tlm_ctx *c, bool any_diel, const float *yhat, const float *
             return rc;
         HIPCHK(c, hipMemsetAsync(c->Vs, 0, (size_t)c->P * 3 * sizeof(float), c->stream));
     }
+    else
+        dfree(c, c->Vs2);
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (c->pf == TLM_PULSE_F32)
     {

@@ -123,3 +123,14 @@ def test_many_probes_in_a_batch_take_single_steps():
         assert [d.step_launches() for d in devs] == [(10, 10), (20, 0)]
     for d in devs:
         d.close()
+
+
+def test_an_upload_without_dielectrics_gives_both_stub_buffers_back():
+    sc = _scene(128, 128, 128, steps=20)
+    with tlm.open_scene(sc) as dev:
+        dev.run(0, 20)
+        dev.sync()
+        before, _ = tlm.device_memory()
+        dev.upload(np.zeros(sc.ncell, np.uint8))
+        after, _ = tlm.device_memory()
+        assert after - before >= 2 * 12 * sc.ncell - (4 << 20)
