@@ -717,6 +717,26 @@ int sync_members(tlm_batch *b)
     return TLM_OK;
 }
 
+// Ticks for timing a launch shape, `ticks` or so: as many as go in whole pairs
+// where members take pairs (single ticks among them, as at a member's odd end,
+// would be timed for the shape that takes pairs as for one that does not); 0 if
+// a member has to end first.
+int pair_window(const tlm_batch *b, int ticks)
+{
+    int even = ticks + ticks % 2;
+    bool any = false;
+    for (const Member &m : b->mem)
+    {
+        const int r = m.nend - member_now(b, m);
+        if (!m.pairs || r <= 0)
+            continue;
+        any = true;
+        if (r % 2)
+            even = std::min(even, r - 1);
+    }
+    return any ? even : ticks;
+}
+
 long long active_cells(const tlm_batch *b)
 {
     long long n = 0;
@@ -983,9 +1003,12 @@ int tlm_batch_autotune(tlm_batch *b, int ticks_per_candidate, tlm_batch_tuning *
         b->dirty = true;
         float ms = 0.f;
         int64_t cu = 0;
-        int rc = tlm_batch_time(b, 1, &ms, &cu); // warm-up (table rebuild)
+        int rc = tlm_batch_time(b, 2, &ms, &cu); // warm-up (table rebuild, the kernels' first run)
+        int window = ticks_per_candidate;
+        while (!rc && (window = pair_window(b, ticks_per_candidate)) == 0)
+            rc = tlm_batch_time(b, 1, &ms, &cu);
         if (!rc)
-            rc = tlm_batch_time(b, ticks_per_candidate, &ms, &cu);
+            rc = tlm_batch_time(b, window, &ms, &cu);
         if (rc)
         {
             b->tune = keep;

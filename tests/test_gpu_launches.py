@@ -134,3 +134,24 @@ def test_an_upload_without_dielectrics_gives_both_stub_buffers_back():
         dev.upload(np.zeros(sc.ncell, np.uint8))
         after, _ = tlm.device_memory()
         assert after - before >= 2 * 12 * sc.ncell - (4 << 20)
+
+
+@pytest.mark.parametrize("short", [3, 4])
+def test_autotune_times_pairs_as_pairs(short):
+    """With windows of one tick too, and with a member that has one step left
+    when the shape that takes pairs is timed."""
+    scs = [_scene(40, 20, 20, steps=400), _scene(33, 20, 7, steps=400), _scene(20, 20, 20, steps=400)]
+    devs = [tlm.open_scene(s) for s in scs]
+    with tlm.TlmBatch() as b:
+        default = b.get_tuning()
+        b.add(devs[0], 400)
+        b.add(devs[1], 399)
+        b.add(devs[2], 8 * short + 1)  # ends while the candidates are timed
+        b.autotune(1)
+        b.sync()
+        assert all(d.step_launches()[1] > 0 for d in devs[:2])
+        b.set_tuning(**default)
+        for d in devs:
+            b.remove(d)
+    for d in devs:
+        d.close()
