@@ -13,11 +13,12 @@ are resident in HBM before the timed region.
 
 Prints ONE JSON line. `value` is Gcell-updates/s of the timed K steps
 (wall clock between two stream synchronisations). `roofline` prices the
-fused scatter/connect kernel, which takes two steps a launch on FP32 grids:
+fused scatter/connect kernel, which takes one or two steps a launch:
 algorithmic bytes per launch (cells * (97 + 24 * f_diel) B for FP32 pulses,
 each input read once and each output written once) over its average launch
 time, measured with HIP events carried by the step launches of the timed
-region on the context stream, against the 8 TB/s HBM peak. `cpu_baseline`
+region on the context stream and counted by the library, against the 8 TB/s
+HBM peak. `cpu_baseline`
 times the CPU restatement of the reference algorithm (oracle/, the
 reference's threading rule min(16, hw-1)) over a 100-step window of the same
 scene. `extra` holds the other configurations: the 256^3 scene, the 512^3
@@ -76,22 +77,37 @@ def fp32_slab_fraction(scene):
     return float(hot.mean())
 
 
-def steps_per_launch(scene):
-    """Steps the fused kernel takes in one launch: two for FP32 pulses on grids
-    up to 768 cells wide with at most 32 source cells, else one."""
-    src = {int(c) for c, _, _ in scene.sources} | {int(c) for pc, _, _ in scene.ports for c in pc}
-    return 2 if scene.pulse == "f32" and scene.nx <= 768 and len(src) <= 32 else 1
+def kernel_launches(dev, ms_per_step):
+    """The launches that dev.time_steps timed, from its time per step: their
+    number, their steps, and what a launch took on average."""
+    launches, pairs = dev.timed_launches()
+    steps = launches + pairs
+    return {"kernel_ms_avg": ms_per_step * steps / launches, "kernel_launches_timed": launches,
+            "kernel_pairs_timed": pairs, "steps_per_launch": round(steps / launches, 3)}
 
 
-def read_traffic(workload):
+def kernel_name(launches, pairs):
+    one, two = "tlm::k_step", "tlm::k_step2"
+    what = "(fused scatter+connect, "
+    if pairs == 0:
+        return f"{one} {what}one step a launch)"
+    if pairs == launches:
+        return f"{two} {what}two steps a launch)"
+    return f"{two} {what}two steps a launch, {pairs} launches) and {one} ({launches - pairs})"
+
+
+def read_traffic(workload, pairs):
     """HBM bytes per launch of the fused kernel from the committed rocprofv3
-    PMC summary of this workload, if present (line 'traffic_bytes_per_launch:')."""
+    PMC summary of this workload (line 'traffic_bytes_per_launch:'), if there
+    is one of the kernel of two steps (pairs) or of one."""
     path = os.path.join(ROOT, "profiles", f"pmc_k_step_{workload}.md")
     if not os.path.exists(path):
         return None
     with open(path) as f:
-        m = re.search(r"traffic_bytes_per_launch:\s*([0-9.eE+]+)", f.read())
-    return float(m.group(1)) if m else None
+        text = f.read()
+    m = re.search(r"traffic_bytes_per_launch:\s*([0-9.eE+]+)", text)
+    k = re.search(r"`tlm::(k_step2?)<", text)
+    return float(m.group(1)) if m and k and (k.group(1) == "k_step2") == pairs else None
 
 
 # Every KERNEL_EVERY-th step launch of a timed region carries a start and an
@@ -124,11 +140,9 @@ def gpu_run(scene, warmup, steps, tag, plain=False, kernel_every=None):
         "wall_s": wall,
         "gcells": cells * steps / wall / 1e9,
         "ms_per_step": wall * 1e3 / steps,
-        "steps_per_launch": steps_per_launch(sc),
-        "kernel_ms_avg": ms_kernel * steps_per_launch(sc),  # ms_kernel: per step
-        "kernel_launches_timed": len({s // steps_per_launch(sc) for s in range(0, steps, kernel_every)}),
         "kernel_every": kernel_every,
     }
+    out.update(kernel_launches(dev, ms_kernel))
     if plain:
         t1 = time.perf_counter()
         dev.time_steps(warmup + steps, steps, kernel_every=0)
@@ -205,6 +219,7 @@ def batched_run(count=256, sample_every=4):
         probe_absmax = 0.0
         for d, sc in zip(devs, scs):
             b.remove(d)
+        launches = [d.step_launches()[0] for d in devs]
         for d, sc in zip(devs[:8], scs[:8]):
             probe_absmax = max(probe_absmax, float(np.abs(d.read_ports(0, sc.total_steps)).max()))
     for d in devs:
@@ -235,10 +250,9 @@ def batched_run(count=256, sample_every=4):
         "port_absmax": probe_absmax,
     }
     out["speedup_vs_one_at_a_time"] = round(out["gcell_s"] / out["one_at_a_time_gcell_s"], 3)
-    # the mix's algorithmic bytes per cell-update (a launch's over its steps); the rate above covers the
-    # whole run, the tail where few members are left included
-    bpc = (sum(sc.ncell * scene_alg_bytes(sc) / steps_per_launch(sc) for sc in scs)
-           / sum(sc.ncell for sc in scs))
+    # the algorithmic bytes of the launches the members took, per cell-update; the
+    # rate above covers the whole run, the tail where few members are left included
+    bpc = sum(sc.ncell * scene_alg_bytes(sc) * m for sc, m in zip(scs, launches)) / work
     out["alg_bytes_per_cell"] = round(bpc, 3)
     out["roofline_frac"] = round(out["gcell_s"] * bpc / HBM_PEAK_GBS, 4)
     path = os.path.join(ROOT, "profiles", f"k_step_batch_{count}.md")
@@ -292,7 +306,7 @@ def served_run(count=200, rate=50.0, baseline_sample=20, seed=5, max_cells=int(2
     from emsolver_amd import serve, tlm
     reqs = serve.served_stream(count=count, rate=rate, seed=seed, device_setup=device_setup)
     srv = serve.TlmServer(block_ticks=32, autotune_ticks=2, keep_results=False, progress_s=20.0,
-                          max_cells=max_cells, tuning={"graph_ticks": GRAPH_TICKS})
+                          max_cells=max_cells, tuning={"graph_ticks": GRAPH_TICKS}, count_launches=True)
     done = srv.serve(reqs)
     summ = serve.summarize(done)
     summ.update({"rate_per_s": rate, "mean_members": round(srv.stats["mean_members"], 2),
@@ -317,15 +331,17 @@ def served_run(count=200, rate=50.0, baseline_sample=20, seed=5, max_cells=int(2
     summ["one_at_a_time_fp32_gcell_s"] = round(alone_work / alone_wall / 1e9, 3)
     summ["one_at_a_time_sample"] = f"first {baseline_sample} requests, FP32, alone"
     summ["speedup_vs_one_at_a_time"] = round(summ["gcell_s"] / summ["one_at_a_time_fp32_gcell_s"], 3)
-    # the HBM roofline of this mix: every request's cell-updates at its own
-    # algorithmic bytes (FP16 requests: 16-bit slabs outside the FP32 band; FP32
-    # ones half a step's, two steps a launch) moved at 8 TB/s
+    # the HBM roofline of this mix: the launches that every request took at its
+    # own algorithmic bytes (FP16 requests: 16-bit slabs outside the FP32 band; a
+    # launch of two steps moves one's) moved at 8 TB/s
     work = byts = f16_work = 0.0
+    took = {c.rid: c for c in done}
     for r in reqs:
         sc = r.build()
+        sc.pulse = took[r.rid].pulse
         w = sc.ncell * sc.total_steps
         work += w
-        byts += w * scene_alg_bytes(sc) / steps_per_launch(sc)
+        byts += sc.ncell * scene_alg_bytes(sc) * took[r.rid].launches
         f16_work += w if sc.pulse != "f32" else 0.0
     ceil = work / (byts / (HBM_PEAK_GBS * 1e9)) / 1e9
     summ["hbm_ceiling_gcell_s"] = round(ceil, 3)
@@ -536,14 +552,15 @@ def free_space_64_run(with_cpu=True):
     # launch (they cost ~20 us of host time per launch at this size)
     with tlm.open_scene(sc) as dev:
         _, ker = dev.time_steps(0, sc.total_steps, kernel_every=1)
+        kl = kernel_launches(dev, ker)
     b = alg_bytes_per_cell(sc)
-    ker *= steps_per_launch(sc)
+    ker = kl["kernel_ms_avg"]
     out = {
         "grid": [64, 64, 64],
         "steps": sc.total_steps,
         "gcell_s": round(sc.ncell * sc.total_steps / wall / 1e9, 3),
         "kernel_us_avg": round(ker * 1e3, 2),
-        "steps_per_launch": steps_per_launch(sc),
+        "steps_per_launch": kl["steps_per_launch"],
         "achieved_gbs": round(sc.ncell * b / (ker * 1e-3) / 1e9, 1),
         "note": "state (25 MB) resident in the Infinity Cache: not an HBM roofline case; "
                 "gcell_s from 1000 steps with no launch events, kernel_us_avg from a second "
@@ -710,6 +727,7 @@ def main():
             "gcell_s": round(r["gcells"], 3),
             "kernel_ms_avg": round(r["kernel_ms_avg"], 4),
             "kernel_launches_timed": r["kernel_launches_timed"],
+            "kernel_pairs_timed": r["kernel_pairs_timed"],
             "steps_per_launch": r["steps_per_launch"],
             "achieved_gbs": round(r["achieved_gbs"], 1),
             "roofline_frac": round(r["achieved_gbs"] / HBM_PEAK_GBS, 4),
@@ -723,7 +741,7 @@ def main():
         r = gpu_run(sc, 10, args.extra_steps, "diel_boxes_256")
         extra["diel_boxes_256"] = roofline_line(r, sc)
         extra["diel_boxes_256"]["steps"] = args.extra_steps
-        extra["diel_boxes_256"]["traffic"] = read_traffic("diel_boxes_256")
+        extra["diel_boxes_256"]["traffic"] = read_traffic("diel_boxes_256", r["kernel_pairs_timed"] > 0)
         log(f"[bench] diel_boxes_256: {r['gcells']:.2f} Gcell/s, kernel {r['kernel_ms_avg']:.3f} ms, "
             f"{r['achieved_gbs']:.0f} GB/s = {r['achieved_gbs'] / HBM_PEAK_GBS:.3f} of peak")
     if not args.no_extra:
@@ -736,7 +754,7 @@ def main():
             extra[f"diel_boxes_512_{pulse}"].update({
                 "fp32_slab_fraction": round(fp32_slab_fraction(sc16), 4),
                 "steps": args.extra_steps,
-                "traffic": read_traffic(f"diel_boxes_512_{pulse}")})
+                "traffic": read_traffic(f"diel_boxes_512_{pulse}", r["kernel_pairs_timed"] > 0)})
             log(f"[bench] diel_boxes_512_{pulse}: {r['gcells']:.2f} Gcell/s, kernel "
                 f"{r['kernel_ms_avg']:.3f} ms, {r['achieved_gbs']:.0f} GB/s = "
                 f"{r['achieved_gbs'] / HBM_PEAK_GBS:.3f} of peak")
@@ -799,10 +817,12 @@ def main():
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(ach / HBM_PEAK_GBS, 4),
-            "traffic": read_traffic(workload),
-            "kernel": "tlm::k_step2 (fused scatter+connect, two steps a launch)",
+            # of a launch of two steps, where there are any
+            "traffic": read_traffic(workload, main_run["kernel_pairs_timed"] > 0),
+            "kernel": kernel_name(main_run["kernel_launches_timed"], main_run["kernel_pairs_timed"]),
             "kernel_ms_avg": round(main_run["kernel_ms_avg"], 5),
             "kernel_launches_timed": main_run["kernel_launches_timed"],
+            "kernel_pairs_timed": main_run["kernel_pairs_timed"],
             "steps_per_launch": main_run["steps_per_launch"],
             "alg_bytes_per_launch": int(round(scene.ncell * main_run["alg_bytes_per_cell"])),
         },

@@ -76,6 +76,7 @@ SIGNATURES = {
     "tlm_time_steps": (C.c_int, [P, C.c_int, C.c_int, C.c_int, fp, fp, C.POINTER(C.c_int)]),
     "tlm_launch_shape": (C.c_int, [P, C.POINTER(C.c_int), C.POINTER(C.c_int),
                                    C.POINTER(C.c_int), C.POINTER(C.c_int)]),
+    "tlm_timed_launches": (C.c_int, [P, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "tlm_step_launches": (C.c_int, [P, i64p, i64p]),
     "tlm_set_tuning": (C.c_int, [P, C.POINTER(Tuning)]),
     "tlm_get_tuning": (C.c_int, [P, C.POINTER(Tuning)]),

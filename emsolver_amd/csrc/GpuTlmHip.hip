@@ -503,9 +503,9 @@ tlm::PulseView pulse_view(const tlm_ctx *c, int n)
 }
 
 
-// kernel_every > 0: the step launches i = 0, k, 2k, ... of the block carry
-// timing events; their summed duration goes to *ms_kernel, their count to
-// *nkernel.
+// kernel_every > 0: the step launches of the steps i = 0, k, 2k, ... of the
+// block carry timing events; their summed duration goes to *ms_kernel, the
+// number of steps they took to *nkernel.
 int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_kernel, int *nkernel)
 {
     if (c->batch)
@@ -718,6 +718,8 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
         *ms_kernel = kern_ms;
         if (nkernel)
             *nkernel = timed_steps;
+        c->timed_launches = nev;
+        c->timed_pairs = timed_steps - nev;
     }
     HIPCHK(c, hipGetLastError());
     return TLM_OK;
@@ -1677,6 +1679,7 @@ int tlm_time_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *m
         *ms_kernel = 0.f;
     if (nkernel)
         *nkernel = 0;
+    c->timed_launches = c->timed_pairs = 0;
     HIPCHK(c, hipSetDevice(c->dev));
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     int rc = queue_steps(c, step0, nsteps, ms_kernel ? kernel_every : 0, ms_kernel, nkernel);
@@ -1688,6 +1691,17 @@ int tlm_time_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *m
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     if (ms_total)
         *ms_total = ms;
+    return TLM_OK;
+}
+
+int tlm_timed_launches(const tlm_ctx *c, int *launches, int *pairs)
+{
+    if (!c)
+        return TLM_ERR_ARG;
+    if (launches)
+        *launches = c->timed_launches;
+    if (pairs)
+        *pairs = c->timed_pairs;
     return TLM_OK;
 }
 

@@ -66,6 +66,7 @@ struct tlm_ctx
     bool pair_refused = false; // ... without room for the second stub buffer
     float *Vs2 = nullptr;    // the stubs a pair of steps writes (allocated at the first one)
     long long launches = 0, pairs = 0; // step launches since the last upload, those of two steps
+    int timed_launches = 0, timed_pairs = 0; // of the last tlm_time_steps
     // state
     int pf = TLM_PULSE_F32; // pulse storage format
     int halo = 8;           // 16-bit formats: FP32 slabs on each side of a source slab

@@ -42,6 +42,7 @@ class Completion:
     cells: int
     steps: int
     pulse: str
+    launches: int = 0      # of the fused step (one or two steps each), where counted
     probes: np.ndarray | None = None
     ports: np.ndarray | None = None
 
@@ -93,7 +94,7 @@ class TlmServer:
 
     def __init__(self, device=0, block_ticks=32, hbm_reserve=4 << 30, max_members=1024,
                  tuning=None, autotune_ticks=0, keep_results=True, progress_s=0.0,
-                 max_cells=0, retune_s=60.0):
+                 max_cells=0, retune_s=60.0, count_launches=False):
         self.device = device
         self.block_ticks = int(block_ticks)
         self.hbm_reserve = int(hbm_reserve)
@@ -105,6 +106,7 @@ class TlmServer:
         # and again every retune_s seconds, as the mix of members changes
         self.retune_s = float(retune_s)
         self.keep_results = keep_results
+        self.count_launches = count_launches  # Completion.launches
         self.progress_s = float(progress_s)  # > 0: a progress line on stderr this often
         # > 0: admit while the cells in flight stay below this (first come,
         # first served; enough cells to keep HBM streaming, few enough that a
@@ -201,6 +203,8 @@ class TlmServer:
             """Read the records of the members that left and free them."""
             for dev, r, sc, adm in finished:
                 c = Completion(r.rid, r.arrival, adm, 0.0, sc.ncell, sc.total_steps, sc.pulse)
+                if self.count_launches:
+                    c.launches = dev.step_launches()[0]
                 if self.keep_results:
                     if dev.nprobe:
                         c.probes = dev.read_probes(0, sc.total_steps)

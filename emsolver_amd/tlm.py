@@ -376,8 +376,9 @@ class TlmDevice:
 
     def time_steps(self, step0, nsteps, kernel_every=1):
         """Run and time steps [step0, step0+nsteps): (ms of the whole block,
-        average ms of one fused step launch over the launches of every
-        kernel_every-th step, or None with kernel_every=0)."""
+        average ms of a step in the launches of every kernel_every-th step, or
+        None with kernel_every=0). A launch takes one or two steps:
+        timed_launches tells how many of each were timed."""
         tot = C.c_float(0)
         ker = C.c_float(0)
         nk = C.c_int(0)
@@ -386,6 +387,13 @@ class TlmDevice:
                                           C.byref(ker) if k > 0 else None, C.byref(nk)),
                   "tlm_time_steps")
         return tot.value, (ker.value / nk.value if k > 0 and nk.value > 0 else None)
+
+    def timed_launches(self):
+        """(launches, pairs): the launches that the last time_steps timed, and
+        how many of them took two steps."""
+        n, p = C.c_int(0), C.c_int(0)
+        self._chk(self.lib.tlm_timed_launches(self.h, C.byref(n), C.byref(p)), "tlm_timed_launches")
+        return n.value, p.value
 
     def set_tuning(self, **changes):
         """Sets the tlm_tuning fields named (kernel, planes, block_waves,

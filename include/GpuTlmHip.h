@@ -200,11 +200,16 @@ int tlm_read_frames(tlm_ctx *ctx, int32_t *steps, float *js, float *planes, int 
  * kernel_every = k > 0 (and ms_kernel not NULL) the fused scatter/connect
  * launches of the steps step0, step0+k, step0+2k, ... carry their own start
  * and end events: *ms_kernel is their summed duration and *nkernel (may be
- * NULL) the number of steps they took (a launch may take two). Events on a launch cost host time (~4 us per launch at
- * 256^3, ~20 us at 64^3), so a sample (k > 1) perturbs the run less than
+ * NULL) the number of steps they took (a launch may take two, and is timed if
+ * one of them is sampled). Events on a launch cost host time (~4 us per launch
+ * at 256^3, ~20 us at 64^3), so a sample (k > 1) perturbs the run less than
  * k = 1; k = 0 measures no launch. */
 int tlm_time_steps(tlm_ctx *ctx, int step0, int nsteps, int kernel_every, float *ms_total,
                    float *ms_kernel, int *nkernel);
+
+/* The launches that the last tlm_time_steps timed, and how many of them took
+ * two steps. Either may be NULL. */
+int tlm_timed_launches(const tlm_ctx *ctx, int *launches, int *pairs);
 
 /* Device-copy bandwidth: copies `bytes` between two device buffers `iters`
  * times with a plain grid-stride float4 kernel (k_copy) and reports

@@ -155,3 +155,19 @@ def test_autotune_times_pairs_as_pairs(short):
             b.remove(d)
     for d in devs:
         d.close()
+
+
+def test_timed_launches():
+    """20 steps from step 5 with an energy record every 16: 15 cannot start a
+    pair and 24 has no partner."""
+    sc = _scene(64, 20, 12, steps=40)
+    sc.energy_every = 16
+    with tlm.open_scene(sc) as dev:
+        dev.run(0, 5)
+        total, per = dev.time_steps(5, 20, kernel_every=1)
+        assert dev.timed_launches() == (11, 9)
+        assert 0 < 20 * per <= 1.05 * total
+        dev.time_steps(25, 10, kernel_every=7)  # steps 25 (a pair with 26) and 32 (a pair with 33)
+        assert dev.timed_launches() == (2, 2)
+        dev.time_steps(35, 4, kernel_every=0)
+        assert dev.timed_launches() == (0, 0)
