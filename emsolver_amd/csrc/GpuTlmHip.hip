@@ -89,9 +89,13 @@ void choose_shape(tlm_ctx *c)
     }
 }
 
+// Energy partials that one workgroup adds up in a launch; more are added in two.
+constexpr long long kEnergyOneStage = 32768;
+
+// One energy partial per 64-cell block, whatever the launch (block_energy).
 size_t energy_parts(const tlm_ctx *c)
 {
-    return (size_t)c->blocks * c->wpb;
+    return (size_t)c->P / tlm::kWave;
 }
 
 // ---- two steps a launch (k_step2) ----
@@ -148,10 +152,6 @@ void choose_pair(tlm_ctx *c)
     const int m = (p.groups + 8 * p.ntile - 1) / (8 * p.ntile);
     p.chunk = (p.groups + 8 * m - 1) / (8 * m);
     p.blocks = 8 * tlm::xcd_chunk_map(p.groups, p.chunk).cpx;
-}
-size_t pair_energy_parts(const tlm_ctx *c)
-{
-    return c->pair.ok ? (size_t)c->pair.blocks * (c->pair.nt / tlm::kWave) : 0;
 }
 
 // The fused step launch; nmon > 0 appends the workgroups that take the
@@ -675,19 +675,19 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
         if (c->every > 0 && (n % c->every) == 0)
         {
             const int idx = n / c->every;
-            const long long np = (long long)(per == 2 ? pair_energy_parts(c) : energy_parts(c));
-            if (np > 8192)
+            const long long np = (long long)energy_parts(c);
+            if (np > kEnergyOneStage)
             {
                 // two stages: 1024 fixed chunks, then one block
                 const long long chunk = (np + 1023) / 1024;
                 const int nb = (int)((np + chunk - 1) / chunk);
-                hipLaunchKernelGGL(tlm::k_energy_chunks, dim3(nb), dim3(256), 0, c->stream,
+                hipLaunchKernelGGL(tlm::k_energy_chunks, dim3(nb), dim3(tlm::kEnergyChunk), 0, c->stream,
                                    c->epart, np, chunk, c->epart2);
-                hipLaunchKernelGGL(tlm::k_energy_reduce, dim3(1), dim3(256), 0, c->stream,
+                hipLaunchKernelGGL(tlm::k_energy_reduce, dim3(1), dim3(tlm::kEnergyReduce), 0, c->stream,
                                    c->epart2, nb, c->energy + idx);
             }
             else
-                hipLaunchKernelGGL(tlm::k_energy_reduce, dim3(1), dim3(256), 0, c->stream,
+                hipLaunchKernelGGL(tlm::k_energy_reduce, dim3(1), dim3(tlm::kEnergyReduce), 0, c->stream,
                                    c->epart, (int)np, c->energy + idx);
             if ((int)c->energy_steps.size() <= idx)
                 c->energy_steps.resize(idx + 1, -1);
@@ -1065,11 +1065,10 @@ int tlm_create(const tlm_grid_desc *d, tlm_ctx **out)
             return bail(hip_fail(c, e, "hipEventCreate"));
     int rc;
     choose_pair(c);
-    c->epart_cap = std::max(energy_parts(c), pair_energy_parts(c));
     if (c->pf == TLM_PULSE_F32 &&
         ((rc = dalloc(c, &c->A, (size_t)c->PB * 12)) || (rc = dalloc(c, &c->B, (size_t)c->PB * 12))))
         return bail(rc);
-    if ((rc = dalloc(c, &c->code, (size_t)c->P)) || (rc = dalloc(c, &c->epart, c->epart_cap)) ||
+    if ((rc = dalloc(c, &c->code, (size_t)c->P)) || (rc = dalloc(c, &c->epart, energy_parts(c))) ||
         (rc = dalloc(c, &c->epart2, 1024)))
         return bail(rc);
     *out = c;
@@ -1743,15 +1742,6 @@ int tlm_set_tuning(tlm_ctx *c, const tlm_tuning *t)
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->tune = *t;
     choose_shape(c);
-    const size_t need = energy_parts(c);
-    if (need > c->epart_cap)
-    {
-        dfree(c, c->epart);
-        int rc = dalloc(c, &c->epart, need);
-        if (rc)
-            return rc;
-        c->epart_cap = need;
-    }
     return TLM_OK;
 }
 

@@ -194,7 +194,6 @@ __global__ void __launch_bounds__(256) k_step_batch(const BatchMember *mem, cons
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const BatchClock t = now();
     const XcdRange gr = xcd_range(blockIdx.x, mon_from, ngroups);
-    double esum = 0.0;
     for (int g = gr.first; g < gr.end; g += gr.step)
     {
         const int mi = gmem[g];
@@ -217,9 +216,9 @@ __global__ void __launch_bounds__(256) k_step_batch(const BatchMember *mem, cons
             a.esc = m.iscl[cur ^ 1];
         }
         if constexpr (PF == PF_F32)
-            strip_task<STUBS, false, false, PF>(a, task, lane, esum);
+            strip_task<STUBS, false, false, PF>(a, task, lane);
         else
-            strip_task16<STUBS, false, PF>(a, task, lane, esum);
+            strip_task16<STUBS, false, PF>(a, task, lane);
     }
 }
 

@@ -53,7 +53,6 @@ struct tlm_ctx
     tlm_tuning tune = {0, 1, 4, 0, 0, 2, -1}; // folding and occupancy chosen per grid
     int strips = 0, zc = 0, nzc = 0, tasks = 0, groups = 0, blocks = 0, wpb = 4;
     int xchunk = 0; // > 0: groups per chunk of the XCD-interleaved map (choose_shape)
-    size_t epart_cap = 0;
     // two steps a launch (k_step2): tiles of tb blocks with hb blocks of rim on
     // either side (ntile of them in a slab), marched over zc slabs by nt threads,
     // a wave holding `cells` blocks; ok: the grid may run pairs
@@ -79,7 +78,7 @@ struct tlm_ctx
     float4 *props = nullptr;
     int nmat = 0;
     bool stubs = false, uploaded = false;
-    double *epart = nullptr, *epart2 = nullptr; // energy partials (per wave, per chunk)
+    double *epart = nullptr, *epart2 = nullptr; // energy partials (per 64-cell block, per chunk)
     // sources
     long long *ucell = nullptr;
     int *ubeg = nullptr, *spol = nullptr;

@@ -186,7 +186,7 @@ struct StepArgs
                           // PEC neighbour bit; padded to a multiple of 4 bytes
                           // (block_flag)
     const float4 *props;  // per dielectric id: (yh, gh, den, 0)
-    double *epart;        // energy partial per wave task
+    double *epart;        // energy partial per 64-cell block
     // 16-bit formats only
     const uint2 *slab;    // per slab: (byte offset inside a plane, 1 if 16-bit storage)
     const float *dsc;     // per slab: 2^E_n (decode A)
@@ -381,6 +381,30 @@ __device__ __forceinline__ double cell_energy(const float v[12])
         e[p & 3] = fma((double)v[p], (double)v[p], e[p & 3]);
     return (e[0] + e[1]) + (e[2] + e[3]);
 }
+// e of the lane that DPP control `ctrl` names, 0 where it names none or the row
+// is not in `rows`.
+template <int ctrl, int rows> __device__ __forceinline__ double dpp(double e)
+{
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(e), ctrl, rows, 0xf, false),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(e), ctrl, rows, 0xf, false));
+}
+// Sum over a wave's 64 cells (one block) of e, in an order of its own whatever
+// launch the block is part of: with the partials added by block, a step's energy
+// is the same bits for every launch shape, and as the first of two steps or alone.
+// Shifts and broadcasts of rows of 16 lanes leave the sum in lane 63. An energy
+// launch of k_step2 at 512^3: 2.75 ms with one sum a wave at the end of its march,
+// 2.80 so, 2.83 by shuffles through LDS; at 256^3 343 and 353 us.
+__device__ __forceinline__ void block_energy(double e, int lane, double *out)
+{
+    e += dpp<0x111, 0xf>(e); // row_shr 1, 2, 4, 8
+    e += dpp<0x112, 0xf>(e);
+    e += dpp<0x114, 0xf>(e);
+    e += dpp<0x118, 0xf>(e);
+    e += dpp<0x142, 0xa>(e); // row_bcast 15: rows 0 and 2 into 1 and 3
+    e += dpp<0x143, 0xc>(e); // row_bcast 31: into rows 2 and 3
+    if (lane == kWave - 1)
+        *out = e;
+}
 
 // Fused scatter + connect. A wavefront owns a strip of 64 consecutive cells
 // of one z-slab (lane = cell) and marches over zc slabs.
@@ -399,7 +423,7 @@ __device__ __forceinline__ double cell_energy(const float v[12])
 // neighbour PEC (-out). This is connect(), TlmSolver.cpp:563-583.
 // One wave task: a 64-cell strip of slabs [k0, k1).
 template <bool STUBS, bool ENERGY, bool NT, int PF, bool FOLD = false>
-__device__ __forceinline__ void strip_task(const StepArgs &a, int task, int lane, double &esum)
+__device__ __forceinline__ void strip_task(const StepArgs &a, int task, int lane)
 {
     static_assert(PF == PF_F32, "the 16-bit formats use strip_task16");
     const int tz = (int)mdiv((unsigned)task, a.mstrips), t = task - tz * a.strips;
@@ -467,6 +491,7 @@ __device__ __forceinline__ void strip_task(const StepArgs &a, int task, int lane
             }
         }
         const unsigned m = code & 0xFFu;
+        double en = 0.0;
         float yhv = 0.f, denv = 4.f;
         if (vtab)
         {
@@ -480,7 +505,7 @@ __device__ __forceinline__ void strip_task(const StepArgs &a, int task, int lane
                 fold_sources(a.fold, (long long)mo, v);
             pec = (m == 1u);
             if (ENERGY)
-                esum += cell_energy(v);
+                en = cell_energy(v);
             if (STUBS && m >= 2u)
             {
                 if (!vtab)
@@ -517,6 +542,8 @@ __device__ __forceinline__ void strip_task(const StepArgs &a, int task, int lane
                 o[p] = 0.f;
         }
         // every lane takes part in the shuffles
+        if (ENERGY)
+            block_energy(en, lane, a.epart + (size_t)k * a.strips + t);
         const float L0 = __shfl_up(o[2], 1, kWave), L1 = __shfl_up(o[3], 1, kWave);
         const float R0 = __shfl_down(o[0], 1, kWave), R1 = __shfl_down(o[1], 1, kWave);
         if (act)
@@ -713,7 +740,7 @@ __device__ __forceinline__ void stpair_at(char *buf, const Slab16 &s, int q, flo
 // delivery rules, same FP32 arithmetic, values rounded where stored). Every
 // per-lane choice of value or slot is a select, not a branch.
 template <bool STUBS, bool ENERGY, int PF>
-__device__ __forceinline__ void strip_task16(const StepArgs &a, int task, int lane, double &esum)
+__device__ __forceinline__ void strip_task16(const StepArgs &a, int task, int lane)
 {
     const int tz = (int)mdiv((unsigned)task, a.mstrips), t = task - tz * a.strips;
     const int f = t * kWave + lane;
@@ -787,6 +814,7 @@ __device__ __forceinline__ void strip_task16(const StepArgs &a, int task, int la
             const unsigned cf = or_opaque(code, lf);
             const unsigned m = cf & 0xFFu;
             const bool pec = !CL && (!act || m == 1u);
+            double en = 0.0;
             float yhv = 0.f, denv = 4.f;
             if (vtab && dblk)
             {
@@ -797,7 +825,7 @@ __device__ __forceinline__ void strip_task16(const StepArgs &a, int task, int la
             if (live)
             {
                 if (ENERGY)
-                    esum += cell_energy(v);
+                    en = cell_energy(v);
                 if (STUBS && m >= 2u)
                 {
                     if (!vtab)
@@ -827,6 +855,8 @@ __device__ __forceinline__ void strip_task16(const StepArgs &a, int task, int la
                 for (int p = 0; p < 12; ++p)
                     v[p] = 0.f;
             }
+            if (ENERGY)
+                block_energy(en, lane, a.epart + (size_t)k * a.strips + t);
             // a PEC cell keeps its incident pulses: o carries them (an idle
             // lane counts as PEC and sends zeros)
 #pragma unroll
@@ -1499,65 +1529,56 @@ __global__ void __launch_bounds__(256) k_step(StepArgs a, MonitorArgs m, int mon
     const int wpb = blockDim.x / kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const XcdRange gr = xcd_range_map(blockIdx.x, a.xm);
-    double esum = 0.0;
     for (int g = gr.first; g < gr.end; g += gr.step)
     {
         const int task = g * wpb + wave;
         if (task < a.tasks)
         {
             if constexpr (PF == PF_F32)
-                strip_task<STUBS, ENERGY, NT, PF, FOLD>(a, task, lane, esum);
+                strip_task<STUBS, ENERGY, NT, PF, FOLD>(a, task, lane);
             else
-                strip_task16<STUBS, ENERGY, PF>(a, task, lane, esum);
+                strip_task16<STUBS, ENERGY, PF>(a, task, lane);
         }
     }
-    if (ENERGY)
-    {
-        for (int off = kWave / 2; off > 0; off >>= 1)
-            esum += __shfl_down(esum, off, kWave);
-        if (lane == 0)
-            a.epart[blockIdx.x * wpb + wave] = esum;
-    }
 }
 
-// First stage of the energy sum: block b adds partials [b*chunk, (b+1)*chunk)
-// in a fixed order (so the result does not depend on scheduling).
+// Sum of part[lo, hi) by a workgroup of N threads, in a fixed order: eight
+// loads of a thread in flight together.
+template <int N> __device__ __forceinline__ double group_sum(const double *part, long long lo, long long hi)
+{
+    __shared__ double s[N];
+    double acc[8] = {};
+    for (long long i = lo + threadIdx.x; i < hi; i += 8 * N)
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            acc[q] += i + q * N < hi ? part[i + q * N] : 0.0;
+    s[threadIdx.x] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+    __syncthreads();
+    for (int w = N / 2; w > 0; w >>= 1)
+    {
+        if ((int)threadIdx.x < w)
+            s[threadIdx.x] += s[threadIdx.x + w];
+        __syncthreads();
+    }
+    return s[0];
+}
+
+// First stage of the energy sum: block b adds partials [b*chunk, (b+1)*chunk).
+constexpr int kEnergyChunk = 256, kEnergyReduce = 1024; // threads
 static __global__ void k_energy_chunks(const double *part, long long nparts, long long chunk, double *out)
 {
-    __shared__ double s[256];
-    const long long lo = blockIdx.x * chunk, hi = min(nparts, lo + chunk);
-    double acc = 0.0;
-    for (long long i = lo + threadIdx.x; i < hi; i += blockDim.x)
-        acc += part[i];
-    s[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1)
-    {
-        if ((int)threadIdx.x < w)
-            s[threadIdx.x] += s[threadIdx.x + w];
-        __syncthreads();
-    }
+    const long long lo = blockIdx.x * chunk;
+    const double e = group_sum<kEnergyChunk>(part, lo, min(nparts, lo + chunk));
     if (threadIdx.x == 0)
-        out[blockIdx.x] = s[0];
+        out[blockIdx.x] = e;
 }
 
-// Sum of the energy partials of one step in a fixed order.
+// Sum of the energy partials of one step.
 static __global__ void k_energy_reduce(const double *part, int nparts, double *out)
 {
-    __shared__ double s[256];
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < nparts; i += blockDim.x)
-        acc += part[i];
-    s[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1)
-    {
-        if ((int)threadIdx.x < w)
-            s[threadIdx.x] += s[threadIdx.x + w];
-        __syncthreads();
-    }
+    const double e = group_sum<kEnergyReduce>(part, 0, nparts);
     if (threadIdx.x == 0)
-        *out = s[0];
+        *out = e;
 }
 
 // Running FP64 DFT of the probe records over steps [n0, n1), in step order.

@@ -48,7 +48,7 @@ struct PairArgs
     const uint16_t *code;
     const uint8_t *uair;  // block flags (StepArgs::uair)
     const float4 *props;
-    double *epart;        // energy partials of step n, one per wave
+    double *epart;        // energy partials of step n, one per 64-cell block
     int nx, ny, nz;
     long long Pp;         // slab pitch (cells)
     float rho;
@@ -340,7 +340,6 @@ __device__ __forceinline__ void pair_tile(const PairArgs &a, int tz, int tt, int
         for (int p = 0; p < 3; ++p)
             s[c][p] = 0.f;
     }
-    double esum = 0.0;
     // The loads of a slab are issued one slab ahead, right after the registers'
     // last use; none is skipped (lanes with nothing to load repeat a cell of
     // the rim), so that the number of loads and stores in flight behind them
@@ -378,8 +377,9 @@ __device__ __forceinline__ void pair_tile(const PairArgs &a, int tz, int tt, int
         if (code[c] & kCodeSource)
             fold_sources(a.fold, (long long)kk * a.Pp + f[c], v[c]);
         const bool in = kk >= k0 && kk < k1;
-        if (ENERGY && in && (tf[c] & TF_ACT) && c * ni + wave < b1 - b0)
-            esum += cell_energy(v[c]);
+        if (ENERGY && in && !rim) // a place past the last block stores that block's sum again
+            block_energy((tf[c] & TF_ACT) ? cell_energy(v[c]) : 0.0, lane,
+                         a.epart + (size_t)kk * a.strips + (b0 - a.hb + bi[c]));
         pair_scatter<STUBS>(v[c], code[c], sn, tab, o);
         if (in)
         {
@@ -412,8 +412,6 @@ __device__ __forceinline__ void pair_tile(const PairArgs &a, int tz, int tt, int
             }
             pair_barrier();
         }
-        if (ENERGY && lane == 0)
-            a.epart[blockIdx.x * nw + wave] = 0.0;
         return;
     }
 
@@ -581,13 +579,6 @@ __device__ __forceinline__ void pair_tile(const PairArgs &a, int tz, int tt, int
         }
         pair_barrier();
     }
-    if (ENERGY)
-    {
-        for (int o = kWave / 2; o > 0; o >>= 1)
-            esum += __shfl_down(esum, o, kWave);
-        if (lane == 0)
-            a.epart[blockIdx.x * nw + wave] = esum;
-    }
 }
 
 template <bool STUBS, bool ENERGY, int C, int NT>
@@ -607,11 +598,7 @@ __global__ void __launch_bounds__(NT, kPairOcc) k_step2(PairArgs a, MonitorArgs 
     }
     const XcdRange gr = xcd_range_map(blockIdx.x, a.xm);
     if (gr.first >= gr.end)
-    {
-        if (ENERGY && (threadIdx.x & (kWave - 1)) == 0)
-            a.epart[blockIdx.x * nw + threadIdx.x / kWave] = 0.0;
         return;
-    }
     const int tz = gr.first / a.ntile;
     pair_tile<STUBS, ENERGY, C, NT>(a, tz, gr.first - tz * a.ntile, nw, lds);
 }
