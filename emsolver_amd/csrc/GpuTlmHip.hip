@@ -774,7 +774,9 @@ void host_clear(float *p, size_t count)
 // its own: order on the device, copy out, write to host_out, so that one
 // thread's copy runs beside the others' writes. 157^3 cells with stubs, 232 MB
 // into fresh memory: 26 ms from pageable copies in one thread, 8.1 here; 64^3, 16 MB: 1.02 and
-// 0.87.
+// 0.87. A state of one chunk goes straight to host_out: making and giving back
+// pinned memory takes longer than its copy (24^3, 0.8 MB: 88 us, 152 through
+// pinned memory; 32^3, 2 MB: 154 and 214).
 int read_back(tlm_ctx *c, float *host_out, const tlm::PulseView *pv, float *soa, int ncomp)
 {
     const long long ncell = (long long)c->nx * c->ny * c->nz;
@@ -785,7 +787,7 @@ int read_back(tlm_ctx *c, float *host_out, const tlm::PulseView *pv, float *soa,
     int rc = dalloc(c, &stage, slot * n);
     if (rc)
         return rc;
-    if (hipHostMalloc((void **)&pin, slot * n * sizeof(float), hipHostMallocDefault) != hipSuccess)
+    if (nchunk > 1 && hipHostMalloc((void **)&pin, slot * n * sizeof(float), hipHostMallocDefault) != hipSuccess)
     {
         (void)hipGetLastError(); // without pinned memory straight to host_out
         pin = nullptr;

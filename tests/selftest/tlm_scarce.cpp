@@ -10,7 +10,8 @@
 //     single steps, without an error left behind, and pairs again after an
 //     upload that finds room;
 //   * an upload without memory for the device map, refused or not;
-//   * a state read back without pinned memory or without threads;
+//   * a state read back without pinned memory or without threads, and a small
+//     one, which asks for neither;
 //   * face lists read without device memory for their order.
 // Prints PASS/FAIL lines and exits 1 on a failure; SKIP without a device.
 //---------------------------------------------------------------------------
@@ -213,6 +214,27 @@ void no_pinned_or_threads(const State &ref)
     tlm_destroy(c);
 }
 
+void small_state()
+{
+    tlm_grid_desc d = {};
+    d.nx = d.ny = d.nz = 32;
+    d.dl = 0.01f;
+    tlm_ctx *c = nullptr;
+    must(tlm_create(&d, &c), nullptr, "tlm_create");
+    const int n = 32 * 32 * 32;
+    const std::vector<uint8_t> mat((size_t)n, 2);
+    must(tlm_upload(c, mat.data(), kY, kG, 1, g_V.data(), g_Vs.data()), c, "tlm_upload");
+    State s;
+    const int pinned = g_pinned, threads = g_threads;
+    must(tlm_read_state(c, s.V.data(), s.Vs.data()), c, "tlm_read_state");
+    check(std::memcmp(s.V.data(), g_V.data(), 12 * n * sizeof(float)) == 0 &&
+              std::memcmp(s.Vs.data(), g_Vs.data(), 3 * n * sizeof(float)) == 0,
+          "a state of 2 MB read back");
+    check(g_pinned == pinned && g_threads == threads, "... without pinned memory or threads", g_pinned - pinned,
+          g_threads - threads);
+    tlm_destroy(c);
+}
+
 void no_list_memory()
 {
     tlm_ctx *c = make();
@@ -274,6 +296,7 @@ int main()
     no_second_stub_buffer(ref);
     no_map(ref);
     no_pinned_or_threads(ref);
+    small_state();
     no_list_memory();
     std::printf(g_fail ? "SCARCETEST FAILED\n" : "SCARCETEST PASSED\n");
     return g_fail ? 1 : 0;
