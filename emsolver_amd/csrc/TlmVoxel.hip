@@ -1578,9 +1578,14 @@ int64_t tlm_huygens_mat(tlm_ctx *c, int o)
     return n;
 }
 
-// Cells of a list in cellIndex order of the unpadded grid (on the host, through
-// an array of its own, 0.4 of the 3.9 ms in which a 256^3 mesh scene was set
-// up and its lists read).
+// Cells of a list in cellIndex order of the unpadded grid. Lists of more than
+// kListHost faces are ordered on the device (on the host, through an array of
+// its own, 0.4 of the 3.9 ms in which a 256^3 mesh scene was set up and its lists
+// read); few faces sooner on the host, without an allocation, a launch and a
+// wait: 32 faces 26 us (47 on the device), 2048 38 (55), 8192 67 (69). The copy
+// blocks after a wait for the stream: queued on it, it took 106 us for 36864
+// faces, 52 so.
+constexpr long long kListHost = 4096;
 static __global__ void k_list_cells(const long long *pc, long long n, long long Pp, long long nxy, long long *out)
 {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1601,22 +1606,23 @@ static int64_t read_list(tlm_ctx *c, const long long *dcell, const int *daxis, i
     {
         static_assert(sizeof(long long) == sizeof(int64_t), "one cell index");
         Scratch s;
-        long long *out;
-        if (s.get(c, &out, (size_t)m) == TLM_OK)
+        long long *out = nullptr;
+        if (m > kListHost && s.get(c, &out, (size_t)m) == TLM_OK)
         {
             k_list_cells<<<(unsigned)((m + kThreads - 1) / kThreads), kThreads, 0, c->stream>>>(dcell, m, c->Pp,
                                                                                                c->nxy, out);
             HIPCHK(c, hipGetLastError());
-            HIPCHK(c, hipMemcpyAsync(cells, out, (size_t)m * sizeof(long long), hipMemcpyDeviceToHost, c->stream));
             HIPCHK(c, hipStreamSynchronize(c->stream));
+            HIPCHK(c, hipMemcpy(cells, out, (size_t)m * sizeof(long long), hipMemcpyDeviceToHost));
         }
         else
         {
-            // no device memory: in the caller's own array
+            // few, or no device memory: in the caller's own array
             (void)hipGetLastError();
             HIPCHK(c, hipMemcpy(cells, dcell, (size_t)m * sizeof(long long), hipMemcpyDeviceToHost));
-            for (long long q = 0; q < m; ++q)
-                cells[q] = cells[q] / c->Pp * c->nxy + cells[q] % c->Pp;
+            const unsigned Pp = (unsigned)c->Pp, pad = (unsigned)(c->Pp - c->nxy);
+            for (long long q = 0; q < m; ++q) // padded cell indices are below 2^31
+                cells[q] -= (long long)((unsigned)cells[q] / Pp) * pad;
         }
     }
     if (m > 0 && axes)

@@ -12,11 +12,13 @@
 //   * an upload without memory for the device map, refused or not;
 //   * a state read back without pinned memory or without threads, and a small
 //     one, which asks for neither;
-//   * face lists read without device memory for their order.
+//   * face lists read without device memory for their order, and the first few
+//     faces of one, which ask for none.
 // Prints PASS/FAIL lines and exits 1 on a failure; SKIP without a device.
 //---------------------------------------------------------------------------
 #include "GpuTlmHip.h"
 
+#include <algorithm>
 #include <cerrno>
 #include <cstdio>
 #include <cstring>
@@ -251,6 +253,16 @@ void no_list_memory()
     must((int)tlm_read_faces(c, b.data(), bx.data(), n), c, "tlm_read_faces");
     g_refuse = kNone;
     check(n > 62000 && a == b && ax == bx, "a list read without device memory", n);
+    const int mallocs = g_mallocs;
+    for (int64_t few : {(int64_t)1, (int64_t)777, (int64_t)4096})
+    {
+        std::vector<int64_t> d((size_t)few);
+        std::vector<int32_t> dx((size_t)few);
+        must((int)tlm_read_faces(c, d.data(), dx.data(), few), c, "tlm_read_faces");
+        check(std::equal(d.begin(), d.end(), a.begin()) && std::equal(dx.begin(), dx.end(), ax.begin()),
+              "the first faces of a list", few);
+    }
+    check(g_mallocs == mallocs, "... without an allocation", g_mallocs - mallocs);
     tlm_destroy(c);
 }
 
