@@ -1544,6 +1544,7 @@ int tlm_set_huygens(tlm_ctx *c, const int64_t *cells, const int32_t *axes, int n
     }
     int rc;
     c->hlat = HuyLattice{};
+    c->hlat_known = false;
     if ((rc = upload(c, &c->hcell, hc.data(), hc.size())) ||
         (rc = upload(c, &c->haxis, ha.data(), ha.size())))
         return rc;
@@ -1552,7 +1553,7 @@ int tlm_set_huygens(tlm_ctx *c, const int64_t *cells, const int32_t *axes, int n
         return rc;
     HIPCHK(c, hipMemset(c->huy8, 0, 8 * (size_t)std::max(1, n) * sizeof(float)));
     c->nh = n;
-    return huy_lattice_scan(c);
+    return TLM_OK;
 }
 
 int tlm_run(tlm_ctx *c, int step0, int nsteps)

@@ -636,6 +636,9 @@ struct Carve
     }
 };
 
+// Workspace of the allocation-free variant.
+constexpr size_t kScratchBytes = (size_t)128 << 20;
+
 // A context keeps its workspace for the next call up to this size (an
 // allocation and its release take longer than the other host work of a call).
 constexpr size_t kKeep = (size_t)64 << 20;
@@ -883,13 +886,81 @@ int lattice_transform(tlm_ctx *c, unsigned char *w, const LatticeShape &S, Outpu
 // 13824 102 against 92, 31104 120 against 140.
 constexpr double kLatticeTerms = 5e7;
 
+// Finds whether the context's faces are the places of a few planes of a box
+// (each once, and most of them there) and records its extent: at the first
+// transform of a list that may use it, in the transform's workspace w of
+// scan_bytes (at tlm_set_huygens it took 40 us, 64^3, of callers who take no far
+// field).
+size_t scan_marks(const tlm_ctx *c)
+{
+    return Carve::piece(2 * (size_t)(c->nx + (long long)c->ny + c->nz));
+}
+size_t scan_bytes(const tlm_ctx *c)
+{
+    return scan_marks(c) + Carve::piece(((size_t)c->nh * 3 / 2 + 1) * sizeof(int)); // huy_lattice_fits
+}
+int huy_lattice_scan(tlm_ctx *c, unsigned char *w)
+{
+    c->hlat = HuyLattice{};
+    c->hlat_known = true;
+    const int n = c->nh;
+    const size_t len = (size_t)c->nx + c->ny + c->nz;
+    hipStream_t st = c->stream;
+    HuyLattice h;
+    FFCHK(hipMemsetAsync(w, 0, 2 * len, st));
+    k_huy_used<<<(n + 255) / 256, 256, 0, st>>>(n, c->hcell, c->haxis, c->nx, c->ny, c->Pp, w, w + len);
+    FFCHK(hipGetLastError());
+    std::vector<uint8_t> m(2 * len);
+    FFCHK(hipMemcpyAsync(m.data(), w, m.size(), hipMemcpyDeviceToHost, st));
+    FFCHK(hipStreamSynchronize(st));
+    const int dims[3] = {c->nx, c->ny, c->nz};
+    size_t at = 0;
+    for (int q = 0; q < 3; at += dims[q], ++q)
+    {
+        int lo = 0, hi = dims[q] - 1;
+        while (lo < hi && !m[at + lo])
+            ++lo;
+        while (hi > lo && !m[at + hi])
+            --hi;
+        h.lo[q] = lo;
+        h.n[q] = hi - lo + 1;
+        for (int i = lo; i <= hi; ++i)
+            if (m[len + at + i])
+            {
+                if (h.nplane == kHuyPlanes)
+                    return TLM_OK;
+                h.axis[h.nplane] = q;
+                h.coord[h.nplane++] = i;
+            }
+    }
+    if (!huy_lattice_fits(h, n))
+        return TLM_OK;
+    const FfLattice L(h);
+    const size_t places = (size_t)L.off[L.nplane] / 4;
+    int *cnt = reinterpret_cast<int *>(w + scan_marks(c)), twice = 0;
+    FFCHK(hipMemsetAsync(cnt, 0, (places + 1) * sizeof(int), st));
+    k_huy_twice<<<(n + 255) / 256, 256, 0, st>>>(n, c->hcell, c->haxis, c->nx, c->Pp, L, cnt, cnt + places);
+    FFCHK(hipGetLastError());
+    FFCHK(hipMemcpyAsync(&twice, cnt + places, sizeof(int), hipMemcpyDeviceToHost, st));
+    FFCHK(hipStreamSynchronize(st));
+    h.ok = !twice;
+    c->hlat = h;
+    return TLM_OK;
+}
+
 // Both entry points of a context: ws(bytes, &p) gives the workspace.
 template <class Ws> int ctx_transform(tlm_ctx *c, const float origin[3], Output &o, Ws ws)
 {
     unsigned char *w = nullptr;
     int rc;
-    if (c->hlat.ok && (double)c->nh * o.dirs(nullptr).n() >= kLatticeTerms && std::isfinite(origin[0]) &&
-        std::isfinite(origin[1]) && std::isfinite(origin[2]))
+    const bool many = c->nh >= kHuyLatticeMin && (double)c->nh * o.dirs(nullptr).n() >= kLatticeTerms &&
+                      std::isfinite(origin[0]) && std::isfinite(origin[1]) && std::isfinite(origin[2]);
+    if (many && !c->hlat_known && scan_bytes(c) <= kScratchBytes)
+    {
+        if ((rc = ws(scan_bytes(c), &w)) || (rc = huy_lattice_scan(c, w)))
+            return rc;
+    }
+    if (many && c->hlat.ok)
     {
         const LatticeShape S(c->hlat, o.dirs(nullptr));
         bool odd = false;
@@ -917,7 +988,6 @@ template <class Ws> int ctx_transform(tlm_ctx *c, const float origin[3], Output 
 // Its workspace: a file-scope device array of kScratchBytes, one instance per
 // GPU the library runs on (held until the process ends). Host code reaches
 // it only through the address hipGetSymbolAddress gives on each device.
-constexpr size_t kScratchBytes = (size_t)128 << 20;
 constexpr int kMaxDevices = 64;
 
 // Its size beyond kScratchBytes: face_ranges may split the faces finer for the
@@ -961,69 +1031,6 @@ int scratch_on(tlm_ctx *c, int dev, unsigned char **out)
 }
 
 } // namespace
-
-namespace tlmi {
-
-// Finds whether the context's faces are the places of a few planes of a box
-// (each once, and most of them there) and records its extent. Called whenever
-// the list changes.
-int huy_lattice_scan(tlm_ctx *c)
-{
-    c->hlat = HuyLattice{};
-    const int n = c->nh, len = c->nx + c->ny + c->nz;
-    if (n < kHuyLatticeMin)
-        return TLM_OK;
-    HuyLattice h;
-    DevBuf marks, seen;
-    if (hipMalloc((void **)&marks.p, 2 * (size_t)len) != hipSuccess)
-    {
-        (void)hipGetLastError(); // no memory: the faces stay a plain list
-        return TLM_OK;
-    }
-    HIPCHK(c, hipMemset(marks.p, 0, 2 * (size_t)len));
-    k_huy_used<<<(n + 255) / 256, 256>>>(n, c->hcell, c->haxis, c->nx, c->ny, c->Pp, marks.p, marks.p + len);
-    HIPCHK(c, hipGetLastError());
-    std::vector<uint8_t> m(2 * (size_t)len);
-    HIPCHK(c, hipMemcpy(m.data(), marks.p, m.size(), hipMemcpyDeviceToHost));
-    const int dims[3] = {c->nx, c->ny, c->nz};
-    for (int q = 0, at = 0; q < 3; at += dims[q], ++q)
-    {
-        int lo = 0, hi = dims[q] - 1;
-        while (lo < hi && !m[at + lo])
-            ++lo;
-        while (hi > lo && !m[at + hi])
-            --hi;
-        h.lo[q] = lo;
-        h.n[q] = hi - lo + 1;
-        for (int i = lo; i <= hi; ++i)
-            if (m[len + at + i])
-            {
-                if (h.nplane == kHuyPlanes)
-                    return TLM_OK;
-                h.axis[h.nplane] = q;
-                h.coord[h.nplane++] = i;
-            }
-    }
-    if (!huy_lattice_fits(h, n))
-        return TLM_OK;
-    const FfLattice L(h);
-    const size_t places = (size_t)L.off[L.nplane] / 4;
-    if (hipMalloc((void **)&seen.p, (places + 1) * sizeof(int)) != hipSuccess)
-    {
-        (void)hipGetLastError(); // no memory: the faces stay a plain list
-        return TLM_OK;
-    }
-    HIPCHK(c, hipMemset(seen.p, 0, (places + 1) * sizeof(int)));
-    int *cnt = reinterpret_cast<int *>(seen.p), twice = 0;
-    k_huy_twice<<<(n + 255) / 256, 256>>>(n, c->hcell, c->haxis, c->nx, c->Pp, L, cnt, cnt + places);
-    HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipMemcpy(&twice, cnt + places, sizeof(int), hipMemcpyDeviceToHost));
-    h.ok = !twice;
-    c->hlat = h;
-    return TLM_OK;
-}
-
-} // namespace tlmi
 
 extern "C" {
 

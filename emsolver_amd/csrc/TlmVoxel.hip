@@ -1555,6 +1555,7 @@ int64_t tlm_huygens_mat(tlm_ctx *c, int o)
     c->hcell = hc;
     c->haxis = ha;
     c->hlat = HuyLattice{};
+    c->hlat_known = true;
     dfree(c, c->huy8);
     if ((rc = dalloc(c, &c->huy8, 8 * (size_t)std::max(1LL, n))))
         return rc;

@@ -98,7 +98,8 @@ struct tlm_ctx
     int *haxis = nullptr;
     float *huy8 = nullptr;
     int nh = 0;
-    tlmi::HuyLattice hlat;           // of the faces, for the far field
+    tlmi::HuyLattice hlat;           // of the faces, for the far field ...
+    bool hlat_known = false;         // ... if it was looked for since they were set
     unsigned char *ff_ws = nullptr; // far-field workspace kept between calls
     size_t ff_bytes = 0;
     long long *pcells = nullptr, *ploop = nullptr;
@@ -160,9 +161,6 @@ int prepare_pair(tlm_ctx *c);
 void mark_fold(tlm_ctx *c, hipStream_t s);
 // Those sources at step n.
 tlm::Fold fold_at(const tlm_ctx *c, int n);
-
-// Sets hlat from the context's list of faces (TlmFarField.hip).
-int huy_lattice_scan(tlm_ctx *c);
 
 // Records the message on the context (or the thread's create error) and
 // returns the code.

@@ -13,7 +13,8 @@
 //   * a state read back without pinned memory or without threads, and a small
 //     one, which asks for neither;
 //   * face lists read without device memory for their order, and the first few
-//     faces of one, which ask for none.
+//     faces of one, which ask for none;
+//   * a list of Huygens faces set without work for a far field that may not come.
 // Prints PASS/FAIL lines and exits 1 on a failure; SKIP without a device.
 //---------------------------------------------------------------------------
 #include "GpuTlmHip.h"
@@ -266,6 +267,29 @@ void no_list_memory()
     tlm_destroy(c);
 }
 
+// Setting a list of faces takes the same allocations whatever its length.
+void huygens_list()
+{
+    tlm_ctx *c = make();
+    must(upload(c), c, "tlm_upload");
+    int took[2] = {};
+    for (int k = 0; k < 2; ++k)
+    {
+        std::vector<int64_t> cells;
+        std::vector<int32_t> axes;
+        for (int q = 0; q < (k ? 3 * kNx * kNy / 2 : 100); ++q) // 6405 faces
+        {
+            cells.push_back(q);
+            axes.push_back(2);
+        }
+        const int mallocs = g_mallocs;
+        must(tlm_set_huygens(c, cells.data(), axes.data(), (int)cells.size()), c, "tlm_set_huygens");
+        took[k] = g_mallocs - mallocs;
+    }
+    check(took[0] == took[1], "allocations for a list of 100 and of 6405 Huygens faces", took[0], took[1]);
+    tlm_destroy(c);
+}
+
 } // namespace
 
 int main()
@@ -310,6 +334,7 @@ int main()
     no_pinned_or_threads(ref);
     small_state();
     no_list_memory();
+    huygens_list();
     std::printf(g_fail ? "SCARCETEST FAILED\n" : "SCARCETEST PASSED\n");
     return g_fail ? 1 : 0;
 }
