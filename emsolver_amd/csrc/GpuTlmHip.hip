@@ -387,6 +387,12 @@ PairKernel pair_kernel(const tlm_ctx *c, bool energy)
     return energy ? pair_kernel_of<false, true>(c) : pair_kernel_of<false, false>(c);
 }
 
+// Steps since the upload from which on it pays to prepare for pairs: that takes
+// 15 us (8^3; more with the allocation of a large buffer), a pair saves 3 (the
+// first run of 1, 4 and 16 steps 19, 32 and 83 us in single steps, 35, 42 and 75
+// with pairs from the first on).
+constexpr long long kPairFirst = 8;
+
 // First pair after an upload: the second stub buffer and the kernels' LDS
 // limit. The buffer starts as a copy: no step touches the stubs of the 32-cell
 // halves of a block without a dielectric cell, and a caller may have uploaded
@@ -531,13 +537,13 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
             return fail(c, TLM_ERR_STATE, "16-bit pulse storage runs contiguous step blocks");
     }
     const bool fold = fold_active(c);
-    if (pair_active(c) && !c->pair_ready)
+    if (pair_active(c) && !c->pair_ready && c->launches + c->pairs + nsteps >= kPairFirst)
     {
         int rc = prepare_pair(c);
         if (rc)
             return rc;
     }
-    const bool pairs = pair_active(c);
+    const bool pairs = pair_active(c) && c->pair_ready;
     if (fold || (pairs && c->nuniq > 0))
         mark_fold(c, c->stream);
     const int nmon0 = c->nf + c->nh + c->np + c->npr;

@@ -171,3 +171,18 @@ def test_timed_launches():
         assert dev.timed_launches() == (2, 2)
         dev.time_steps(35, 4, kernel_every=0)
         assert dev.timed_launches() == (0, 0)
+
+
+def test_pairs_begin_with_the_eighth_step():
+    """A run of few steps is not worth preparing for pairs."""
+    sc = _scene(24, 20, 28, steps=40)
+    with tlm.open_scene(sc) as dev:
+        for n, m, want in ((0, 4, (4, 0)), (4, 3, (7, 0)), (7, 3, (9, 1)), (10, 30, (24, 16))):
+            dev.run(n, m)
+            assert dev.step_launches() == want
+        dev.upload(sc.mat, *tlm.stub_admittances(sc.epsr, sc.sigma, sc.dl))
+        dev.run(0, 7)
+        assert dev.step_launches() == (7, 0)
+    with tlm.open_scene(sc) as dev:
+        dev.run(0, 8)
+        assert dev.step_launches() == (4, 4)
