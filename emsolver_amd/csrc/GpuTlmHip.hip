@@ -16,9 +16,9 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -731,25 +731,6 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
     return TLM_OK;
 }
 
-// Runs work(w) on up to `n` threads, w = 0 on the calling one; fewer where
-// the system gives no more. work must finish the job whichever of them run.
-template <class F> void on_threads(int n, const F &work)
-{
-    std::vector<std::thread> t;
-    t.reserve((size_t)n);
-    try
-    {
-        for (int w = 1; w < n; ++w)
-            t.emplace_back(work, w);
-    }
-    catch (const std::system_error &)
-    {
-    }
-    work(0);
-    for (auto &x : t)
-        x.join();
-}
-
 // Threads that move host memory: a first write to fresh memory costs more in
 // page faults (45 us a MB) than the copy itself, and they are taken side by
 // side. Their pinned memory stays at 8 MB, above which it takes 2 to 4 ms to
@@ -757,6 +738,27 @@ template <class F> void on_threads(int n, const F &work)
 // threads of 2 MB, 2.5 with six or eight; 157^3 8.1, 7.2 with six).
 constexpr int kHostThreads = 4;
 constexpr size_t kHostChunk = (size_t)2 << 20; // bytes per turn of a thread
+
+// Runs work(w) on up to n <= kHostThreads threads, w = 0 on the calling one;
+// fewer where the system gives no more threads or memory for them (no exception
+// leaves an entry point of the library). work must finish the job whichever of
+// them run.
+template <class F> void on_threads(int n, const F &work)
+{
+    std::thread t[kHostThreads];
+    try
+    {
+        for (int w = 1; w < n; ++w)
+            t[w] = std::thread(work, w);
+    }
+    catch (const std::exception &)
+    {
+    }
+    work(0);
+    for (auto &x : t)
+        if (x.joinable())
+            x.join();
+}
 
 int host_threads(size_t bytes)
 {
@@ -799,7 +801,7 @@ int read_back(tlm_ctx *c, float *host_out, const tlm::PulseView *pv, float *soa,
         pin = nullptr;
     }
     hipError_t e = hipSuccess;
-    std::vector<hipEvent_t> ev((size_t)n, nullptr);
+    hipEvent_t ev[kHostThreads] = {};
     for (int w = 0; w < n && e == hipSuccess; ++w)
         e = hipEventCreateWithFlags(&ev[w], hipEventDisableTiming);
     std::atomic<long long> next{0};
