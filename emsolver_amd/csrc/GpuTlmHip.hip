@@ -136,9 +136,9 @@ void choose_pair(tlm_ctx *c)
     // slabs per tile: the fewest slab iterations (zc and the two beside them)
     // over the rounds that the CUs take
     long long best = 0;
-    for (int nzc = (c->nz + 63) / 64; nzc <= c->nz; ++nzc)
+    for (int most = std::min(64, c->nz); most >= 1; --most)
     {
-        const int z = (c->nz + nzc - 1) / nzc;
+        const int nzc = (c->nz + most - 1) / most, z = (c->nz + nzc - 1) / nzc;
         const long long cost = ((long long)p.ntile * ((c->nz + z - 1) / z) + kCus - 1) / kCus * (z + 2);
         if (best == 0 || cost < best)
         {
