@@ -113,7 +113,10 @@ size_t energy_parts(const tlm_ctx *c)
 // The rim is 2 hb blocks of step n done twice: a tile of tb >= 8 blocks pays
 // up to hb = 12 (768 x 128 x 256: 318 against 414 us a step for two k_step
 // launches), one of 2 blocks at hb = 15 does not (606 against 263 us), so
-// grids wider than 768 cells keep single steps.
+// grids wider than 768 cells keep single steps. Over 100 grids of 330, 513, 600,
+// 700 and 768 cells of width, 3 to 768 rows and 3 to 768 slabs, with and without
+// stubs, a pair takes 0.54 to 0.96 of the single steps' time in all but two (513 x
+// 8 x 300 with stubs 1.02, 700 x 16 x 16 with stubs 1.04).
 constexpr int kPairMaxRim = 12, kPairWaves = 16, kCus = 256;
 void choose_pair(tlm_ctx *c)
 {

@@ -32,7 +32,8 @@
 // Stubs are read from Vs and written to Vs2 (a rim cell's stubs are read by
 // a tile that does not own them, so the pair cannot update them in place).
 // The intermediate pulses never reach memory; the monitors of step n+1
-// recompute them for the cells they need (PairPulses).
+// recompute them for the cells they need (PairPulses), seven cells' work for
+// each, so contexts with very many records keep single steps (pair_suits).
 #pragma once
 
 #include "tlm_kernels.h"

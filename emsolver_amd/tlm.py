@@ -398,7 +398,8 @@ class TlmDevice:
     def set_tuning(self, **changes):
         """Sets the tlm_tuning fields named (kernel, planes, block_waves,
         nontemporal, grid_blocks, fold, occupancy); the others keep their
-        current values. Results are bit-identical for every setting."""
+        current values. Results are bit-identical for every setting; FP32
+        contexts take two steps a launch with the default settings only."""
         cur = self.get_tuning()
         unknown = set(changes) - set(cur)
         if unknown:
@@ -666,7 +667,9 @@ def device_memory(device=0):
 
 
 def estimate_bytes(nx, ny, nz, pulse="f32", stubs=True) -> int:
-    """Device bytes a context of this shape allocates (monitors excluded)."""
+    """Device bytes a context of this shape allocates (monitors excluded, and
+    the second stub buffer that an FP32 context with dielectric cells may take
+    for two steps a launch)."""
     lib = _native.load()
     d = _native.GridDesc(int(nx), int(ny), int(nz), 0.01, 0.0, PULSE_TYPES[pulse], 0, 0)
     return int(lib.tlm_estimate_bytes(C.byref(d), int(bool(stubs))))
@@ -719,7 +722,8 @@ class TlmBatch:
     def set_tuning(self, **changes):
         """Sets the tlm_batch_tuning fields named (planes, block_waves,
         grid_blocks, graph_ticks, planes16); the others keep their current
-        values."""
+        values. FP32 members take two ticks a launch with the default planes,
+        block_waves and grid_blocks only."""
         cur = self.get_tuning()
         unknown = set(changes) - set(cur)
         if unknown:

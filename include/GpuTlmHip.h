@@ -220,8 +220,8 @@ int tlm_copy_bandwidth(int device, size_t bytes, int iters, float *gbps, float *
 /* Tuning of the fused scatter/connect kernel (no effect on results, which
  * are bit-identical for every setting). No counterpart in the reference.
  * With the default settings an FP32 context takes two steps a launch where it
- * can; any other setting is the shape of the launch of a single step, and
- * every step is then one. */
+ * can (tlm_step_launches tells); any other setting is the shape of the launch
+ * of a single step, and every step is then one. */
 typedef struct tlm_tuning {
     int32_t kernel;      /* 0: one cell per lane, 64-cell strips per wavefront (only variant) */
     int32_t planes;      /* z slabs marched per wave task; 0 = automatic. Default 1 with FP32
@@ -244,8 +244,8 @@ typedef struct tlm_tuning {
 int tlm_set_tuning(tlm_ctx *ctx, const tlm_tuning *t);
 int tlm_get_tuning(const tlm_ctx *ctx, tlm_tuning *t);
 
-/* Launch shape chosen for the fused kernel: strips per slab, slabs per wave
- * task, workgroup count, threads per workgroup. For reporting. */
+/* Launch shape chosen for the fused kernel of a single step: strips per slab,
+ * slabs per wave task, workgroup count, threads per workgroup. For reporting. */
 int tlm_launch_shape(const tlm_ctx *ctx, int *rows_per_group, int *planes_per_group,
                      int *groups, int *threads_per_group);
 
@@ -297,6 +297,9 @@ void tlm_schedule_tables(int waveform, float f0, float dt, int step0, int nsteps
  * A member gives the same bits alone and in a batch. While a context is a
  * member, tlm_run and the tlm_set_* / tlm_upload calls on it are refused;
  * its readers work after tlm_batch_sync.
+ * With the default planes, block_waves and grid_blocks FP32 members take two
+ * ticks a launch where they can; any other value of these three is the shape of
+ * the launch of a single tick, and every tick of the batch is then one.
  * ------------------------------------------------------------------- */
 typedef struct tlm_batch_tuning {
     int32_t planes;      /* z slabs per wave task (cells per lane); 0 = all of nz */
@@ -345,9 +348,10 @@ int tlm_batch_autotune(tlm_batch *b, int ticks_per_candidate, tlm_batch_tuning *
 int tlm_device_memory(int device, size_t *free_bytes, size_t *total_bytes);
 /* Device bytes a context of this shape allocates (pulses, stubs if any
  * dielectric, cell codes and per-step work buffers; monitors excluded). An
- * FP32 context with dielectric cells that is run by tlm_run or joins a batch
- * takes a second stub buffer (12 bytes per cell) if that is at most a quarter
- * of what is free, and steps without it otherwise. */
+ * FP32 context with dielectric cells that tlm_run has taken to its eighth step,
+ * or that joins a batch, takes a second stub buffer (12 bytes per cell, not
+ * counted here) if that is at most a quarter of what is free, and steps without
+ * it otherwise. */
 int64_t tlm_estimate_bytes(const tlm_grid_desc *desc, int has_stubs);
 
 /* ---------------------------------------------------------------------
