@@ -785,8 +785,8 @@ void host_clear(float *p, size_t count)
 // its own: order on the device, copy out, write to host_out, so that one
 // thread's copy runs beside the others' writes. 157^3 cells with stubs, 232 MB
 // into fresh memory: 26 ms from pageable copies in one thread, 8.1 here; 64^3, 16 MB: 1.02 and
-// 0.87. A state of one chunk goes straight to host_out: making and giving back
-// pinned memory takes longer than its copy (24^3, 0.8 MB: 88 us, 152 through
+// 0.87. A state of one chunk goes straight to host_out in one copy: making and
+// giving back pinned memory takes longer (24^3, 0.8 MB: 88 us, 152 through
 // pinned memory; 32^3, 2 MB: 154 and 214).
 int read_back(tlm_ctx *c, float *host_out, const tlm::PulseView *pv, float *soa, int ncomp)
 {
@@ -798,7 +798,26 @@ int read_back(tlm_ctx *c, float *host_out, const tlm::PulseView *pv, float *soa,
     int rc = dalloc(c, &stage, slot * n);
     if (rc)
         return rc;
-    if (nchunk > 1 && hipHostMalloc((void **)&pin, slot * n * sizeof(float), hipHostMallocDefault) != hipSuccess)
+    // cells [c0, c0 + cnt) ordered at d and copied to h
+    auto queue = [&](long long c0, long long cnt, float *d, float *h) {
+        const unsigned g = (unsigned)((cnt + 255) / 256);
+        if (pv)
+            hipLaunchKernelGGL(tlm::k_pulses_out, dim3(g), dim3(256), 0, c->stream, *pv, d, c->nxy, c0, cnt);
+        else
+            hipLaunchKernelGGL(tlm::k_stubs_out, dim3(g), dim3(256), 0, c->stream, soa, d, c->nxy, c->Pp, c0, cnt);
+        const hipError_t r = hipGetLastError();
+        return r != hipSuccess ? r
+                               : hipMemcpyAsync(h, d, (size_t)cnt * ncomp * sizeof(float), hipMemcpyDeviceToHost,
+                                                c->stream);
+    };
+    if (nchunk == 1)
+    {
+        const hipError_t r = queue(0, ncell, stage, host_out), w = hipStreamSynchronize(c->stream);
+        dfree(c, stage);
+        return r == hipSuccess && w == hipSuccess ? (int)TLM_OK
+                                                  : hip_fail(c, r != hipSuccess ? r : w, "tlm_read_state");
+    }
+    if (hipHostMalloc((void **)&pin, slot * n * sizeof(float), hipHostMallocDefault) != hipSuccess)
     {
         (void)hipGetLastError(); // without pinned memory straight to host_out
         pin = nullptr;
@@ -811,24 +830,15 @@ int read_back(tlm_ctx *c, float *host_out, const tlm::PulseView *pv, float *soa,
     std::atomic<int> bad{(int)e};
     if (e == hipSuccess)
         on_threads(n, [&](int w) {
-            float *d = stage + slot * w;
             hipError_t r = hipSetDevice(c->dev);
             for (long long i; r == hipSuccess && bad == hipSuccess && (i = next++) < nchunk;)
             {
                 const long long c0 = i * per, cnt = std::min(per, ncell - c0);
-                const unsigned g = (unsigned)((cnt + 255) / 256);
-                if (pv)
-                    hipLaunchKernelGGL(tlm::k_pulses_out, dim3(g), dim3(256), 0, c->stream, *pv, d, c->nxy, c0, cnt);
-                else
-                    hipLaunchKernelGGL(tlm::k_stubs_out, dim3(g), dim3(256), 0, c->stream, soa, d, c->nxy, c->Pp, c0,
-                                       cnt);
-                const size_t bytes = (size_t)cnt * ncomp * sizeof(float);
                 float *h = pin ? pin + slot * w : host_out + c0 * ncomp;
-                if ((r = hipGetLastError()) == hipSuccess &&
-                    (r = hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, c->stream)) == hipSuccess &&
+                if ((r = queue(c0, cnt, stage + slot * w, h)) == hipSuccess &&
                     (r = hipEventRecord(ev[w], c->stream)) == hipSuccess &&
                     (r = hipEventSynchronize(ev[w])) == hipSuccess && pin)
-                    std::memcpy(host_out + c0 * ncomp, h, bytes);
+                    std::memcpy(host_out + c0 * ncomp, h, (size_t)cnt * ncomp * sizeof(float));
             }
             if (r != hipSuccess)
                 bad = (int)r;
