@@ -1000,6 +1000,16 @@ int materialize(tlm_ctx *c, int step0)
 
 using namespace tlmi;
 
+// Cells of a map whose largest id tlm_upload finds on the host.
+static constexpr long long kMapHost = 1 << 18;
+static uint8_t host_max(const uint8_t *p, size_t n)
+{
+    uint8_t m = 0;
+    for (size_t i = 0; i < n; ++i)
+        m = std::max(m, p[i]);
+    return m;
+}
+
 extern "C" {
 
 int tlm_device_count(void)
@@ -1150,7 +1160,16 @@ int tlm_upload(tlm_ctx *c, const uint8_t *mat, const float *yhat, const float *g
             (void)hipGetLastError(); // the plane that the next step writes: nothing else reads it
     }
     const hipError_t e = hipMemcpyAsync(map, mat, (size_t)ncell, hipMemcpyHostToDevice, c->stream);
-    rc = e == hipSuccess ? build_codes(c, map, nmat, &max_id) : hip_fail(c, e, "hipMemcpyAsync");
+    rc = e == hipSuccess ? (int)TLM_OK : hip_fail(c, e, "hipMemcpyAsync");
+    // the largest id, of a small map sooner on the host than by a launch and a
+    // wait for its result (first upload of a context 4^3 70 us, 96 on the device,
+    // 24^3 73 and 100, 64^3 134 and 157; 80^3 on the device 190)
+    if (ncell <= kMapHost)
+        max_id = (int)std::max<unsigned>(1u, host_max(mat, (size_t)ncell)) - 2;
+    else if (!rc)
+        rc = largest_id(c, map, &max_id);
+    if (!rc)
+        rc = build_codes(c, map, nmat, max_id);
     (void)hipStreamSynchronize(c->stream); // before the map goes, also after a failure
     dfree(c, own);
     return rc ? rc : install_material(c, max_id >= 0, yhat, ghat, nmat, V, Vs);

@@ -1106,7 +1106,7 @@ bool grid_ok(const tlm_voxel_grid *g)
 
 namespace tlmi {
 
-int build_codes(tlm_ctx *c, const uint8_t *mat, int nmat, int *max_id)
+int largest_id(tlm_ctx *c, const uint8_t *mat, int *max_id)
 {
     const long long ncell = (long long)c->nx * c->ny * c->nz;
     Scratch s;
@@ -1119,8 +1119,14 @@ int build_codes(tlm_ctx *c, const uint8_t *mat, int nmat, int *max_id)
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpyAsync(max_id, dmax, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (*max_id >= nmat)
+    return TLM_OK;
+}
+
+int build_codes(tlm_ctx *c, const uint8_t *mat, int nmat, int max_id)
+{
+    if (max_id >= nmat)
         return fail(c, TLM_ERR_ARG, "material id without a yhat/ghat entry");
+    int rc;
     const long long nblk = c->P / tlm::kWave;
     // padded to a multiple of 4 bytes for the step's dword loads of the flags
     if ((rc = upload(c, &c->uair, (const uint8_t *)nullptr, (size_t)((nblk + 3) / 4 * 4))))
@@ -1460,7 +1466,7 @@ int tlm_upload_mat(tlm_ctx *c, const float *yhat, const float *ghat, int nmat)
     if (nmat < 0 || (nmat > 0 && (!yhat || !ghat)))
         return fail(c, TLM_ERR_ARG, "tlm_upload_mat: bad arguments");
     int max_id = -1;
-    if ((rc = build_codes(c, c->mat, nmat, &max_id)))
+    if ((rc = largest_id(c, c->mat, &max_id)) || (rc = build_codes(c, c->mat, nmat, max_id)))
         return rc;
     return install_material(c, max_id >= 0, yhat, ghat, nmat, nullptr, nullptr);
 }

@@ -146,10 +146,11 @@ struct tlm_ctx
 
 namespace tlmi {
 
-// Cell codes and block flags of a device map (cellIndex order, 16-byte aligned);
-// *max_id: its largest dielectric index, -1 if none. Refuses one without an
-// entry among nmat (TlmVoxel.hip).
-int build_codes(tlm_ctx *c, const uint8_t *mat, int nmat, int *max_id);
+// Largest dielectric index of a device map (cellIndex order, 16-byte aligned), -1
+// if none; cell codes and block flags of a map with that largest index. Refuses
+// one without an entry among nmat (TlmVoxel.hip).
+int largest_id(tlm_ctx *c, const uint8_t *mat, int *max_id);
+int build_codes(tlm_ctx *c, const uint8_t *mat, int nmat, int max_id);
 
 // Whether a pair of steps can add the context's sources and is worth it with
 // its monitors.

@@ -226,6 +226,9 @@ void small_state()
     must(tlm_create(&d, &c), nullptr, "tlm_create");
     const int n = 32 * 32 * 32;
     const std::vector<uint8_t> mat((size_t)n, 2);
+    const int mallocs = g_mallocs;
+    must(tlm_upload(c, mat.data(), kY, kG, 1, nullptr, nullptr), c, "tlm_upload");
+    check(g_mallocs - mallocs == 3, "a small map: block flags, materials and stubs allocated, no more", g_mallocs - mallocs, 3);
     must(tlm_upload(c, mat.data(), kY, kG, 1, g_V.data(), g_Vs.data()), c, "tlm_upload");
     State s;
     const int pinned = g_pinned, threads = g_threads;
