@@ -390,11 +390,17 @@ PairKernel pair_kernel(const tlm_ctx *c, bool energy)
     return energy ? pair_kernel_of<false, true>(c) : pair_kernel_of<false, false>(c);
 }
 
-// Steps since the upload from which on it pays to prepare for pairs: that takes
-// 15 us (8^3; more with the allocation of a large buffer), a pair saves 3 (the
-// first run of 1, 4 and 16 steps 19, 32 and 83 us in single steps, 35, 42 and 75
-// with pairs from the first on).
-constexpr long long kPairFirst = 8;
+// Steps since the upload from which on it pays to prepare for pairs. That takes
+// 15 us or, with the allocation of a large buffer, 30; a pair of a small grid
+// saves 3 (8^3: the first run of 1, 4 and 16 steps 19, 32 and 83 us in single
+// steps, 35, 42 and 75 with pairs from the first on; 64^3 22, 47, 142 and 49, 66,
+// 148). From 3 M cells on it takes less than the first pair saves (first run of 2
+// steps 162^3 225 us in single steps, 187 as a pair, 256^3 755 and 530; 128^3 85
+// and 111).
+long long pair_first(const tlm_ctx *c)
+{
+    return (long long)c->nx * c->ny * c->nz < (3LL << 20) ? 8 : 2;
+}
 
 // First pair after an upload: the second stub buffer and the kernels' LDS
 // limit. The buffer starts as a copy: no step touches the stubs of the 32-cell
@@ -540,7 +546,7 @@ int queue_steps(tlm_ctx *c, int step0, int nsteps, int kernel_every, float *ms_k
             return fail(c, TLM_ERR_STATE, "16-bit pulse storage runs contiguous step blocks");
     }
     const bool fold = fold_active(c);
-    if (pair_active(c) && !c->pair_ready && c->launches + c->pairs + nsteps >= kPairFirst)
+    if (pair_active(c) && !c->pair_ready && c->launches + c->pairs + nsteps >= pair_first(c))
     {
         int rc = prepare_pair(c);
         if (rc)

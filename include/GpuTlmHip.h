@@ -348,8 +348,8 @@ int tlm_batch_autotune(tlm_batch *b, int ticks_per_candidate, tlm_batch_tuning *
 int tlm_device_memory(int device, size_t *free_bytes, size_t *total_bytes);
 /* Device bytes a context of this shape allocates (pulses, stubs if any
  * dielectric, cell codes and per-step work buffers; monitors excluded). An
- * FP32 context with dielectric cells that tlm_run has taken to its eighth step,
- * or that joins a batch, takes a second stub buffer (12 bytes per cell, not
+ * FP32 context with dielectric cells that tlm_run has taken to its second step
+ * (eighth, below 3 M cells), or that joins a batch, takes a second stub buffer (12 bytes per cell, not
  * counted here) if that is at most a quarter of what is free, and steps without
  * it otherwise. */
 int64_t tlm_estimate_bytes(const tlm_grid_desc *desc, int has_stubs);

@@ -174,7 +174,7 @@ def test_timed_launches():
 
 
 def test_pairs_begin_with_the_eighth_step():
-    """A run of few steps is not worth preparing for pairs."""
+    """A run of few steps of a small grid is not worth preparing for pairs."""
     sc = _scene(24, 20, 28, steps=40)
     with tlm.open_scene(sc) as dev:
         for n, m, want in ((0, 4, (4, 0)), (4, 3, (7, 0)), (7, 3, (9, 1)), (10, 30, (24, 16))):
@@ -186,3 +186,7 @@ def test_pairs_begin_with_the_eighth_step():
     with tlm.open_scene(sc) as dev:
         dev.run(0, 8)
         assert dev.step_launches() == (4, 4)
+    with tlm.open_scene(_scene(148, 148, 148, steps=40)) as dev:  # 3.2 M cells
+        dev.run(0, 1)
+        dev.run(1, 2)
+        assert dev.step_launches() == (2, 1)
