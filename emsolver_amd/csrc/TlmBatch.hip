@@ -1003,7 +1003,7 @@ int tlm_batch_autotune(tlm_batch *b, int ticks_per_candidate, tlm_batch_tuning *
         b->dirty = true;
         float ms = 0.f;
         int64_t cu = 0;
-        int rc = tlm_batch_time(b, 2, &ms, &cu); // warm-up (table rebuild, the kernels' first run)
+        int rc = tlm_batch_time(b, pairs_wanted(b) ? 2 : 1, &ms, &cu); // warm-up (tables, the kernel's first run)
         int window = ticks_per_candidate;
         while (!rc && (window = pair_window(b, ticks_per_candidate)) == 0)
             rc = tlm_batch_time(b, 1, &ms, &cu);

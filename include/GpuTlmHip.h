@@ -340,8 +340,8 @@ int tlm_batch_time(tlm_batch *b, int nticks, float *ms, int64_t *cell_updates);
 /* Online autotuner: times real ticks of the batch under each candidate
  * launch shape (slabs per wave task, waves per workgroup, grid) and keeps
  * the fastest per cell update; results do not depend on the shape. A
- * candidate takes two ticks and then ticks_per_candidate, made even (and ended
- * before a member's odd last step) for a shape that takes two ticks a launch. */
+ * candidate takes one tick and then ticks_per_candidate; a shape that takes two
+ * ticks a launch two and an even number, ended before a member's odd last step. */
 int tlm_batch_autotune(tlm_batch *b, int ticks_per_candidate, tlm_batch_tuning *best);
 
 /* Free and total device memory (admission control of a serving loop). */
