@@ -260,9 +260,9 @@ def batched_run(count=256, sample_every=4):
         with open(path) as f:
             m = re.search(r"traffic_bytes_per_tick:\s*([0-9.eE+]+)", f.read())
         if m:
-            # HBM bytes of one tick with every member active (rocprofv3 PMC)
+            # HBM bytes of one of two ticks in a launch, every member active (rocprofv3 PMC)
             out["traffic_bytes_per_tick"] = float(m.group(1))
-            out["alg_bytes_per_tick"] = round(bpc * sum(sc.ncell for sc in scs))
+            out["alg_bytes_per_tick"] = round(sum(sc.ncell * scene_alg_bytes(sc) for sc in scs) / 2)
     log(f"[bench] batched_{count}: {out['gcell_s']:.2f} Gcell/s aggregate in {wall:.1f}s "
         f"(tuning {tuning}); one at a time {out['one_at_a_time_gcell_s']:.2f} Gcell/s")
     return out
