@@ -1200,18 +1200,19 @@ int install_material(tlm_ctx *c, bool any_diel, const float *yhat, const float *
     if (rc)
         return rc;
     c->nmat = nmat;
-    c->stubs = any_diel;
     if (c->pf == TLM_PULSE_F32)
     {
         HIPCHK(c, hipMemsetAsync(c->A, 0, (size_t)c->PB * 12, c->stream));
         HIPCHK(c, hipMemsetAsync(c->B, 0, (size_t)c->PB * 12, c->stream));
     }
+    c->stubs = false;
     dfree(c, c->Vs);
     c->pair_ready = c->pair_refused = false;
-    if (c->stubs)
+    if (any_diel)
     {
         if ((rc = dalloc(c, &c->Vs, (size_t)c->P * 3)))
             return rc;
+        c->stubs = true;
         HIPCHK(c, hipMemsetAsync(c->Vs, 0, (size_t)c->P * 3 * sizeof(float), c->stream));
     }
     else

@@ -1126,6 +1126,7 @@ int build_codes(tlm_ctx *c, const uint8_t *mat, int nmat, int max_id)
 {
     if (max_id >= nmat)
         return fail(c, TLM_ERR_ARG, "material id without a yhat/ghat entry");
+    c->uploaded = false; // until install_material is through: a failure leaves nothing to run
     int rc;
     const long long nblk = c->P / tlm::kWave;
     // padded to a multiple of 4 bytes for the step's dword loads of the flags

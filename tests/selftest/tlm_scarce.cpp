@@ -9,7 +9,8 @@
 //   * a context without room for the second stub buffer of pairs of steps takes
 //     single steps, without an error left behind, and pairs again after an
 //     upload that finds room;
-//   * an upload without memory for the device map, refused or not;
+//   * an upload without memory for the device map, refused or not; an upload that
+//     fails half way, which leaves nothing to run;
 //   * a state read back without pinned memory or without threads, and a small
 //     one, which asks for neither;
 //   * face lists read without device memory for their order, and the first few
@@ -198,6 +199,29 @@ void no_map(const State &ref)
     tlm_destroy(c);
 }
 
+// A second upload that finds no room for the stubs, or for the block flags.
+void failed_upload(const State &ref)
+{
+    const size_t flags = (size_t)((kNx * kNy + 63) / 64 * kNz + 3) / 4 * 4;
+    for (size_t refused : {kStubs, flags})
+    {
+        tlm_ctx *c = make();
+        must(upload(c), c, "tlm_upload");
+        run(c, 0, 10);
+        g_refuse_size = refused;
+        const int rc = upload(c);
+        g_refuse_size = kNone;
+        check(rc == TLM_ERR_NOMEM, "an upload without room", rc, TLM_ERR_NOMEM);
+        const int ran = tlm_run(c, 10, 2);
+        check(ran == TLM_ERR_STATE, "... leaves nothing to run", ran, TLM_ERR_STATE);
+        (void)read(c);
+        must(upload(c), c, "tlm_upload");
+        run(c, 0, kSteps);
+        check(read(c) == ref, "... and the next one all of it");
+        tlm_destroy(c);
+    }
+}
+
 void no_pinned_or_threads(const State &ref)
 {
     tlm_ctx *c = make();
@@ -334,6 +358,7 @@ int main()
 
     no_second_stub_buffer(ref);
     no_map(ref);
+    failed_upload(ref);
     no_pinned_or_threads(ref);
     small_state();
     no_list_memory();
