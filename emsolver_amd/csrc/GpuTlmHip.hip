@@ -2020,9 +2020,17 @@ int64_t tlm_build_pec_faces(int nx, int ny, int nz, const uint8_t *mat, int64_t 
         for (int j = 0; j < ny; ++j)
             for (int i = 0; i < nx; ++i)
             {
-                long long c = ((long long)k * ny + j) * nx + i;
-                if (mat[c] != 1)
-                    continue;
+                // a row's next PEC cell by memchr (157 x 131 x 143 cells, one plane PEC, twice:
+                // 0.4 ms; by a byte at a time 1.8 or 2.4 on one host, as the loop happened to be placed)
+                const uint8_t *row = mat + ((long long)k * ny + j) * nx;
+                if (row[i] != 1)
+                {
+                    const void *p = std::memchr(row + i, 1, (size_t)(nx - i));
+                    if (!p)
+                        break;
+                    i = (int)(static_cast<const uint8_t *>(p) - row);
+                }
+                const long long c = row + i - mat;
                 const int co[3] = {i, j, k};
                 for (int a = 0; a < 3; ++a)
                     for (int s = -1; s <= 1; s += 2)
